@@ -166,18 +166,19 @@ def work(case):
 
 
 def tolerance(case):
-    # fp32 sums of fp16 products: about 1e-7 relative.  Ids may swap where two
-    # scores lie closer than that, which long result lists see most.  Cosine
-    # inputs are rounded to fp16 once after their fp32 norm, whose last bit may
-    # move single elements by one fp16 step.
+    # fp32 sums of fp16 products: about 1e-7 relative, and 2e-6 at most over 30
+    # drawn cases against 64 bits.  Ids may swap where two scores lie closer than
+    # that, which long result lists see most (7e-4 of them at most, measured).
+    # Cosine inputs are rounded to fp16 once after their fp32 norm, whose last
+    # bit may move single elements by one fp16 step.
     cosine = case["metric"] == "cosine"
     if case["op"] == "scores":
         if not case["fp32"]:
             return {"rel": 2e-4, "max": 4e-3}  # an fp16 step where the sum sits on a rounding boundary
         return {"rel": 2e-5 if cosine else 2e-6, "max": 1e-3 if cosine else 1e-4}
     if case["op"] == "build":
-        return {"rel": 1e-4, "max": 4e-3, "differ": 0.01}
-    return {"rel": 2e-5 if cosine else 2e-6, "max": 1e-3 if cosine else 1e-4, "differ": 0.01}
+        return {"rel": 1e-4, "max": 4e-3, "differ": 0.003}
+    return {"rel": 2e-5 if cosine else 2e-6, "max": 1e-3 if cosine else 1e-4, "differ": 0.003}
 
 
 def _stored(case, r):
