@@ -11,6 +11,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -729,18 +730,42 @@ int cvs_scores(const void* q, const void* x, int64_t nq, int64_t n, int64_t d, v
 
 namespace {
 
-// Chunks per row for cvs_topk_rows: enough workgroups to keep ~4 per CU busy,
-// chunks of at least max(4096, 2k) columns, at most kSelectMaxLists of them.
-int64_t rowtopk_chunks(int64_t nq, int64_t n, int64_t k, int cus) {
-  const int64_t want = ceil_div(4 * (int64_t)cus, std::max<int64_t>(nq, 1));
-  const int64_t most = std::max<int64_t>(1, n / std::max<int64_t>(4096, 2 * k));
-  int64_t c = std::max<int64_t>(1, std::min<int64_t>({want, most, (int64_t)kSelectMaxLists}));
-  const int64_t len = ceil_div(n, c);
-  return ceil_div(n, len);
+// Plan of cvs_topk_rows (see cvs_rowtopk.hip); rows of at most kRowCap columns
+// need no workspace.  At most kRowBatch rows run in one set of launches, so
+// the candidate arrays stay within 64 MB whatever the batch.
+constexpr int64_t kRowBatch = 1024;
+
+struct RowPlan {
+  int64_t rows = 0;  // rows per set of launches
+  int64_t groups = 0, rank = 0, len = 0, chunks = 1;
+  int64_t off_count = 0, off_cand = 0, ws_bytes = 0;
+};
+
+RowPlan row_plan(int64_t nq, int64_t n, int64_t k, int cus) {
+  RowPlan P;
+  P.rows = std::max<int64_t>(1, std::min<int64_t>(nq, kRowBatch));
+  if (n <= kRowCap) return P;
+  // The sample: a 32nd of the row, at least 16384 scores (a quarter of a short
+  // row), so that about 8 or more of the row's k best are in it for k = 256
+  // (30 at k = 1000 over 1M columns); the threshold is the score `rank` from
+  // the top of the sample, 15% and five standard deviations (and 5) past where
+  // the k-th best is expected, so that fewer than k scores practically never
+  // reach it and at most a few thousand do (kRowCap = 8192 fit).
+  P.groups = std::min<int64_t>(n / 128, std::max<int64_t>(512, n / 1024));
+  const double mu = (double)k * 32.0 * (double)P.groups / (double)n;
+  P.rank = (int64_t)(1.15 * mu + 5.0 * std::sqrt(mu) + 5.0);
+  // about 8 filter workgroups per CU, of 1 to 16 rounds of 4096 columns
+  const int64_t want = ceil_div(P.rows * n, 8 * (int64_t)cus);
+  P.len = std::max<int64_t>(4096, std::min<int64_t>(65536, align_up(want, 4096)));
+  P.chunks = ceil_div(n, P.len);
+  P.off_count = align_up(P.rows * 4, 256);
+  P.off_cand = P.off_count + align_up(P.rows * 4, 256);
+  P.ws_bytes = P.off_cand + P.rows * (int64_t)kRowCap * 8;
+  return P;
 }
 
 int check_topk_rows(int64_t nq, int64_t n, int64_t k) {
-  if (k < 1 || k > kSelectMaxK) return fail(CVS_ERR_INVALID, "topk_rows supports 1 <= k <= %d", kSelectMaxK);
+  if (k < 1 || k > kRowTopkMaxK) return fail(CVS_ERR_INVALID, "topk_rows supports 1 <= k <= %d", kRowTopkMaxK);
   if (k > n) return fail(CVS_ERR_INVALID, "k must not exceed the row length");
   if (n >= INT_MAX) return fail(CVS_ERR_INVALID, "rows must have fewer than 2^31 columns");
   if (nq < 0 || nq >= INT_MAX) return fail(CVS_ERR_INVALID, "too many rows");
@@ -755,9 +780,7 @@ int cvs_topk_rows_plan(int64_t nq, int64_t n, int64_t k, int device, int64_t* wo
   if (rc != CVS_OK) return rc;
   rc = check_topk_rows(nq, n, k);
   if (rc != CVS_OK) return rc;
-  const int64_t c = rowtopk_chunks(nq, n, k, di.cus);
-  if (nq * c >= INT_MAX) return fail(CVS_ERR_INVALID, "too many rows");
-  if (workspace_bytes) *workspace_bytes = c > 1 ? align_up(nq * c * k * 4, 256) * 2 : 0;
+  if (workspace_bytes) *workspace_bytes = row_plan(nq, n, k, di.cus).ws_bytes;
   return CVS_OK;
 }
 
@@ -772,49 +795,36 @@ int cvs_topk_rows(const float* scores, int64_t nq, int64_t n, int64_t k, int fla
   if (nq == 0) return CVS_OK;
   if (scores == nullptr || out_v == nullptr || out_i == nullptr) return fail(CVS_ERR_INVALID, "pointers must not be null");
   if (reinterpret_cast<uintptr_t>(scores) % 4 != 0) return fail(CVS_ERR_INVALID, "scores must be 4-byte aligned");
-  const int64_t c = rowtopk_chunks(nq, n, k, di.cus);
-  if (nq * c >= INT_MAX) return fail(CVS_ERR_INVALID, "too many rows");
-  const int64_t part = align_up(nq * c * k * 4, 256);
-  if (c > 1) {
-    if (workspace == nullptr || workspace_bytes < 2 * part)
-      return fail(CVS_ERR_INVALID, "workspace too small: need %lld bytes, got %lld", (long long)(2 * part),
+  const RowPlan P = row_plan(nq, n, k, di.cus);
+  if (P.ws_bytes > 0) {
+    if (workspace == nullptr || workspace_bytes < P.ws_bytes)
+      return fail(CVS_ERR_INVALID, "workspace too small: need %lld bytes, got %lld", (long long)P.ws_bytes,
                   (long long)workspace_bytes);
     if (reinterpret_cast<uintptr_t>(workspace) % 256 != 0) return fail(CVS_ERR_INVALID, "workspace must be 256-byte aligned");
   }
   DeviceGuard guard(device);
   if (guard.err != hipSuccess) return hip_fail(guard.err, "hipSetDevice");
-  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const int ids64 = (flags & CVS_FLAG_IDS_INT64) ? 1 : 0;
+  char* ws = static_cast<char*>(workspace);
   RowTopkArgs r{};
   r.scores = scores;
   r.n = n;
-  r.len = ceil_div(n, c);
-  r.chunks = (int)c;
   r.k = (int)k;
-  if (c == 1) {  // one chunk per row: the first stage is the answer
-    r.out_v = out_v;
-    r.out_i = out_i;
-    r.ids64 = ids64;
-    hipError_t e = launch_rowtopk(r, (int)nq, s);
-    return e == hipSuccess ? CVS_OK : hip_fail(e, "row top-k launch");
+  r.out_v = out_v;
+  r.out_i = out_i;
+  r.ids64 = (flags & CVS_FLAG_IDS_INT64) ? 1 : 0;
+  if (P.ws_bytes > 0) {
+    r.groups = (int)P.groups;
+    r.rank = (int)P.rank;
+    r.len = P.len;
+    r.chunks = (int)P.chunks;
+    r.tau = reinterpret_cast<uint32_t*>(ws);
+    r.count = reinterpret_cast<int*>(ws + P.off_count);
+    r.cand = reinterpret_cast<uint64_t*>(ws + P.off_cand);
   }
-  char* ws = static_cast<char*>(workspace);
-  r.out_v = reinterpret_cast<float*>(ws);
-  r.out_i = ws + part;
-  r.ids64 = 0;
-  hipError_t e = launch_rowtopk(r, (int)(nq * c), s);
-  if (e != hipSuccess) return hip_fail(e, "row top-k launch");
-  SelectArgs sa{};  // second stage: merge the c sorted chunk lists of each row
-  sa.lv = r.out_v;
-  sa.li = reinterpret_cast<const int*>(r.out_i);
-  sa.nlists = (int)c;
-  sa.cap = (int)k;
-  sa.k = (int)k;
-  sa.out_v = out_v;
-  sa.out_i = out_i;
-  sa.ids64 = ids64;
-  e = launch_select(0, sa, (int)nq, s);
-  if (e != hipSuccess) return hip_fail(e, "select launch");
+  for (r.row0 = 0; r.row0 < nq; r.row0 += P.rows) {
+    hipError_t e = launch_row_topk(r, (int)std::min<int64_t>(P.rows, nq - r.row0), reinterpret_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return hip_fail(e, "row top-k launch");
+  }
   return CVS_OK;
 }
 

@@ -126,16 +126,26 @@ struct GemvArgs {
   float gamma;
 };
 
-// Row top-k, first stage: one workgroup per (row, chunk of `len` columns).
+// Exact top-k of fp32 score rows (cvs_rowtopk.hip): row r of a launch is row
+// row0 + r of the matrix and of the outputs.
+constexpr int kRowTopkMaxK = 1024;
+constexpr int kRowCap = 8192;  // candidates per row; shorter rows are sorted whole
 struct RowTopkArgs {
   const float* scores;  // [rows, n] fp32
   int64_t n;
-  int64_t len;          // columns per chunk
-  int chunks;           // chunks per row (ceil(n / len))
+  int64_t row0;
   int k;
-  float* out_v;         // [rows * chunks, k]
-  void* out_i;          // [rows * chunks, k] int32 column ids (int64 when ids64)
+  float* out_v;         // [rows, k]
+  void* out_i;          // [rows, k] int32 column ids (int64 when ids64)
   int ids64;
+  // rows longer than kRowCap
+  int groups;           // sampled groups of 32 scores per row
+  int rank;             // the sample's rank taken as threshold
+  int64_t len;          // columns per filter workgroup (a multiple of 4)
+  int chunks;           // ceil(n / len)
+  uint32_t* tau;        // [rows of a launch] threshold order keys
+  int* count;           // [rows of a launch] scores that reached them
+  uint64_t* cand;       // [rows of a launch, kRowCap] their keys
 };
 
 // Row preparation: dst[r, :d] = src[r, :d] (scaled to unit L2 norm when
@@ -261,7 +271,7 @@ hipError_t launch_gemv(const GemvArgs& a, int grid, hipStream_t s);  // any d % 
 hipError_t launch_select(int mode, const SelectArgs& a, int nq, hipStream_t s);
 hipError_t launch_rescore(const SelectArgs& a, int nq, hipStream_t s);
 hipError_t launch_prep(const PrepArgs& a, hipStream_t s);
-hipError_t launch_rowtopk(const RowTopkArgs& a, int blocks, hipStream_t s);
+hipError_t launch_row_topk(const RowTopkArgs& a, int rows, hipStream_t s);
 hipError_t launch_q8_build(const Q8BuildArgs& a, hipStream_t s);
 hipError_t launch_q8_queries(const Q8QueryArgs& a, hipStream_t s);
 
@@ -269,6 +279,5 @@ bool scan_cfg_available(const ScanCfg& cfg, int mode);
 
 constexpr int kSelectMaxLists = 8192;
 constexpr int kMaxCap = 512;  // largest candidate-list capacity (k <= 256)
-constexpr int kSelectMaxK = 1024;  // largest k of the select kernel (row top-k of a score matrix)
 
 }  // namespace cvs

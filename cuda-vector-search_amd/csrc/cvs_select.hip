@@ -12,9 +12,7 @@
 // like the reference's.
 //
 // Threshold mode returns only the score of the k-th best key (used to turn the
-// sampling pre-pass's unit maxima into per-query thresholds).  With one list
-// per query holding a whole score row it is also the row top-k of a score
-// matrix (k up to 1024: the large-k path).
+// sampling pre-pass's unit maxima into per-query thresholds).
 //
 // Rescore mode finishes the int8 pre-filter: list entries are (score upper
 // bound, row id) pairs whose bound reached the threshold, and exact scores are
@@ -50,7 +48,6 @@ struct SelSharedT {
   uint64_t thr_key;
 };
 typedef SelSharedT<kSelectMaxLists> SelShared;
-typedef SelSharedT<1> RowShared;  // no list offsets: ~38 KB, several workgroups per CU
 
 // Cuts keys[0..nb) down to its k largest keys (nb > k), in place and in any
 // order, and returns the k-th largest key.  Whole block.
@@ -444,28 +441,13 @@ __device__ __forceinline__ uint64_t block_cut_hist(SH& S, int nb, int k, int lim
 // way and sorted by rank, leaving the k best first.  Whole block.  Every thread
 // reads the count before any thread can append again, so all take the same
 // branch.  Returns true when keys[0..min(nbuf, k)) are sorted (descending).
-template <bool HIST = true, class SH>
+template <class SH>
 __device__ __forceinline__ bool end_batch(SH& S, int k, bool last) {
   __shared__ uint64_t red[kWaves];
   __syncthreads();
   int nb = S.nbuf;
   bool sorted = false;
-  if (!HIST) {  // exact cuts only (the row top-k: large k, registers needed elsewhere)
-    if (last && nb <= kBlock) {
-      block_rank_sort(S.keys, nb);
-      sorted = true;
-      if (threadIdx.x == 0 && nb > k) {
-        S.nbuf = k;
-        S.thr_key = S.keys[k - 1];
-      }
-    } else if (nb > kBuf - kBatch || (last && nb > k)) {
-      const uint64_t kth = block_keep_top(S, nb, k);
-      if (threadIdx.x == 0) {
-        S.nbuf = k;
-        S.thr_key = kth;
-      }
-    }
-  } else if (!last && nb > kBuf - kBatch) {  // make room: a loose cut, else the exact one
+  if (!last && nb > kBuf - kBatch) {  // make room: a loose cut, else the exact one
     int m = 0;
     const uint64_t cut = block_cut_hist(S, nb, k, kBuf - kBatch, red, &m);
     if (m <= kBuf - kBatch) {
@@ -481,26 +463,20 @@ __device__ __forceinline__ bool end_batch(SH& S, int k, bool last) {
       }
     }
   } else if (last && nb > k) {
-    uint64_t kth = 0ull;
-    if (nb > kBlock) {  // down to at most kBlock keys holding the k best
+    if (nb > kBlock) {  // down to at most kBlock keys holding the k best (k <= kBlock)
       int m = 0;
       block_cut_hist(S, nb, k, kBlock, red, &m, false);
       if (m > kBlock) {
-        kth = block_keep_top(S, nb, k);
+        block_keep_top(S, nb, k);
         m = k;
       }
       nb = m;
     }
-    if (nb <= kBlock) {
-      block_rank_sort(S.keys, nb);  // sorted: the k best first
-      sorted = true;
-      if (threadIdx.x == 0) {
-        S.nbuf = k;
-        S.thr_key = S.keys[k - 1];
-      }
-    } else if (threadIdx.x == 0) {  // k > kBlock: the exact cut's k keys, unsorted
+    block_rank_sort(S.keys, nb);  // sorted: the k best first
+    sorted = true;
+    if (threadIdx.x == 0) {
       S.nbuf = k;
-      S.thr_key = kth;
+      S.thr_key = S.keys[k - 1];
     }
   }
   __syncthreads();
@@ -1297,78 +1273,7 @@ __global__ __launch_bounds__(kBlock) void rescore_kernel(SelectArgs a) {
     const_cast<int*>(a.lcount)[(int64_t)q * NL + L0 + tid] = kept[tid];
 }
 
-// Exact top-k of one chunk of one score row: workgroup b takes row b / chunks,
-// columns [c*len, min((c+1)*len, n)) with c = b % chunks, and writes its k
-// best (value, column) sorted to out[b].  Each thread loads kRowU values per
-// round with all loads in flight, then appends the ones above the running k-th
-// best key in kBatch-sized steps (wave-aggregated LDS appends).
-constexpr int kRowU = 32;
-
-__global__ __launch_bounds__(kBlock) void rowtopk_kernel(RowTopkArgs a) {
-  __shared__ RowShared S;
-  const int tid = threadIdx.x;
-  const int lane = tid % kWave;
-  const int b = blockIdx.x;
-  const int q = b / a.chunks;
-  const int c = b % a.chunks;
-  const int64_t start = (int64_t)c * a.len;
-  const int cnt = (int)min<int64_t>(a.len, a.n - start);
-  const float* src = a.scores + (int64_t)q * a.n + start;
-  const int k = a.k;
-  if (tid == 0) {
-    S.nbuf = 0;
-    S.thr_key = 0ull;
-  }
-  __syncthreads();
-  constexpr int kRound = kRowU * kBlock;
-  for (int base = 0; base < cnt; base += kRound) {
-    float val[kRowU];
-#pragma unroll
-    for (int u = 0; u < kRowU; ++u) {  // coalesced; a slot past the end re-reads column 0
-      const int gi = base + u * kBlock + tid;
-      val[u] = src[gi < cnt ? gi : 0];
-    }
-#pragma unroll
-    for (int sub = 0; sub < kRowU / (kBatch / kBlock); ++sub) {
-      const uint64_t t = S.thr_key;
-#pragma unroll
-      for (int j = 0; j < kBatch / kBlock; ++j) {
-        const int u = sub * (kBatch / kBlock) + j;
-        const int gi = base + u * kBlock + tid;
-        const uint64_t key = make_key(val[u], (int)(start + gi));
-        const bool pass = gi < cnt && key > t;
-        const uint64_t mk = __ballot(pass);
-        int pos = 0;
-        if (lane == 0 && mk) pos = atomicAdd(&S.nbuf, __popcll(mk));
-        pos = __shfl(pos, 0);
-        if (pass) S.keys[pos + lanes_below(mk)] = key;
-      }
-      const bool last = base + (sub + 1) * kBatch >= cnt;
-      end_batch<false>(S, k, last);
-      if (last) break;
-    }
-  }
-  const int nb = min(S.nbuf, k);
-  block_sort_keys(S.keys, nb);
-  for (int r = tid; r < k; r += kBlock) {
-    const bool ok = r < nb;
-    const int64_t o = (int64_t)b * k + r;
-    a.out_v[o] = ok ? key_score(S.keys[r]) : -__builtin_inff();
-    const int id = ok ? key_id(S.keys[r]) : -1;
-    if (a.ids64)
-      ((int64_t*)a.out_i)[o] = id;
-    else
-      ((int*)a.out_i)[o] = id;
-  }
-}
-
 }  // namespace
-
-hipError_t launch_rowtopk(const RowTopkArgs& a, int blocks, hipStream_t s) {
-  if (a.k < 1 || a.k > kSelectMaxK || a.chunks < 1 || a.len < 1 || blocks < 1) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(rowtopk_kernel, dim3(blocks), dim3(kBlock), 0, s, a);
-  return hipGetLastError();
-}
 
 hipError_t launch_rescore(const SelectArgs& a, int nq, hipStream_t s) {
   if (a.q == nullptr || a.x == nullptr || a.li == nullptr || a.lv == nullptr || a.lcount == nullptr || a.d < 8 ||
@@ -1386,7 +1291,7 @@ hipError_t launch_rescore(const SelectArgs& a, int nq, hipStream_t s) {
 }
 
 hipError_t launch_select(int mode, const SelectArgs& a, int nq, hipStream_t s) {
-  if (a.nlists < 1 || a.nlists > kSelectMaxLists || a.k < 1 || a.k > kSelectMaxK) return hipErrorInvalidValue;
+  if (a.nlists < 1 || a.nlists > kSelectMaxLists || a.k < 1 || a.k > kBlock) return hipErrorInvalidValue;
   switch (mode) {
     case kSelFinal:
       hipLaunchKernelGGL(select_kernel<kSelFinal>, dim3(nq), dim3(kBlock), 0, s, a);

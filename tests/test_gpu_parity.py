@@ -641,6 +641,37 @@ def test_topk_rows_with_infinite_scores(eng, nq, n, k):
     np.testing.assert_array_equal(v.cpu().numpy(), np.take_along_axis(sn, order, axis=1))
 
 
+@pytest.mark.parametrize("nq,n,k,data", [
+    (3, 8192, 1024, "normal"), (3, 8193, 1, "normal"), (2, 12289, 1024, "normal"),  # whole rows / filtered, odd strides
+    (1030, 9001, 257, "normal"),           # more rows than one set of launches takes
+    (2, 70001, 1000, "equal"),             # every score reaches the threshold: streamed again
+    (2, 70001, 1000, "burst"),             # the sample sees every high score, too few reach it: streamed again
+    (2, 300000, 1000, "block"),            # the best scores side by side in one filter workgroup
+    (2, 40000, 300, "nan"),                # NaN above +inf, as the keys order them
+])
+def test_topk_rows_threshold_edges(eng, nq, n, k, data):
+    say(f"topk_rows nq={nq} n={n} k={k} {data}")
+    g = torch.Generator().manual_seed(n + k)
+    s = torch.randn(nq, n, generator=g)
+    if data == "equal":
+        s[:] = 0.25
+    elif data == "burst":  # 512 groups of 32 every 136 columns, from column 52: 500 high scores, all sampled
+        s = s * 1e-3
+        s[:, 60:60 + 136 * 500:136] += 9.0
+    elif data == "block":
+        s[:, 100000:103000] += 50.0
+    elif data == "nan":
+        s[0, 17::911] = float("nan")
+        s[1, 5] = float("inf")
+    v, i = eng.topk_rows(s.cuda(), k)
+    torch.cuda.synchronize()
+    bits = s.numpy().view(np.uint32).astype(np.int64)
+    key = np.where(bits & 0x80000000, 0xFFFFFFFF - bits, bits | 0x80000000)  # the order of the keys
+    order = np.lexsort((np.broadcast_to(np.arange(n), key.shape), -key), axis=1)[:, :k]
+    np.testing.assert_array_equal(i.cpu().numpy(), order)
+    np.testing.assert_array_equal(v.cpu().numpy(), np.take_along_axis(s.numpy(), order, axis=1))
+
+
 def test_topk_rows_errors(eng):
     s = torch.zeros(2, 100, device="cuda")
     with pytest.raises(RuntimeError, match="1 <= k <= 1024"):
