@@ -828,12 +828,9 @@ int cvs_topk_rows(const float* scores, int64_t nq, int64_t n, int64_t k, int fla
   return CVS_OK;
 }
 
-int cvs_prep_rows(const void* src, void* dst, int64_t n, int64_t d, int64_t src_stride, int64_t dst_width,
-                  int normalize, int device, void* stream) {
-  DevInfo di;
-  int rc = dev_info(device, &di);
-  if (rc != CVS_OK) return rc;
-  if (!di.gfx950) return fail(CVS_ERR_INVALID, "libcvs_hip targets gfx950 (MI355X); device %d is %s", device, di.arch);
+namespace {
+
+int check_prep(const void* src, const void* dst, int64_t n, int64_t d, int64_t src_stride, int64_t dst_width) {
   if (d < 1 || d >= INT_MAX) return fail(CVS_ERR_INVALID, "row width %lld must be in [1, 2^31)", (long long)d);
   if (dst_width < d || dst_width >= INT_MAX)
     return fail(CVS_ERR_INVALID, "destination width %lld must be in [d, 2^31)", (long long)dst_width);
@@ -845,8 +842,11 @@ int cvs_prep_rows(const void* src, void* dst, int64_t n, int64_t d, int64_t src_
     return fail(CVS_ERR_INVALID, "rows must be fp16-aligned");
   if (src == dst && src_stride != dst_width)
     return fail(CVS_ERR_INVALID, "in-place preparation needs src_stride == dst_width");
-  DeviceGuard guard(device);
-  if (guard.err != hipSuccess) return hip_fail(guard.err, "hipSetDevice");
+  return CVS_OK;
+}
+
+PrepArgs prep_args(const void* src, void* dst, int64_t n, int64_t d, int64_t src_stride, int64_t dst_width,
+                   int normalize) {
   PrepArgs a{};
   a.src = static_cast<const _Float16*>(src);
   a.dst = static_cast<_Float16*>(dst);
@@ -855,6 +855,22 @@ int cvs_prep_rows(const void* src, void* dst, int64_t n, int64_t d, int64_t src_
   a.d = (int)d;
   a.dst_width = (int)dst_width;
   a.normalize = normalize ? 1 : 0;
+  return a;
+}
+
+}  // namespace
+
+int cvs_prep_rows(const void* src, void* dst, int64_t n, int64_t d, int64_t src_stride, int64_t dst_width,
+                  int normalize, int device, void* stream) {
+  DevInfo di;
+  int rc = dev_info(device, &di);
+  if (rc != CVS_OK) return rc;
+  if (!di.gfx950) return fail(CVS_ERR_INVALID, "libcvs_hip targets gfx950 (MI355X); device %d is %s", device, di.arch);
+  rc = check_prep(src, dst, n, d, src_stride, dst_width);
+  if (rc != CVS_OK || n == 0) return rc;
+  DeviceGuard guard(device);
+  if (guard.err != hipSuccess) return hip_fail(guard.err, "hipSetDevice");
+  const PrepArgs a = prep_args(src, dst, n, d, src_stride, dst_width, normalize);
   hipError_t e = launch_prep(a, reinterpret_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "row preparation launch");
   return CVS_OK;
@@ -1388,13 +1404,14 @@ int cvs_q8_corpus_bytes(int64_t n, int64_t d, int64_t* bytes) {
   return CVS_OK;
 }
 
-int cvs_q8_build(const void* x, int64_t n, int64_t d, void* xq, int64_t xq_bytes, int device, void* stream) {
-  DevInfo di;
-  int rc = dev_info(device, &di);
-  if (rc != CVS_OK) return rc;
-  if (!di.gfx950) return fail(CVS_ERR_INVALID, "libcvs_hip targets gfx950 (MI355X); device %d is %s", device, di.arch);
+}  // extern "C"
+
+namespace {
+
+// Checks of cvs_q8_build, and its kernel arguments.
+int q8_build_args(const void* x, int64_t n, int64_t d, void* xq, int64_t xq_bytes, Q8BuildArgs* a) {
   int64_t need = 0;
-  rc = cvs_q8_corpus_bytes(n, d, &need);
+  const int rc = cvs_q8_corpus_bytes(n, d, &need);
   if (rc != CVS_OK) return rc;
   if (x == nullptr || reinterpret_cast<uintptr_t>(x) % 16 != 0) return fail(CVS_ERR_INVALID, "corpus must be 16-byte aligned");
   if (xq == nullptr || reinterpret_cast<uintptr_t>(xq) % 256 != 0)
@@ -1402,13 +1419,50 @@ int cvs_q8_build(const void* x, int64_t n, int64_t d, void* xq, int64_t xq_bytes
   if (xq_bytes < need)
     return fail(CVS_ERR_INVALID, "int8 corpus too small: need %lld bytes, got %lld", (long long)need, (long long)xq_bytes);
   const Q8Layout L = q8_layout(n, d);
+  *a = Q8BuildArgs{static_cast<const _Float16*>(x), n, (int)d, (int)L.dq, static_cast<signed char*>(xq),
+                   reinterpret_cast<float4*>(static_cast<char*>(xq) + L.off_meta),
+                   reinterpret_cast<float*>(static_cast<char*>(xq) + L.off_xmax),
+                   reinterpret_cast<int*>(static_cast<char*>(xq) + L.off_perm)};
+  return CVS_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int cvs_q8_build(const void* x, int64_t n, int64_t d, void* xq, int64_t xq_bytes, int device, void* stream) {
+  DevInfo di;
+  int rc = dev_info(device, &di);
+  if (rc != CVS_OK) return rc;
+  if (!di.gfx950) return fail(CVS_ERR_INVALID, "libcvs_hip targets gfx950 (MI355X); device %d is %s", device, di.arch);
+  Q8BuildArgs a;
+  rc = q8_build_args(x, n, d, xq, xq_bytes, &a);
+  if (rc != CVS_OK) return rc;
   DeviceGuard guard(device);
   if (guard.err != hipSuccess) return hip_fail(guard.err, "hipSetDevice");
-  Q8BuildArgs a{static_cast<const _Float16*>(x), n, (int)d, (int)L.dq, static_cast<signed char*>(xq),
-                reinterpret_cast<float4*>(static_cast<char*>(xq) + L.off_meta),
-                reinterpret_cast<float*>(static_cast<char*>(xq) + L.off_xmax),
-                reinterpret_cast<int*>(static_cast<char*>(xq) + L.off_perm)};
-  hipError_t e = launch_q8_build(a, reinterpret_cast<hipStream_t>(stream));
+  hipError_t e = launch_q8_build(a, false, reinterpret_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "int8 corpus build launch");
+  return CVS_OK;
+}
+
+int cvs_q8_prep_build(const void* src, void* dst, int64_t n, int64_t d, int64_t src_stride, int64_t dst_width,
+                      int normalize, void* xq, int64_t xq_bytes, int device, void* stream) {
+  DevInfo di;
+  int rc = dev_info(device, &di);
+  if (rc != CVS_OK) return rc;
+  if (!di.gfx950) return fail(CVS_ERR_INVALID, "libcvs_hip targets gfx950 (MI355X); device %d is %s", device, di.arch);
+  rc = check_prep(src, dst, n, d, src_stride, dst_width);
+  if (rc != CVS_OK) return rc;
+  Q8BuildArgs a;
+  rc = q8_build_args(dst, n, dst_width, xq, xq_bytes, &a);
+  if (rc != CVS_OK) return rc;
+  DeviceGuard guard(device);
+  if (guard.err != hipSuccess) return hip_fail(guard.err, "hipSetDevice");
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  PrepArgs p = prep_args(src, dst, n, d, src_stride, dst_width, normalize);
+  hipError_t e = q8_build_keys(a, &p, s);
+  if (e == hipSuccess) e = launch_prep(p, s);
+  if (e == hipSuccess) e = launch_q8_build(a, true, s);
   if (e != hipSuccess) return hip_fail(e, "int8 corpus build launch");
   return CVS_OK;
 }

@@ -158,6 +158,12 @@ struct PrepArgs {
   int d;
   int dst_width;       // elements per destination row (>= d)
   int normalize;
+  // when key is not null, also what the int8 companion's row order needs of
+  // each destination row (q8_build_keys): the bits of its largest magnitude and
+  // its id; xmax (when not null) is set to 0
+  uint16_t* key;       // [n]
+  int* ids;            // [n]
+  float* xmax;
 };
 
 // Exact selection over candidate lists: one workgroup per query.
@@ -272,7 +278,9 @@ hipError_t launch_select(int mode, const SelectArgs& a, int nq, hipStream_t s);
 hipError_t launch_rescore(const SelectArgs& a, int nq, hipStream_t s);
 hipError_t launch_prep(const PrepArgs& a, hipStream_t s);
 hipError_t launch_row_topk(const RowTopkArgs& a, int rows, hipStream_t s);
-hipError_t launch_q8_build(const Q8BuildArgs& a, hipStream_t s);
+// keyed: the row keys are in place already (launch_prep with q8_build_keys' fields)
+hipError_t launch_q8_build(const Q8BuildArgs& a, bool keyed, hipStream_t s);
+hipError_t q8_build_keys(const Q8BuildArgs& a, PrepArgs* p, hipStream_t s);
 hipError_t launch_q8_queries(const Q8QueryArgs& a, hipStream_t s);
 
 bool scan_cfg_available(const ScanCfg& cfg, int mode);

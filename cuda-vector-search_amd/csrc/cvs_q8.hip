@@ -38,7 +38,8 @@ constexpr float kNormUp = 1.0f + 1.0f / 2048.0f;  // > 1 + d * 2^-24 for d <= 81
 // like their bit patterns; NaNs are skipped as fmaxf skips them), 16 lanes per
 // row, and the row ids to carry along.
 __global__ __launch_bounds__(kBlock) void q8_rowkey_kernel(const _Float16* x, int64_t n, int d, uint16_t* key,
-                                                           int* ids) {
+                                                           int* ids, float* xmax) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *xmax = 0.f;  // (q8_build_kernel takes the maximum into it)
   const int64_t row = (int64_t)blockIdx.x * (kBlock / 16) + (threadIdx.x >> 4);
   const int l16 = threadIdx.x & 15;
   float m = 0.f;
@@ -58,77 +59,78 @@ __global__ __launch_bounds__(kBlock) void q8_rowkey_kernel(const _Float16* x, in
   }
 }
 
+// The largest magnitude of each 64-row block, the last of its rows in the sort's
+// ascending keys, into bmeta[blk].w (key is overwritten by the int8 rows), and
 // perm[r] = r for the padding rows r in [n, rows).
-__global__ __launch_bounds__(kBlock) void q8_perm_pad_kernel(int* perm, int64_t n, int64_t rows) {
-  const int64_t r = n + (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (r < rows) perm[r] = (int)r;
+__global__ __launch_bounds__(kBlock) void q8_block_max_kernel(const uint16_t* key, int* perm, float4* bmeta, int64_t n,
+                                                              int64_t nblk) {
+  const int64_t blk = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (blk >= nblk) return;
+  const int64_t last = min(64 * blk + 64, n) - 1;
+  bmeta[blk].w = (float)__builtin_bit_cast(_Float16, key[last]);
+  if (blk == nblk - 1)
+    for (int64_t r = n; r < 64 * nblk; ++r) perm[r] = (int)r;
 }
 
-// One workgroup per 64-row block of the companion; thread t takes companion
-// row t/4 (corpus row perm[t/4]) and the 8-element pieces p = t%4, t%4 + 4,
-// ... of it (4 consecutive lanes read 64 contiguous bytes).  Pass 1: block max
-// |x|; pass 2 (re-reading the rows, now in cache): quantise, write the int8 row
-// and its zero padding, and reduce the row's residual and value norms.
-__global__ __launch_bounds__(kBlock) void q8_build_kernel(Q8BuildArgs a) {
-  __shared__ float red[kBlock / kWave];
-  __shared__ float fmax_s[kBlock / kWave], xmax_s[kBlock / kWave];
+// One workgroup per 64-row block of the companion, 8 lanes per row, which read
+// corpus row perm[r] once, 128 bytes per load and kQ8Loads loads in flight, with
+// the block's scale known beforehand (q8_block_max_kernel), write the int8 row
+// and its zero padding and sum the row's norms.  Memory-bound: 2 d bytes read
+// and dq written per row.  Holding a block's rows in registers for both passes
+// (the scale found here) left one workgroup per CU at d = 1024: 1140 us for
+// 300k rows.  The whole companion build (row keys, sort, blocks), against 4
+// lanes a row and rows read twice: 500k x 768 744 -> 431 us, 300k x 1024 670 ->
+// 402 us, 500k x 384 369 -> 252 us.
+constexpr int kQ8Loads = 6;  // 8-element pieces per lane and round (dq is a multiple of 64 * 6)
+__global__ __launch_bounds__(512) void q8_build_kernel(Q8BuildArgs a) {
+  constexpr int NW = 512 / kWave;
+  __shared__ float fmax_s[NW], xmax_s[NW];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int w = tid >> 6;
   const int64_t blk = blockIdx.x;
-  const int64_t row = blk * 64 + (tid >> 2);
-  const int part = tid & 3;
+  const int64_t row = blk * 64 + (tid >> 3);
+  const int part = tid & 7;
   const bool live = row < a.n;
-  const int pieces = a.d / 8;  // 8-element pieces per row
-  const int64_t srow = live ? a.perm[row] : 0;
-  const half8* src = reinterpret_cast<const half8*>(a.x + srow * (int64_t)a.d);
-
-  float m = 0.f;
-  if (live) {
-    for (int p = part; p < pieces; p += 4) {
-      const half8 v = src[p];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) m = fmaxf(m, fabsf((float)v[j]));
-    }
-  }
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
-  if (lane == 0) red[w] = m;
-  __syncthreads();
-  const float M = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  const int np = live ? a.d / 64 : 0;  // this lane's pieces
+  const half8* src = reinterpret_cast<const half8*>(a.x + (live ? a.perm[row] : 0) * (int64_t)a.d) + part;
+  const float M = a.bmeta[blk].w;
   const float s = M / 127.f;
   const float inv = M > 0.f ? 127.f / M : 0.f;
 
-  signed char* dst = a.xq + row * (int64_t)a.dq;
+  signed char* dst = a.xq + row * (int64_t)a.dq + 8 * part;
   float ff = 0.f, xx = 0.f;
-  for (int p = part; p < pieces; p += 4) {
-    half8 v = {};
-    if (live) v = src[p];
-    int2 packed;
-    unsigned lo = 0, hi = 0;
+#pragma unroll 1
+  for (int i0 = 0; 64 * i0 < a.dq; i0 += kQ8Loads) {
+    half8 v[kQ8Loads];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float xv = (float)v[j];
-      const signed char c = q8_quant(xv, inv);
-      const float f = fmaf(-s, (float)c, xv);
-      ff = fmaf(f, f, ff);
-      xx = fmaf(xv, xv, xx);
-      if (j < 4) lo |= (unsigned)(unsigned char)c << (8 * j);
-      else hi |= (unsigned)(unsigned char)c << (8 * (j - 4));
+    for (int i = 0; i < kQ8Loads; ++i) v[i] = src[8 * max(0, min(i0 + i, np - 1))];  // (clamped: they issue together)
+#pragma unroll
+    for (int i = 0; i < kQ8Loads; ++i) {
+      if (i0 + i >= np) v[i] = half8{};
+      unsigned lo = 0, hi = 0;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float xv = (float)v[i][j];
+        const signed char c = q8_quant(xv, inv);
+        const float f = fmaf(-s, (float)c, xv);
+        ff = fmaf(f, f, ff);
+        xx = fmaf(xv, xv, xx);
+        if (j < 4) lo |= (unsigned)(unsigned char)c << (8 * j);
+        else hi |= (unsigned)(unsigned char)c << (8 * (j - 4));
+      }
+      *reinterpret_cast<int2*>(dst + 64 * (i0 + i)) = int2{(int)lo, (int)hi};  // (zero past d)
     }
-    packed.x = (int)lo;
-    packed.y = (int)hi;
-    *reinterpret_cast<int2*>(dst + 8 * p) = packed;
   }
-  for (int c = a.d + 8 * part; c < a.dq; c += 32) *reinterpret_cast<int2*>(dst + c) = int2{0, 0};
-  // row norms: the row's 4 threads are consecutive lanes
-  ff += __shfl_xor(ff, 1);
-  ff += __shfl_xor(ff, 2);
-  xx += __shfl_xor(xx, 1);
-  xx += __shfl_xor(xx, 2);
+  // row norms: the row's 8 threads are consecutive lanes
+#pragma unroll
+  for (int off = 1; off < 8; off <<= 1) {
+    ff += __shfl_xor(ff, off);
+    xx += __shfl_xor(xx, off);
+  }
   float fn = sqrtf(ff) * kNormUp, xn = sqrtf(xx) * kNormUp;
 #pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) {
+  for (int off = kWave / 2; off >= 8; off >>= 1) {
     fn = fmaxf(fn, __shfl_xor(fn, off));
     xn = fmaxf(xn, __shfl_xor(xn, off));
   }
@@ -138,25 +140,16 @@ __global__ __launch_bounds__(kBlock) void q8_build_kernel(Q8BuildArgs a) {
   }
   __syncthreads();
   if (tid == 0) {
-    float4 meta;
-    meta.x = s;
-    meta.y = fmaxf(fmaxf(fmax_s[0], fmax_s[1]), fmaxf(fmax_s[2], fmax_s[3]));
-    meta.z = fmaxf(fmaxf(xmax_s[0], xmax_s[1]), fmaxf(xmax_s[2], xmax_s[3]));
-    meta.w = 0.f;
-    a.bmeta[blk] = meta;
-  }
-}
-
-// One workgroup: the corpus-wide maximum row norm (max of the blocks' .z).
-__global__ __launch_bounds__(kBlock) void q8_xmax_kernel(const float4* bmeta, int64_t nblk, float* xmax) {
-  __shared__ float red[kBlock / kWave];
-  float m = 0.f;
-  for (int64_t b = threadIdx.x; b < nblk; b += kBlock) m = fmaxf(m, bmeta[b].z);
+    float4 meta = float4{s, fmax_s[0], xmax_s[0], 0.f};
 #pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-  __syncthreads();
-  if (threadIdx.x == 0) *xmax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    for (int i = 1; i < NW; ++i) {
+      meta.y = fmaxf(meta.y, fmax_s[i]);
+      meta.z = fmaxf(meta.z, xmax_s[i]);
+    }
+    a.bmeta[blk] = meta;
+    // the corpus-wide maximum: non-negative floats order like their bits (a NaN norm is left out)
+    if (meta.z >= 0.f) atomicMax(reinterpret_cast<int*>(a.xmax), __float_as_int(meta.z));
+  }
 }
 
 // One wave per query row; the whole grid also clears a.zero[0, nzero).
@@ -174,35 +167,61 @@ __global__ __launch_bounds__(kBlock) void q8_query_kernel(Q8QueryArgs a) {
 // live in the companion's own int8-row region (rows * dq >= 384 n bytes, far
 // more than the ~14 n bytes they take), which q8_build_kernel overwrites only
 // after the sort, in stream order: the build allocates nothing.
-hipError_t launch_q8_build(const Q8BuildArgs& a, hipStream_t s) {
-  if (a.d < 8 || a.d % 8 != 0 || a.dq < a.d || a.dq % 128 != 0 || a.perm == nullptr) return hipErrorInvalidValue;
-  const int64_t blocks = (a.n + 63) / 64;
-  if (blocks <= 0 || blocks > 0x7fffffff || a.n >= 0x7fffffff) return hipErrorInvalidValue;
-  const int64_t n = a.n, rows = blocks * 64;
-  size_t sort_bytes = 0;
-  hipError_t e = rocprim::radix_sort_pairs(nullptr, sort_bytes, (const uint16_t*)nullptr, (uint16_t*)nullptr,
-                                           (const int*)nullptr, (int*)nullptr, (unsigned)n, 0, 15, s);
+namespace {
+struct Q8SortBufs {
+  uint16_t *key_in, *key_out;
+  int* ids;
+  void* tmp;
+  size_t sort_bytes;
+};
+hipError_t q8_sort_bufs(const Q8BuildArgs& a, Q8SortBufs* b, hipStream_t s) {
+  if (a.d < 64 || a.d % 64 != 0 || a.d > 1536 || a.dq < a.d || a.dq % (64 * kQ8Loads) != 0 || a.dq > 1536 || a.perm == nullptr)
+    return hipErrorInvalidValue;
+  if (a.n < 1 || a.n >= 0x7fffffff) return hipErrorInvalidValue;
+  b->sort_bytes = 0;
+  hipError_t e = rocprim::radix_sort_pairs(nullptr, b->sort_bytes, (const uint16_t*)nullptr, (uint16_t*)nullptr,
+                                           (const int*)nullptr, (int*)nullptr, (unsigned)a.n, 0, 15, s);
   if (e != hipSuccess) return e;
-  const size_t keys_bytes = ((size_t)n * sizeof(uint16_t) + 255) / 256 * 256;
-  const size_t ids_bytes = ((size_t)n * sizeof(int) + 255) / 256 * 256;
-  if (2 * keys_bytes + ids_bytes + sort_bytes > (size_t)rows * (size_t)a.dq) return hipErrorInvalidValue;
+  const size_t keys_bytes = ((size_t)a.n * sizeof(uint16_t) + 255) / 256 * 256;
+  const size_t ids_bytes = ((size_t)a.n * sizeof(int) + 255) / 256 * 256;
+  const size_t rows = ((size_t)a.n + 63) / 64 * 64;
+  if (2 * keys_bytes + ids_bytes + b->sort_bytes > rows * (size_t)a.dq) return hipErrorInvalidValue;
   char* buf = reinterpret_cast<char*>(a.xq);
-  uint16_t* key_in = reinterpret_cast<uint16_t*>(buf);
-  uint16_t* key_out = reinterpret_cast<uint16_t*>(buf + keys_bytes);
-  int* ids = reinterpret_cast<int*>(buf + 2 * keys_bytes);
-  void* tmp = buf + 2 * keys_bytes + ids_bytes;
-  const int per = kBlock / 16;
-  hipLaunchKernelGGL(q8_rowkey_kernel, dim3((unsigned)((n + per - 1) / per)), dim3(kBlock), 0, s, a.x, n, a.d,
-                     key_in, ids);
-  e = hipGetLastError();
+  b->key_in = reinterpret_cast<uint16_t*>(buf);
+  b->key_out = reinterpret_cast<uint16_t*>(buf + keys_bytes);
+  b->ids = reinterpret_cast<int*>(buf + 2 * keys_bytes);
+  b->tmp = buf + 2 * keys_bytes + ids_bytes;
+  return hipSuccess;
+}
+}  // namespace
+
+hipError_t q8_build_keys(const Q8BuildArgs& a, PrepArgs* p, hipStream_t s) {
+  Q8SortBufs b;
+  hipError_t e = q8_sort_bufs(a, &b, s);
   if (e != hipSuccess) return e;
-  e = rocprim::radix_sort_pairs(tmp, sort_bytes, key_in, key_out, ids, a.perm, (unsigned)n, 0, 15, s);
+  p->key = b.key_in;
+  p->ids = b.ids;
+  p->xmax = a.xmax;
+  return hipSuccess;
+}
+
+hipError_t launch_q8_build(const Q8BuildArgs& a, bool keyed, hipStream_t s) {
+  Q8SortBufs b;
+  hipError_t e = q8_sort_bufs(a, &b, s);
   if (e != hipSuccess) return e;
-  if (rows > n)
-    hipLaunchKernelGGL(q8_perm_pad_kernel, dim3((unsigned)((rows - n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s,
-                       a.perm, n, rows);
-  hipLaunchKernelGGL(q8_build_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, s, a);
-  hipLaunchKernelGGL(q8_xmax_kernel, dim3(1), dim3(kBlock), 0, s, a.bmeta, blocks, a.xmax);
+  if (!keyed) {
+    const int per = kBlock / 16;
+    hipLaunchKernelGGL(q8_rowkey_kernel, dim3((unsigned)((a.n + per - 1) / per)), dim3(kBlock), 0, s, a.x, a.n, a.d,
+                       b.key_in, b.ids, a.xmax);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  e = rocprim::radix_sort_pairs(b.tmp, b.sort_bytes, b.key_in, b.key_out, b.ids, a.perm, (unsigned)a.n, 0, 15, s);
+  if (e != hipSuccess) return e;
+  const int64_t nblk = (a.n + 63) / 64;
+  hipLaunchKernelGGL(q8_block_max_kernel, dim3((unsigned)((nblk + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, b.key_out,
+                     a.perm, a.bmeta, a.n, nblk);
+  hipLaunchKernelGGL(q8_build_kernel, dim3((unsigned)nblk), dim3(512), 0, s, a);
   return hipGetLastError();
 }
 

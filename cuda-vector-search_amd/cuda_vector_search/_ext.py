@@ -150,6 +150,8 @@ def _bind(lib: ctypes.CDLL) -> ctypes.CDLL:
     lib.cvs_q8_corpus_bytes.argtypes = [i64, i64, ctypes.POINTER(i64)]
     lib.cvs_q8_build.restype = i32
     lib.cvs_q8_build.argtypes = [vp, i64, i64, vp, i64, i32, vp]
+    lib.cvs_q8_prep_build.restype = i32
+    lib.cvs_q8_prep_build.argtypes = [vp, vp, i64, i64, i64, i64, i32, vp, i64, i32, vp]
     lib.cvs_q8_plan.restype = i32
     lib.cvs_q8_plan.argtypes = [i64, i64, i64, i64, i32, i32, ctypes.POINTER(i64), ctypes.POINTER(i64)]
     lib.cvs_q8_topk.restype = i32
@@ -214,10 +216,8 @@ class Engine:
         return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
 
     # -- row preparation (index.py:27-41 on the GPU) ----------------------------
-    def prep_rows(self, src, dst, normalize: bool) -> None:
-        """dst[:, :d] = src (L2-normalised when `normalize`), dst[:, d:] = 0, in one
-        kernel.  src: [n, d] fp16 CUDA rows with unit column stride; dst: [n, w]
-        contiguous fp16, w >= d; dst may be src itself (in place, w == d)."""
+    @staticmethod
+    def _check_prep(src, dst) -> None:
         import torch
 
         if not (src.is_cuda and dst.is_cuda and src.dtype == torch.float16 and dst.dtype == torch.float16):
@@ -226,6 +226,12 @@ class Engine:
             raise RuntimeError("prep_rows needs [n, d] rows with unit column stride")
         if not dst.is_contiguous():
             raise RuntimeError("prep_rows needs a contiguous destination")
+
+    def prep_rows(self, src, dst, normalize: bool) -> None:
+        """dst[:, :d] = src (L2-normalised when `normalize`), dst[:, d:] = 0, in one
+        kernel.  src: [n, d] fp16 CUDA rows with unit column stride; dst: [n, w]
+        contiguous fp16, w >= d; dst may be src itself (in place, w == d)."""
+        self._check_prep(src, dst)
         n, d = src.shape
         rc = self.lib.cvs_prep_rows(src.data_ptr(), dst.data_ptr(), n, d, src.stride(0), dst.shape[1],
                                     1 if normalize else 0, src.device.index, self._stream(src.device))
@@ -353,6 +359,21 @@ class Engine:
         xq = torch.empty(self.q8_corpus_bytes(n, d), dtype=torch.uint8, device=x.device)
         rc = self.lib.cvs_q8_build(x.data_ptr(), n, d, xq.data_ptr(), xq.numel(), x.device.index,
                                    self._stream(x.device))
+        if rc != 0:
+            raise self._error(rc)
+        return xq
+
+    def q8_prep_build(self, src, dst, normalize: bool):
+        """prep_rows(src, dst, normalize), then q8_build(dst), in one pass less over the rows."""
+        import torch
+
+        self._check_prep(src, dst)
+        self._check_matrix(dst, "corpus")
+        n, d = src.shape
+        xq = torch.empty(self.q8_corpus_bytes(n, dst.shape[1]), dtype=torch.uint8, device=dst.device)
+        rc = self.lib.cvs_q8_prep_build(src.data_ptr(), dst.data_ptr(), n, d, src.stride(0), dst.shape[1],
+                                        1 if normalize else 0, xq.data_ptr(), xq.numel(), dst.device.index,
+                                        self._stream(dst.device))
         if rc != 0:
             raise self._error(rc)
         return xq

@@ -127,43 +127,66 @@ class Index:
         on_gpu = self.device.type == "cuda"
 
         x = src.to(self.device, torch.float16 if on_gpu else torch.float32)
-        if copy and x.data_ptr() == src.data_ptr():  # .to() returned the caller's storage
-            x = x.clone()
-        x = x.contiguous()
+        shared = x.data_ptr() == src.data_ptr()  # .to() returned the caller's storage
         # The reference asks only _ext.available() here (index.py:78); available()
         # is False when the engine library cannot be loaded, and then the index
         # uses the torch path as the reference does without its kernels.
         self._use_kernels = on_gpu and _ext.available()
-        if self._use_kernels:
-            # one HIP pass each: normalise in place (the caller's tensor too when
-            # copy=False, as in the reference), then zero-pad into a new tensor
-            eng = _ext.load()
-            if metric == "cosine" and x.shape[0] > 0:
-                eng.prep_rows(x, x, True)
-            width = x.shape[1] + (-x.shape[1]) % PAD
-            if width != x.shape[1]:
-                xp = torch.empty((x.shape[0], width), dtype=x.dtype, device=x.device)
-                eng.prep_rows(x, xp, False)
-                x = xp
-            self._x = x
-        else:
-            if metric == "cosine":
-                _normalize_(x)
-            self._x = _padded(x) if on_gpu else x
         self._xq = None
         self._xq_stamp = None  # (version, data_ptr, shape) of _x when _xq was built
         self._xq_ready = None  # event recorded after the build of _xq
         self._xq_lock = threading.Lock()
-        if self._use_kernels and int8_prefilter is not False and self._x.shape[1] <= Q8_MAX_WIDTH:
-            if int8_prefilter or int8_builds(self._x.shape[0], self._x.shape[1]):
+        if self._use_kernels:
+            if not x.is_contiguous():
+                x = x.contiguous()
+                shared = shared and x.data_ptr() == src.data_ptr()
+            self._store(x, shared, copy, int8_prefilter)
+            return
+        if copy and shared:
+            x = x.clone()
+        x = x.contiguous()
+        if metric == "cosine":
+            _normalize_(x)
+        self._x = _padded(x) if on_gpu else x
+
+    def _store(self, x: torch.Tensor, shared: bool, copy: bool, int8_prefilter: bool | None) -> None:
+        """Stores the contiguous fp16 rows ``x`` normalised (cosine), padded, and with
+        their int8 companion when there is to be one.  ``shared``: ``x`` is the
+        caller's memory, read-only when ``copy``, else normalised in place as in
+        the reference (also where padding then stores a copy).  One pass over the
+        rows where the result goes to new memory (500k x 768 cosine: a clone, an
+        in-place pass and the companion's pass for the row maxima took 283 + 605
+        + 150 us before they were one)."""
+        eng = _ext.load()
+        n, d = x.shape
+        width = d + (-d) % PAD
+        cosine = self.metric == "cosine"
+        if shared and not copy and cosine and width != d:
+            eng.prep_rows(x, x, True)
+            cosine = False
+        if (shared and copy) or width != d:
+            out = torch.empty((n, width), dtype=x.dtype, device=x.device)
+        else:
+            out = x
+        int8 = (int8_prefilter is not False and width <= Q8_MAX_WIDTH
+                and (int8_prefilter or int8_builds(n, width)))
+        self._x = out
+        if out is x and not cosine:
+            if int8:
                 self._build_int8()
+        elif int8:
+            self._set_int8(eng.q8_prep_build(x, out, cosine), self._corpus_stamp())
+        elif n > 0:
+            eng.prep_rows(x, out, cosine)
 
     def _corpus_stamp(self):
         return (self._x._version, self._x.data_ptr(), tuple(self._x.shape))
 
     def _build_int8(self) -> None:
         stamp = self._corpus_stamp()
-        xq = _ext.load().q8_build(self._x)  # enqueued on the current stream
+        self._set_int8(_ext.load().q8_build(self._x), stamp)  # enqueued on the current stream
+
+    def _set_int8(self, xq: torch.Tensor, stamp) -> None:
         ready = torch.cuda.Event()
         ready.record()
         self._xq, self._xq_stamp, self._xq_ready = xq, stamp, ready

@@ -205,6 +205,9 @@ int cvs_prep_rows(const void* src, void* dst, int64_t n, int64_t d, int64_t src_
  *   whenever x changes.  The row-order sort's keys, ids and scratch (about 14
  *   bytes per row) are placed in xq's own int8-row region before the rows
  *   are written, so the call allocates nothing.
+ * cvs_q8_prep_build: cvs_prep_rows(src, dst, ...) and then cvs_q8_build of dst
+ *   [n, dst_width], in one pass less over the rows (the preparation also notes
+ *   each row's largest magnitude).
  * cvs_q8_plan / cvs_q8_topk: as cvs_fused_plan / cvs_fused_topk (1 <= k <= 256,
  *   auto plan only; flags CVS_FLAG_IDS_INT64, and the pre-pass flags for the
  *   sampling pass), with the companion of x as xq.  plan_out[0] is the int8
@@ -216,6 +219,8 @@ int cvs_prep_rows(const void* src, void* dst, int64_t n, int64_t d, int64_t src_
  */
 int cvs_q8_corpus_bytes(int64_t n, int64_t d, int64_t* bytes);
 int cvs_q8_build(const void* x, int64_t n, int64_t d, void* xq, int64_t xq_bytes, int device, void* stream);
+int cvs_q8_prep_build(const void* src, void* dst, int64_t n, int64_t d, int64_t src_stride, int64_t dst_width,
+                      int normalize, void* xq, int64_t xq_bytes, int device, void* stream);
 int cvs_q8_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int flags, int device, int64_t* plan_out,
                 int64_t* workspace_bytes);
 int cvs_q8_topk(const void* q, const void* x, const void* xq, int64_t xq_bytes, int64_t nq, int64_t n, int64_t d,

@@ -725,6 +725,37 @@ def test_q8_build_matches_oracle(eng, n, d):
     assert np.array_equal(perm, ref_p) and raw.size == off_perm + 4 * ref_p.size
 
 
+@pytest.mark.parametrize("n,d,width", [(1, 1, 64), (65, 7, 64), (300, 100, 128), (17, 383, 384), (129, 384, 384),
+                                       (64, 387, 448), (1000, 768, 768), (33, 769, 832), (200, 1535, 1536)])
+@pytest.mark.parametrize("normalize", [False, True])
+def test_q8_prep_build_equals_its_two_steps(eng, n, d, width, normalize):
+    """Bitwise: the rows as prep_rows writes them (from an unaligned source too),
+    the companion as q8_build makes it of them."""
+    say(f"q8 prep build n={n} d={d} width={width} normalize={normalize}")
+    g = torch.Generator().manual_seed(n + d)
+    x = (torch.randn(n, d + 3, generator=g) * torch.rand(n, 1, generator=g)).half().cuda()[:, 3:]
+    x[n // 2] = 0.0
+    want = torch.empty((n, width), dtype=torch.float16, device="cuda")
+    eng.prep_rows(x, want, normalize)
+    ref = oracle.normalize_rows(x.cpu().numpy()) if normalize else x.cpu().numpy()
+    assert np.all(within_one_ulp(want[:, :d].cpu().numpy(), ref)) and not want[:, d:].any()
+    wantq = eng.q8_build(want)
+    got = torch.full((n, width), 7.0, dtype=torch.float16, device="cuda")
+    gotq = eng.q8_prep_build(x, got, normalize)
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    body = -(-n // 64) * 64 * _q8_row(width)
+    meta = body + -(-n // 64) * 16 + 4  # (up to 255 bytes of padding follow the rows, 12 the maximum norm)
+    pad = -body % 256
+    assert torch.equal(gotq[:body], wantq[:body])
+    assert torch.equal(gotq[body + pad:meta + pad], wantq[body + pad:meta + pad])
+    assert torch.equal(gotq[-4 * (-(-n // 64) * 64):], wantq[-4 * (-(-n // 64) * 64):])
+
+
+def _q8_row(width):
+    return 384 if width <= 384 else 768 if width <= 768 else 1536
+
+
 Q8_CASES = [(1, 30000, 384, 10), (7, 20000, 320, 5), (33, 25000, 384, 64), (65, 30000, 512, 10),
             (129, 20000, 768, 100), (256, 40000, 384, 10), (300, 20000, 1024, 256), (40, 20000, 1536, 1),
             # 8-wave int8 kernels with a sampled threshold and a partial last tile
