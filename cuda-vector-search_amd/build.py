@@ -42,12 +42,12 @@ FLAGS = [
     f"-I{INCLUDE}", f"-I{CSRC}",
 ]
 
-SOURCES = ["cvs_scan.hip", "cvs_scan_q8.hip", "cvs_select.hip", "cvs_rowtopk.hip", "cvs_gemv.hip", "cvs_prep.hip", "cvs_q8.hip", "cvs_capi.hip"]
+SOURCES = ["cvs_scan.hip", "cvs_gscan.hip", "cvs_scan_q8.hip", "cvs_select.hip", "cvs_rowtopk.hip", "cvs_gemv.hip", "cvs_prep.hip", "cvs_q8.hip", "cvs_capi.hip"]
 
 # Per-source extra flags.  The scan keeps its MFMA accumulators in VGPRs (the
 # query fragments are pinned in AGPRs explicitly): the epilogue then reads the
 # scores without 64 v_accvgpr_read per tile (measured 3-6% faster scan).
-MFMA_SOURCES = ["cvs_scan.hip", "cvs_scan_q8.hip"]  # kernels whose MFMA results the build checks
+MFMA_SOURCES = ["cvs_scan.hip", "cvs_gscan.hip", "cvs_scan_q8.hip"]  # kernels whose MFMA results the build checks
 EXTRA = {"cvs_scan.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "cvs_scan_q8.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
@@ -85,7 +85,7 @@ def build(jobs: int | None = None, verbose: bool = False) -> Path:
     for src in MFMA_SOURCES:
         asm = BUILD / (Path(src).stem + ".s")
         asms.append(asm)
-        cmds.append([HIPCC, *FLAGS, *EXTRA[src], "--cuda-device-only", "-S", "-c", CSRC / src, "-o", asm])
+        cmds.append([HIPCC, *FLAGS, *EXTRA.get(src, []), "--cuda-device-only", "-S", "-c", CSRC / src, "-o", asm])
     with ThreadPoolExecutor(max_workers=jobs or min(len(cmds), os.cpu_count() or 1)) as ex:
         list(ex.map(lambda c: _run(c, verbose), cmds))
     early = [p for asm in asms for p in hazard_check.check(asm)]

@@ -161,6 +161,106 @@ int64_t align_up(int64_t v, int64_t a) { return ceil_div(v, a) * a; }
 // Reference's register-state rule (kernels.cu:499,518), kept for forced plans.
 int slots_per_lane(int64_t k) { return k <= 32 ? 1 : k <= 64 ? 2 : k <= 128 ? 4 : 8; }
 
+// Time of a scan, in columns of a 128 x 128 block of scores (about 9.3 ns): each
+// of `groups` query groups over ntiles tiles in `chunks` chunks, `slots`
+// workgroups resident, `tile` columns per tile; a workgroup's start and end cost 8 us.
+// Several groups' chunks go round the 8 XCDs (the busiest one counts).
+double scan_cost(int64_t groups, int64_t ntiles, int64_t chunks, int64_t slots, double tile) {
+  const int64_t tpc = ceil_div(ntiles, chunks), used = ceil_div(ntiles, tpc);
+  const int64_t rounds = groups > 1 && chunks % 8 == 0 ? ceil_div(groups * ceil_div(used, 8), slots / 8)
+                                                       : ceil_div(groups * used, slots);
+  return (double)rounds * ((double)tpc * tile + 860.0);
+}
+
+// Chunks of a tiled-GEMM scan, one workgroup per (group, chunk): the count that
+// ends soonest, the most chunks among equals (more CUs pull the corpus from
+// HBM: 256 x 1024 over 200k rows with 128 chunks 178 us, with 112 202).  With
+// several groups a multiple of the 8 XCDs, so that a chunk's groups share one XCD's
+// L2.
+int64_t gemm_chunks(int64_t groups, int64_t ntiles, int64_t slots, int64_t max_chunks, double tile) {
+  const int64_t step = groups > 1 && ntiles >= 8 && max_chunks >= 8 ? 8 : 1;
+  const int64_t most = std::min<int64_t>({max_chunks, align_up(ntiles, step), std::max<int64_t>(step, 2 * slots)}) / step * step;
+  int64_t best = step;
+  double cost = -1;
+  for (int64_t c = step; c <= most; c += step) {
+    const double t = scan_cost(groups, ntiles, c, slots, tile);
+    if (cost < 0 || t <= cost) {
+      cost = t;
+      best = c;
+    }
+  }
+  return best;
+}
+
+// Workgroups of a tiled-GEMM scan resident on a CU: two of the small tiles
+// (80 KB of LDS each), one of the large.
+int64_t gemm_per_cu(const ScanCfg& c) { return c.qb * c.rb <= 4 ? 2 : 1; }
+
+// Columns' time of a tile of a tiled-GEMM scan: per 128 x 128 block d + 40 in a
+// 256 x 256 tile, 10% more with 128 queries, 1.15 d in two resident small
+// tiles (measured per tile: d = 1024 9.9, 9.9, 11.4 us per block, d = 768 8.7,
+// 9.5; d = 256 2.9, 3.0, 3.0; d = 128 1.7, 1.75, 1.4), for which a resident
+// small tile counts twice.  A small tile alone on its CU takes 0.85 of that.
+// One group of 128 queries waits for the corpus instead, least with the larger
+// tiles' longer stages (100 x 1024 over 600k rows: 277 us, small tiles 320).
+double gemm_tile_cost(const ScanCfg& c, int64_t d, int64_t groups, bool alone) {
+  const double blocks = 0.25 * c.qb * c.rb;
+  const bool stream = groups == 1 && c.qb == 2;
+  if (c.qb * c.rb > 4)
+    return std::max(blocks * (c.qb == 4 ? 1.0 : 1.1) * (double)(d + 40), stream ? 2.5 * (double)d : 0.0);
+  return stream && !alone ? 2.9 * (double)d : 2 * blocks * 1.15 * (double)d * (alone ? 0.85 : 1.0);
+}
+
+// The tiled-GEMM scan for an automatic plan (false: the query-stationary scan).
+// Never up to 32 queries (both are bound by the corpus stream, within 5% of
+// each other), nor where the query-stationary scan has a kernel of exactly this
+// width with enough queries per wave: 384 and 768 (1000 x 384 over 100k rows:
+// 142 us against 167-173; 256 x 768, k = 100, over 200k: 146 against 175), and up
+// to 64 queries 1536 (64 over 100k: 82 against 90-97).  Otherwise the kernel
+// whose rounds end soonest: the query-stationary scan runs 3.3 times the
+// columns' time above 768 (short fragments and half-rate MFMAs, or both operands
+// from LDS) and twice it below, but in tiles of as little as 64 x 32, which fill
+// the GPU on small corpora (156 x 1536 over 7730 rows: 45 us against 53-71).
+// Whole searches, query-stationary -> tiled (us): 794 x 1664 over 276k rows
+// 2455 -> 960, 645 x 1536 over 32k 246 -> 139, 300 x 2048 over 50k 292 -> 130,
+// 100 x 1024 over 600k 433 -> 277, 1000 x 128 over 1M 573 -> 386, 231 x 256 over 1M
+// 256 -> 220, 48 x 1024 over 600k 302 -> 250, 64 x 256 over 300k 62 -> 50.
+// Up to 64 queries the corpus stream decides between the tiles: 128 rows, two
+// a CU, below d = 1024 (64 x 256: 50 us against 55 with 256 rows), 256
+// rows from there (48 x 1024: 250 against 257).
+bool gemm_cfg(int64_t nq, int64_t n, int64_t d, int64_t k, int cus, const ScanCfg& qstat, ScanCfg* out) {
+  if (nq <= 32 || d == 384 || d == 768 || (d == 1536 && nq <= 64) || d > kGscanMaxWidth) return false;
+  // its sampling pass needs 4 tiles of 128 rows and 2k units, 8 a tile, out of a
+  // quarter of the tiles; smaller corpora keep the finer-grained scan
+  const int64_t stiles = ceil_div(n, 128) / 4;
+  if (stiles < 4 || 8 * stiles < 2 * k) return false;
+  // one group over a corpus past the MALL: both stream it, the query-stationary
+  // scan a little better (100 x 512, k = 100, over 1M rows: 269 us
+  // against 287; over 100k rows 56 against 49)
+  if (nq > 64 && nq <= 128 && d > 384 && d < 768 && n >= (1 << 19)) return false;
+  const int64_t qgroups = ceil_div(nq, qstat.bq()), qtiles = ceil_div(n, qstat.tile_rows());
+  const int64_t qchunks = std::max<int64_t>(1, std::min<int64_t>(ceil_div(cus, qgroups), qtiles / 2));
+  const double qblocks = (double)(qstat.bq() * qstat.tile_rows()) / 16384.0;
+  double cost = scan_cost(qgroups, qtiles, qchunks, cus, qblocks * (d > 768 ? 3.3 * (double)d : 2.0 * (double)(d + 40)));
+  const ScanCfg small[1] = {{32, 2, 1, d < 1024 ? 2 : 4, -1}};
+  const ScanCfg large[3] = {{32, 2, 4, 4, -1}, {32, 2, 2, 4, -1}, {32, 2, 2, 2, -1}};
+  const ScanCfg* cfgs = nq <= 64 ? small : large;
+  bool found = false;
+  for (int i = 0; i < (nq <= 64 ? 1 : 3); ++i) {
+    const ScanCfg& c = cfgs[i];
+    const int64_t groups = ceil_div(nq, c.bq()), ntiles = ceil_div(n, c.tile_rows());
+    const int64_t slots = cus * gemm_per_cu(c);
+    const double tile = gemm_tile_cost(c, d, groups, groups * ntiles <= cus);
+    const double t = scan_cost(groups, ntiles, gemm_chunks(groups, ntiles, slots, kSelectMaxLists / 2, tile), slots, tile);
+    if (t < (found ? cost : 0.85 * cost)) {  // (15%: the model's error)
+      cost = t;
+      *out = c;
+      found = true;
+    }
+  }
+  return found;
+}
+
 struct Plan {
   bool gemv = false;
   ScanCfg cfg{};
@@ -172,8 +272,10 @@ struct Plan {
   int64_t nlists = 0, cap = 0;
   // gemv
   int64_t gemv_grid = 0, rows_per_wave = 0;
-  // sampling pre-pass
+  // sampling pre-pass (of the scan's configuration, or a smaller-tiled one)
   bool prepass = false;
+  ScanCfg scfg{};
+  int64_t s_groups = 1, s_ntiles = 0;
   bool tau_in_scan = false;  // one sampling maximum per workgroup, thresholds found by the scan
   bool topk = false;         // CVS_FLAG_REGISTER_TOPK: running top-k in registers, no pre-pass
   // sampling and thresholds inside the scan (mode kAppendIn) instead of the
@@ -192,7 +294,7 @@ struct Plan {
 // int8 pre-filter samples more densely: every candidate it keeps costs a
 // random row read, so a tighter threshold pays for itself).
 int make_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int64_t bq, int64_t chunks, int flags,
-              int cus, Plan* p, int64_t sample_div = 16, bool allow_tau_in_scan = true) {
+              int cus, Plan* p, int64_t sample_div = 16, bool allow_tau_in_scan = true, bool allow_gemm = true) {
   if (k < 1 || k > 256) return fail(CVS_ERR_INVALID, "fused_topk supports 1 <= k <= 256");
   if (k > n) return fail(CVS_ERR_INVALID, "k must not exceed the corpus size");
   if (bq < 0) return fail(CVS_ERR_INVALID, "bq must be 0 (auto) or one of 16, 32, 64, 128, 256");
@@ -232,6 +334,10 @@ int make_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int64_t bq, int64_t c
       while (!cfg_for(bq, d, &tmp)) bq >>= 1;
     }
     if (!cfg_for(bq, d, &P.cfg)) return fail(CVS_ERR_INVALID, "bq=%lld is not supported at width %lld", (long long)bq, (long long)d);
+    if (ScanCfg g; allow_gemm && !forced_bq && gemm_cfg(nq, n, d, k, cus, P.cfg, &g)) {
+      P.cfg = g;
+      bq = g.bq();
+    }
     P.bq = bq;
     P.groups = ceil_div(std::max<int64_t>(nq, 1), bq);
     P.tile_rows = P.cfg.tile_rows();
@@ -243,6 +349,11 @@ int make_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int64_t bq, int64_t c
       c = std::max<int64_t>(1, std::min<int64_t>(chunks, max_chunks));
       P.tpc = ceil_div(P.ntiles, c);
       c = ceil_div(P.ntiles, P.tpc);
+    } else if (P.cfg.gemm()) {
+      c = gemm_chunks(P.groups, P.ntiles, cus * gemm_per_cu(P.cfg), max_chunks,
+                      gemm_tile_cost(P.cfg, d, P.groups, P.groups * P.ntiles <= cus));
+      P.tpc = ceil_div(P.ntiles, c);
+      if (P.groups == 1) c = ceil_div(P.ntiles, P.tpc);
     } else {
       c = std::max<int64_t>(1, ceil_div(cus, P.groups));
       c = std::min<int64_t>(c, std::max<int64_t>(1, P.ntiles / 2));
@@ -265,13 +376,21 @@ int make_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int64_t bq, int64_t c
     // maxima, so the expected number of candidates that pass it is about
     // k * ntiles / s), run by at most one workgroup per CU, each on spt
     // consecutive tiles.
-    const int64_t upt = P.cfg.units_per_tile();  // sampling units per tile
-    int64_t s = std::min<int64_t>(16384 / sample_div, std::max<int64_t>(P.ntiles / sample_div, ceil_div(8 * k, upt)));
-    s = std::min<int64_t>(s, (flags & CVS_FLAG_FORCE_PREPASS) ? P.ntiles : P.ntiles / 4);
+    // (The tiled-GEMM scan samples in its smallest tiles: more workgroups for the
+    // same sample; 645 x 1536 over 32k rows: sampling 42 -> 19 us.)
+    P.scfg = P.cfg;
+    if (P.cfg.gemm()) P.scfg = {32, 2, nq > 64 ? 2 : 1, 2, -1};
+    P.s_groups = ceil_div(std::max<int64_t>(nq, 1), P.scfg.bq());
+    P.s_ntiles = ceil_div(n, P.scfg.tile_rows());
+    const int64_t upt = P.scfg.units_per_tile();  // sampling units per tile
+    int64_t s = std::min<int64_t>(16384 / sample_div, std::max<int64_t>({P.s_ntiles / sample_div, ceil_div(8 * k, upt),
+                                                                         P.scfg.gemm() ? 4 : 0}));
+    s = std::min<int64_t>(s, (flags & CVS_FLAG_FORCE_PREPASS) ? P.s_ntiles : P.s_ntiles / 4);
     P.prepass = !(flags & CVS_FLAG_NO_PREPASS) &&
                 (((flags & CVS_FLAG_FORCE_PREPASS) && s >= 1) || (s >= 4 && s * upt >= 2 * k));
     if (P.prepass) {
-      const int64_t wgs = std::max<int64_t>(1, std::min<int64_t>(s, cus / P.groups));
+      const int64_t s_slots = cus * (P.scfg.gemm() ? gemm_per_cu(P.scfg) : 1);
+      const int64_t wgs = std::max<int64_t>(1, std::min<int64_t>(s, s_slots / P.s_groups));
       P.spt = std::max<int64_t>(1, s / wgs);
       P.nsample = wgs;
       // One unit per (workgroup, row split, lane group) when that still leaves
@@ -398,7 +517,7 @@ namespace {
 // or GEMV, 3 final select; skipped stages get back-to-back marks.
 int run_fused(const void* q, const void* x, int64_t nq, int64_t n, int64_t d, int64_t k, int64_t bq,
               int64_t chunks, int flags, void* workspace, int64_t workspace_bytes, float* out_v,
-              void* out_i, int64_t* plan_out, int device, void* stream, hipEvent_t* marks) {
+              void* out_i, int64_t* plan_out, int device, void* stream, hipEvent_t* marks, bool allow_gemm = true) {
   DevInfo di;
   int rc = dev_info(device, &di);
   if (rc != CVS_OK) return rc;
@@ -406,7 +525,7 @@ int run_fused(const void* q, const void* x, int64_t nq, int64_t n, int64_t d, in
   rc = check_inputs(q, x, nq, n, d);
   if (rc != CVS_OK) return rc;
   Plan P;
-  rc = make_plan(nq, n, d, k, bq, chunks, flags, di.cus, &P);
+  rc = make_plan(nq, n, d, k, bq, chunks, flags, di.cus, &P, 16, true, allow_gemm);
   if (rc != CVS_OK) return rc;
   if (plan_out) {
     plan_out[0] = P.bq;
@@ -510,10 +629,12 @@ int run_fused(const void* q, const void* x, int64_t nq, int64_t n, int64_t d, in
       pa.nsample = (int)P.nsample;
       pa.spt = (int)P.spt;
       pa.agg = P.agg;
+      pa.groups = (int)P.s_groups;
+      pa.ntiles = P.s_ntiles;
       // two query groups of one sampled chunk on one XCD: its rows come from HBM once
-      pa.xcd_pair = (P.groups > 1 && P.nsample % 8 == 0) ? 1 : 0;
+      pa.xcd_pair = (P.s_groups > 1 && P.nsample % 8 == 0) ? 1 : 0;
       pa.units = (int)P.units;
-      e = launch_scan(P.cfg, kMax, pa, (int)(P.groups * P.nsample), s);
+      e = launch_scan(P.scfg, kMax, pa, (int)(P.s_groups * P.nsample), s);
       if (e != hipSuccess) return hip_fail(e, "sample pass launch");
       mark(1);
       if (P.tau_in_scan) {  // the scan takes the k-th largest of each query's maxima itself
@@ -644,6 +765,13 @@ int cvs_fused_topk_noalloc(const void* q, const void* x, int64_t nq, int64_t n, 
   Plan P;
   rc = make_plan(nq, n, d, k, 0, 0, flags, di.cus, &P);
   if (rc != CVS_OK) return rc;
+  // the tiled-GEMM scan keeps more lists per query: where they do not fit, the
+  // query-stationary one
+  const bool allow_gemm = P.ws_bytes <= kScratchBytes;
+  if (!allow_gemm) {
+    rc = make_plan(nq, n, d, k, 0, 0, flags, di.cus, &P, 16, true, false);
+    if (rc != CVS_OK) return rc;
+  }
   if (P.ws_bytes > kScratchBytes)
     return fail(CVS_ERR_INVALID,
                 "the allocation-free search needs %lld bytes of workspace for these sizes, more than its "
@@ -659,7 +787,7 @@ int cvs_fused_topk_noalloc(const void* q, const void* x, int64_t nq, int64_t n, 
   // The fused path needs no zeroed workspace (every list count and threshold is
   // written before it is read), so nothing is cleared here.
   return run_fused(q, x, nq, n, d, k, 0, 0, flags, ws, kScratchBytes, out_v, out_i, plan_out, device, stream,
-                   nullptr);
+                   nullptr, allow_gemm);
 }
 
 int cvs_fused_topk_marked(const void* q, const void* x, int64_t nq, int64_t n, int64_t d, int64_t k,
@@ -948,7 +1076,7 @@ int make_q8_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int flags, int cus
     return fail(CVS_ERR_INVALID, "the int8 pre-filter supports widths up to %lld, not %lld", (long long)kQ8MaxWidth,
                 (long long)d);
   Q8Plan P;
-  int rc = make_plan(nq, n, d, k, 0, 0, flags, cus, &P.sample, kQ8SampleDiv, false);
+  int rc = make_plan(nq, n, d, k, 0, 0, flags, cus, &P.sample, kQ8SampleDiv, false, false);
   if (rc != CVS_OK) return rc;
   P.dq = q8_row_bytes(d);
   const int ks = (int)(P.dq / 32);

@@ -235,7 +235,8 @@ struct Q8QueryArgs {
 
 // Scan configurations: MFMA shape ms (16 or 32), queries per wave 16*... = ms*qb,
 // tile rows = rs*rb*ms, widest row = ksmax * (ms == 16 ? 32 : 16); ksmax = 0:
-// rows of any width (queries staged through LDS instead of held in registers).
+// rows of any width (queries staged through LDS instead of held in registers);
+// ksmax = -1 (ms = 32, qs = 2): the tiled-GEMM scan (cvs_gscan.hip), any width.
 // Row splits of a scan configuration (waves = qs * rs): 4 waves, one per SIMD,
 // except 8 (two per SIMD) for qs = 8.
 constexpr int scan_row_splits(int qs) { return qs >= 4 ? 1 : 4 / qs; }
@@ -248,11 +249,15 @@ struct ScanCfg {
   int tile_rows() const { return rs() * rb * ms; }
   int wave_rows() const { return rb * ms; }
   int dmax() const { return ksmax * (ms == 16 ? 32 : 16); }  // 0: no limit
-  int units_per_tile() const { return rs() * (64 / ms); }
+  bool gemm() const { return ksmax < 0; }
+  int units_per_tile() const { return rs() * (64 / ms) * (gemm() ? rb : 1); }
 };
+constexpr int64_t kGscanMaxWidth = 1 << 16;  // (32-bit byte offsets within a tile)
 
 // Returns hipErrorInvalidValue when no kernel is instantiated for (cfg, mode).
 hipError_t launch_scan(const ScanCfg& cfg, int mode, const ScanArgs& a, int grid, hipStream_t s);
+// cfg.gemm(): modes kAppend and kMax of configs {32, 2, 4, 4, -1}, {32, 2, 2, 4, -1} and {32, 2, 2, 2, -1}.
+hipError_t launch_gscan(const ScanCfg& cfg, int mode, const ScanArgs& a, int grid, hipStream_t s);
 // Mode kTopK: instantiated for cfg {32, 1, 1, 1, 24} only (batches <= 32, width <= 384).
 bool scan_topk_available(const ScanCfg& cfg, int64_t d, int64_t k);
 hipError_t launch_scan_topk(const ScanCfg& cfg, const ScanArgs& a, int grid, hipStream_t s);

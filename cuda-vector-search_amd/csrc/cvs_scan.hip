@@ -1420,6 +1420,7 @@ bool scan_cfg_available(const ScanCfg& c, int mode) {
 }
 
 hipError_t launch_scan(const ScanCfg& c, int mode, const ScanArgs& a, int grid, hipStream_t s) {
+  if (c.gemm()) return launch_gscan(c, mode, a, grid, s);
   if (mode == kAppendQ8 || mode == kMaxQ8) {
 #define CVS_LAUNCH_Q8(MS, QS, QB, RB, KS)                                      \
   if (c.ms == MS && c.qs == QS && c.qb == QB && c.rb == RB && c.ksmax == KS) \

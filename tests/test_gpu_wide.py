@@ -177,3 +177,66 @@ def test_wide_int8_is_refused_by_the_engine(eng):
         eng.q8_build(x)
     with pytest.raises(RuntimeError, match="widths up to 1536"):
         eng.q8_plan(4, 128, 2048, 10)
+
+
+# The tiled-GEMM scan (every auto plan past 32 queries at widths other than 384
+# and 768, once the corpus is large enough): each tile shape, widths of one
+# stage and up, partial tiles and query blocks, a chunk of one tile, several
+# groups, ties and lists that fill.
+@pytest.mark.parametrize("nq,n,d,k", [
+    (33, 4097, 64, 1), (64, 20001, 128, 100), (40, 9000, 1024, 10),          # 64-query tiles, 128 and 256 rows
+    (65, 30001, 256, 10), (128, 70000, 1024, 64), (100, 33000, 1600, 256),   # 128-query tiles
+    (257, 40003, 192, 17), (600, 50000, 1088, 100), (513, 20000, 2048, 5),   # several groups
+])
+def test_tiled_scan_is_exact(eng, nq, n, d, k):
+    say(f"tiled scan nq={nq} n={n} d={d} k={k}")
+    x, q = make(n, d, nq, seed=n + d + k)
+    x[n // 2:n // 2 + 40] = x[3]  # exact ties
+    q[1] = x[3]
+    plan, _ = eng.plan(nq, n, d, k)
+    assert plan[0] in (64, 128, 256)
+    xd, qd = x.cuda(), q.cuda()
+    v, i, _ = eng.fused_topk(qd, xd, k)
+    forced = 16 if d > 768 or k > 128 else 32  # the query-stationary scan
+    v2, i2, p2 = eng.fused_topk(qd, xd, k, bq=forced)
+    torch.cuda.synchronize()
+    assert p2.tolist()[0] == forced
+    oracle.check_exact(q, x, k, v.cpu().numpy(), i.cpu().numpy())
+    # both sum the fp16 products in fp32 (in other orders): |S - S'| <= 2 d 2^-24 |q||x|
+    torch.testing.assert_close(v, v2, rtol=0, atol=2 * d * 2.0**-24)
+    assert (i != i2).float().mean().item() < 0.02
+
+
+@pytest.mark.parametrize("nq,n,d,k", [(200, 30000, 1024, 10), (300, 20000, 128, 200)])
+def test_tiled_scan_cuts_full_lists(eng, nq, n, d, k):
+    """Rows in ascending order of their scores fill every list many times over
+    (no sampling), so that lists are cut to their k best as they go."""
+    say(f"tiled scan, full lists nq={nq} n={n} d={d} k={k}")
+    g = torch.Generator().manual_seed(5)
+    base = torch.nn.functional.normalize(torch.randn(1, d, generator=g), dim=1)
+    x = (base * torch.linspace(0.1, 1.0, n)[:, None] + 0.001 * torch.randn(n, d, generator=g)).half()
+    q = (base + 0.01 * torch.randn(nq, d, generator=g)).half()
+    v, i, _ = eng.fused_topk(q.cuda(), x.cuda(), k, flags=_ext.FLAG_NO_PREPASS)
+    v2, i2, _ = eng.fused_topk(q.cuda(), x.cuda(), k)
+    torch.cuda.synchronize()
+    assert torch.equal(v, v2) and torch.equal(i, i2)
+    oracle.check_exact(q, x, k, v.cpu().numpy(), i.cpu().numpy())
+
+
+def test_noalloc_keeps_what_its_scratch_held(eng):
+    """The allocation-free search of sizes whose tiled plan outgrows its scratch
+    runs the query-stationary plan, as it did."""
+    nq, n, d, k = 1000, 200000, 128, 10
+    _, ws = eng.plan(nq, n, d, k)
+    assert ws > _ext.NOALLOC_SCRATCH_BYTES
+    x, q = make(n, d, nq, seed=9)
+    xd, qd = x.cuda(), q.cuda()
+    v = torch.empty((nq, k), dtype=torch.float32, device="cuda")
+    i = torch.empty((nq, k), dtype=torch.int32, device="cuda")
+    rc = eng.lib.cvs_fused_topk_noalloc(qd.data_ptr(), xd.data_ptr(), nq, n, d, k, 0, v.data_ptr(), i.data_ptr(), None,
+                                        0, eng._stream(qd.device))
+    assert rc == 0, eng.lib.cvs_last_error()
+    v2, i2, _ = eng.fused_topk(qd, xd, k)
+    torch.cuda.synchronize()
+    torch.testing.assert_close(v, v2, rtol=0, atol=2 * d * 2.0**-24)
+    assert (i != i2).float().mean().item() < 0.001
