@@ -13,10 +13,13 @@
 // padding columns zeroed.  Source and destination may be the same rows (the
 // group reads its whole row before writing it).  Memory-bound: 2*d bytes read
 // and 2*width bytes written per row; 16 lanes a row read 256 consecutive bytes
-// per load and keep 3 to 12 loads in flight each.
+// per load and keep 3 to 12 loads in flight each.  The sum of squares is in
+// fp64 and the scaling a two-float product: fewer instructions than an fp32
+// division, and the fp32 quotient is the nearest one whatever the order of the
+// sum (an fp32 norm moved one stored element in ~2^14 by an fp16 step).
 //
-// 500k x 768, normalised: 602 us with one wave a row and 2-byte loads, 303 us
-// (5.1 TB/s) so; 300k x 777, padded to 832: 381 -> 193 us.
+// 500k x 768, normalised: 602 us with one wave a row and 2-byte loads, 266 us
+// (5.8 TB/s) so; 300k x 777, padded to 832: 381 -> 184 us.
 #include "cvs_common.h"
 #include "cvs_kernels.h"
 
@@ -54,10 +57,10 @@ __global__ __launch_bounds__(kBlock) void prep_rows_kernel(PrepArgs a) {
     }
     return v;
   };
-  float ss = 0.f;
+  double ss = 0.;  // the squares are exact in fp32
   auto add = [&](const half8& v) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) ss += (float)v[j] * (float)v[j];
+    for (int j = 0; j < 8; ++j) ss += (double)((float)v[j] * (float)v[j]);
   };
   half8 v[P ? P : 1];
   if constexpr (P > 0) {
@@ -69,17 +72,31 @@ __global__ __launch_bounds__(kBlock) void prep_rows_kernel(PrepArgs a) {
 #pragma unroll 4
     for (int c = l; c < np; c += LPR) add(piece(c));
   }
-  float nrm = 1.f;
-  if (a.normalize) {  // x / max(||x||, 1e-12), divided per element like the reference
+  float inv = 1.f, inv_lo = 0.f;  // 1 / max(||x||, 1e-12) as a sum of two floats
+  if (a.normalize) {
 #pragma unroll
     for (int off = LPR / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
-    nrm = fmaxf(sqrtf(ss), 1e-12f);
+    double r = (double)rsqrtf((float)ss);
+    r *= 1.5 - 0.5 * ss * r * r;  // a Newton step: 2^-24 -> 2^-46
+    if (ss < 1e-24) r = 1e12;
+    if (ss > 1e30) r = 0.;  // an infinite element: the finite ones become 0, as divided by infinity
+    inv = (float)r;
+    inv_lo = (float)(r - (double)inv);
   }
+  // The fp32 number nearest to x / ||x||, then fp16 as the reference rounds.
+  auto scaled = [&](_Float16 h) {
+#pragma clang fp contract(off)
+    const float x = (float)h;
+    const float p = x * inv;
+    float r = p - fmaf(-x, inv_lo, fmaf(-x, inv, p));  // (keeps the sign of a zero)
+    asm("" : "+v"(r));  // rounded to fp32 before fp16 (not a mixed-precision fma), as the reference's quotient
+    return (_Float16)r;
+  };
   float m = 0.f;  // the stored row's largest magnitude (NaNs skipped)
   auto put = [&](int c, half8 x) {
     if (a.normalize)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) x[j] = (_Float16)((float)x[j] / nrm);
+      for (int j = 0; j < 8; ++j) x[j] = scaled(x[j]);
     if (a.key != nullptr)
 #pragma unroll
       for (int j = 0; j < 8; ++j) m = fmaxf(m, fabsf((float)x[j]));
