@@ -172,12 +172,15 @@ double scan_cost(int64_t groups, int64_t ntiles, int64_t chunks, int64_t slots, 
   return (double)rounds * ((double)tpc * tile + 860.0);
 }
 
-// Chunks of a tiled-GEMM scan, one workgroup per (group, chunk): the count that
-// ends soonest, the most chunks among equals (more CUs pull the corpus from
+// Chunks of a scan, one workgroup per (group, chunk): the count that ends
+// soonest, the most chunks among equals (more CUs pull the corpus from
 // HBM: 256 x 1024 over 200k rows with 128 chunks 178 us, with 112 202).  With
 // several groups a multiple of the 8 XCDs, so that a chunk's groups share one XCD's
-// L2.
-int64_t gemm_chunks(int64_t groups, int64_t ntiles, int64_t slots, int64_t max_chunks, double tile) {
+// L2.  (A workgroup per CU, rounded up to such a multiple, overran the GPU at 3, 5,
+// 6 and 7 groups and left a second round nearly empty: 600 x 384 over 1M rows
+// through the int8 path 522 us, now 425; 700 x 768 over 200k 461 -> 316; 700 x 768,
+// k = 100, over 1M 1404 -> 986; scores of 300 x 768 over 100k 137 -> 87.)
+int64_t best_chunks(int64_t groups, int64_t ntiles, int64_t slots, int64_t max_chunks, double tile) {
   const int64_t step = groups > 1 && ntiles >= 8 && max_chunks >= 8 ? 8 : 1;
   const int64_t most = std::min<int64_t>({max_chunks, align_up(ntiles, step), std::max<int64_t>(step, 2 * slots)}) / step * step;
   int64_t best = step;
@@ -190,6 +193,14 @@ int64_t gemm_chunks(int64_t groups, int64_t ntiles, int64_t slots, int64_t max_c
     }
   }
   return best;
+}
+
+// Columns' time of a tile of the query-stationary scan: 3.3 times that of the
+// tiled-GEMM scan above 768 columns (short fragments and half-rate MFMAs, or both
+// operands from LDS), twice it below (about it at exactly 384 and 768).
+double qstat_tile_cost(const ScanCfg& c, int64_t d) {
+  const double blocks = (double)(c.bq() * c.tile_rows()) / 16384.0;
+  return blocks * (d > 768 ? 3.3 * (double)d : (d == 384 || d == 768 ? 1.2 : 2.0) * (double)(d + 40));
 }
 
 // Workgroups of a tiled-GEMM scan resident on a CU: two of the small tiles
@@ -217,10 +228,9 @@ double gemm_tile_cost(const ScanCfg& c, int64_t d, int64_t groups, bool alone) {
 // width with enough queries per wave: 384 and 768 (1000 x 384 over 100k rows:
 // 142 us against 167-173; 256 x 768, k = 100, over 200k: 146 against 175), and up
 // to 64 queries 1536 (64 over 100k: 82 against 90-97).  Otherwise the kernel
-// whose rounds end soonest: the query-stationary scan runs 3.3 times the
-// columns' time above 768 (short fragments and half-rate MFMAs, or both operands
-// from LDS) and twice it below, but in tiles of as little as 64 x 32, which fill
-// the GPU on small corpora (156 x 1536 over 7730 rows: 45 us against 53-71).
+// whose rounds end soonest: the query-stationary scan's tiles take longer but
+// are as small as 64 x 32, which fill the GPU on small corpora (156 x 1536 over
+// 7730 rows: 45 us against 53-71).
 // Whole searches, query-stationary -> tiled (us): 794 x 1664 over 276k rows
 // 2455 -> 960, 645 x 1536 over 32k 246 -> 139, 300 x 2048 over 50k 292 -> 130,
 // 100 x 1024 over 600k 433 -> 277, 1000 x 128 over 1M 573 -> 386, 231 x 256 over 1M
@@ -240,8 +250,7 @@ bool gemm_cfg(int64_t nq, int64_t n, int64_t d, int64_t k, int cus, const ScanCf
   if (nq > 64 && nq <= 128 && d > 384 && d < 768 && n >= (1 << 19)) return false;
   const int64_t qgroups = ceil_div(nq, qstat.bq()), qtiles = ceil_div(n, qstat.tile_rows());
   const int64_t qchunks = std::max<int64_t>(1, std::min<int64_t>(ceil_div(cus, qgroups), qtiles / 2));
-  const double qblocks = (double)(qstat.bq() * qstat.tile_rows()) / 16384.0;
-  double cost = scan_cost(qgroups, qtiles, qchunks, cus, qblocks * (d > 768 ? 3.3 * (double)d : 2.0 * (double)(d + 40)));
+  double cost = scan_cost(qgroups, qtiles, qchunks, cus, qstat_tile_cost(qstat, d));
   const ScanCfg small[1] = {{32, 2, 1, d < 1024 ? 2 : 4, -1}};
   const ScanCfg large[3] = {{32, 2, 4, 4, -1}, {32, 2, 2, 4, -1}, {32, 2, 2, 2, -1}};
   const ScanCfg* cfgs = nq <= 64 ? small : large;
@@ -251,7 +260,7 @@ bool gemm_cfg(int64_t nq, int64_t n, int64_t d, int64_t k, int cus, const ScanCf
     const int64_t groups = ceil_div(nq, c.bq()), ntiles = ceil_div(n, c.tile_rows());
     const int64_t slots = cus * gemm_per_cu(c);
     const double tile = gemm_tile_cost(c, d, groups, groups * ntiles <= cus);
-    const double t = scan_cost(groups, ntiles, gemm_chunks(groups, ntiles, slots, kSelectMaxLists / 2, tile), slots, tile);
+    const double t = scan_cost(groups, ntiles, best_chunks(groups, ntiles, slots, kSelectMaxLists / 2, tile), slots, tile);
     if (t < (found ? cost : 0.85 * cost)) {  // (15%: the model's error)
       cost = t;
       *out = c;
@@ -350,22 +359,16 @@ int make_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int64_t bq, int64_t c
       P.tpc = ceil_div(P.ntiles, c);
       c = ceil_div(P.ntiles, P.tpc);
     } else if (P.cfg.gemm()) {
-      c = gemm_chunks(P.groups, P.ntiles, cus * gemm_per_cu(P.cfg), max_chunks,
+      c = best_chunks(P.groups, P.ntiles, cus * gemm_per_cu(P.cfg), max_chunks,
                       gemm_tile_cost(P.cfg, d, P.groups, P.groups * P.ntiles <= cus));
       P.tpc = ceil_div(P.ntiles, c);
       if (P.groups == 1) c = ceil_div(P.ntiles, P.tpc);
     } else {
-      c = std::max<int64_t>(1, ceil_div(cus, P.groups));
-      c = std::min<int64_t>(c, std::max<int64_t>(1, P.ntiles / 2));
-      c = std::min<int64_t>(c, max_chunks);
-      if (P.groups > 1 && c >= 8) {
-        // keep the XCD-aware mapping exact: chunk count a multiple of the 8 XCDs
-        c = std::min<int64_t>(align_up(c, 8), (max_chunks / 8) * 8);
-        P.tpc = ceil_div(P.ntiles, c);
-      } else {
-        P.tpc = ceil_div(P.ntiles, c);
-        c = ceil_div(P.ntiles, P.tpc);
-      }
+      const int64_t most = std::min<int64_t>(max_chunks, std::max<int64_t>(1, P.groups > 1 ? align_up(P.ntiles / 2, 8) : P.ntiles / 2));
+      c = P.groups == 1 ? std::min<int64_t>(cus, most)
+                        : best_chunks(P.groups, P.ntiles, cus, most, qstat_tile_cost(P.cfg, d));
+      P.tpc = ceil_div(P.ntiles, c);
+      if (P.groups == 1 || c % 8 != 0) c = ceil_div(P.ntiles, P.tpc);
     }
     P.chunks = c;
     P.xcd_pair = (P.groups > 1 && c % 8 == 0) ? 1 : 0;
@@ -822,18 +825,12 @@ int cvs_scores(const void* q, const void* x, int64_t nq, int64_t n, int64_t d, v
   const int64_t groups = ceil_div(nq, bq);
   const int64_t ntiles = ceil_div(n, cfg.tile_rows());
   const int64_t max_chunks = std::min<int64_t>(ntiles, 65535);
-  int64_t c = std::max<int64_t>(1, ceil_div(di.cus, groups));
-  c = std::min<int64_t>({c, std::max<int64_t>(1, ntiles / 2), max_chunks});
-  int64_t tpc;
-  int xcd_pair = 0;
-  if (groups > 1 && c >= 8) {
-    c = std::min<int64_t>(align_up(c, 8), (max_chunks / 8) * 8);
-    tpc = ceil_div(ntiles, c);
-    xcd_pair = 1;
-  } else {
-    tpc = ceil_div(ntiles, c);
-    c = ceil_div(ntiles, tpc);
-  }
+  const int64_t most = std::min<int64_t>(max_chunks, std::max<int64_t>(1, groups > 1 ? align_up(ntiles / 2, 8) : ntiles / 2));
+  int64_t c = groups == 1 ? std::min<int64_t>(di.cus, most)
+                          : best_chunks(groups, ntiles, di.cus, most, qstat_tile_cost(cfg, d));
+  const int64_t tpc = ceil_div(ntiles, c);
+  const int xcd_pair = groups > 1 && c % 8 == 0 ? 1 : 0;
+  if (!xcd_pair) c = ceil_div(ntiles, tpc);
   if (groups * c > INT_MAX) return fail(CVS_ERR_INVALID, "too many queries");
 
   DeviceGuard guard(device);
@@ -1109,16 +1106,11 @@ int make_q8_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int flags, int cus
     P.ntiles = ceil_div(n, P.cfg.tile_rows());
     const int64_t rs = P.cfg.rs();
     const int64_t max_chunks = std::min<int64_t>({P.ntiles, 65535, kSelectMaxLists / rs});
-    int64_t c = std::max<int64_t>(1, ceil_div(cus, P.groups));
-    c = std::min<int64_t>(c, std::max<int64_t>(1, P.ntiles / 2));
-    c = std::min<int64_t>(c, max_chunks);
-    if (P.groups > 1 && c >= 8) {
-      c = std::min<int64_t>(align_up(c, 8), (max_chunks / 8) * 8);
-      P.tpc = ceil_div(P.ntiles, c);
-    } else {
-      P.tpc = ceil_div(P.ntiles, c);
-      c = ceil_div(P.ntiles, P.tpc);
-    }
+    const int64_t most = std::min<int64_t>(max_chunks, std::max<int64_t>(1, P.groups > 1 ? align_up(P.ntiles / 2, 8) : P.ntiles / 2));
+    int64_t c = P.groups == 1 ? std::min<int64_t>(cus, most)  // (an int8 column's time is half an fp16 one's)
+                              : best_chunks(P.groups, P.ntiles, cus, most, 0.5 * qstat_tile_cost(P.cfg, P.dq));
+    P.tpc = ceil_div(P.ntiles, c);
+    if (P.groups == 1 || c % 8 != 0) c = ceil_div(P.ntiles, P.tpc);
     P.chunks = c;
     P.xcd_pair = (P.groups > 1 && c % 8 == 0) ? 1 : 0;
     P.nlists = c * rs;

@@ -240,3 +240,16 @@ def test_noalloc_keeps_what_its_scratch_held(eng):
     torch.cuda.synchronize()
     torch.testing.assert_close(v, v2, rtol=0, atol=2 * d * 2.0**-24)
     assert (i != i2).float().mean().item() < 0.001
+
+
+@pytest.mark.parametrize("nq,n,d,k", [(513, 9000, 384, 10), (700, 4100, 768, 20), (300, 2100, 768, 5), (257, 600, 320, 3)])
+def test_several_query_groups_are_exact(eng, nq, n, d, k):
+    """3, 5 and 6 query groups: chunk counts that are multiples of 8 and not, some
+    chunks empty, on every path that splits its corpus by groups."""
+    say(f"groups nq={nq} n={n} d={d} k={k}")
+    x, q = make(n, d, nq, seed=nq + n)
+    index = Index(x.cuda(), metric="ip", int8_prefilter=True)
+    for method in ("fused", "int8"):
+        v, i = index.search(q.cuda(), k, method=method)
+        oracle.check_exact(q, x, k, v.cpu().numpy(), i.cpu().numpy())
+    np.testing.assert_allclose(index.scores(q.cuda()).cpu().numpy(), oracle.scores(q, x), rtol=0, atol=1e-3)
