@@ -181,13 +181,15 @@ double scan_cost(int64_t groups, int64_t ntiles, int64_t chunks, int64_t slots, 
 // through the int8 path 522 us, now 425; 700 x 768 over 200k 461 -> 316; 700 x 768,
 // k = 100, over 1M 1404 -> 986; scores of 300 x 768 over 100k 137 -> 87.)
 int64_t best_chunks(int64_t groups, int64_t ntiles, int64_t slots, int64_t max_chunks, double tile) {
-  const int64_t step = groups > 1 && ntiles >= 8 && max_chunks >= 8 ? 8 : 1;
-  const int64_t most = std::min<int64_t>({max_chunks, align_up(ntiles, step), std::max<int64_t>(step, 2 * slots)}) / step * step;
+  if (groups == 1) return std::max<int64_t>(1, std::min<int64_t>({slots, ntiles, max_chunks}));
+  const int64_t step = ntiles >= 8 && max_chunks >= 8 ? 8 : 1;
+  const int64_t most = std::min<int64_t>(max_chunks, align_up(ntiles, step)) / step * step;
   int64_t best = step;
   double cost = -1;
-  for (int64_t c = step; c <= most; c += step) {
+  for (int r = 1; r <= 3; ++r) {  // the most chunks that r rounds hold
+    const int64_t c = std::max<int64_t>(step, std::min<int64_t>(most, r * slots / (groups * step) * step));
     const double t = scan_cost(groups, ntiles, c, slots, tile);
-    if (cost < 0 || t <= cost) {
+    if (cost < 0 || t < cost || (t == cost && c > best)) {
       cost = t;
       best = c;
     }
@@ -270,7 +272,28 @@ bool gemm_cfg(int64_t nq, int64_t n, int64_t d, int64_t k, int cus, const ScanCf
   return found;
 }
 
+// Whether a search of few rows scores them all into a matrix and takes each
+// row's top k whole (two launches, one workgroup a row) instead of sampling,
+// filtering into lists and selecting (three to five).  Measured (us, GPU time,
+// lists / matrix): always where the corpus is too small to sample for this k,
+// whose lists then fill and are cut over and over (1000 x 768 over 16000 rows, k =
+// 100 988 / 100; 40 x 384 over 1000, k = 10 29 / 16); long results up to 16k rows
+// (200 x 384 over 16000, k = 100 111 / 36; past it only small batches: 8 x 768 over
+// 32000 40 / 34, 40 x 384 26 / 35); short ones while few scores are stored, more of
+// them where the scans are slow (1 x 384 over 5000, k = 10 19 / 9, over 32000
+// 20 / 24; 200 x 384 over 8000 28 / 26, 1000 x 384 42 / 50; 200 x 768 over
+// 16000 39 / 34).
+constexpr int64_t kDirectBytes = 256ll << 20;  // of scores (the MALL holds them)
+bool direct_search(int64_t nq, int64_t n, int64_t d, int64_t k, bool sampled) {
+  if (n > kRowDirect || nq * n * 4 > kDirectBytes) return false;
+  if (!sampled) return true;
+  if (k >= 32) return nq <= 16 || (n <= 16384 && nq * n <= 8000000);
+  if (nq == 1) return n <= 16384 || d >= 768;
+  return d >= 768 ? n <= 16384 && nq * n <= 3300000 : n <= 8192 && nq * n <= 1700000;
+}
+
 struct Plan {
+  bool direct = false;  // score matrix (off_lv) and whole-row top k
   bool gemv = false;
   ScanCfg cfg{};
   int64_t bq = 0;       // reported plan[0]
@@ -301,9 +324,11 @@ struct Plan {
 
 // sample_div: the sampling pre-pass scores about 1/sample_div of the tiles (the
 // int8 pre-filter samples more densely: every candidate it keeps costs a
-// random row read, so a tighter threshold pays for itself).
+// random row read, so a tighter threshold pays for itself).  allow_lean: the
+// tiled-GEMM scan and the score-matrix search may be taken (their workspaces
+// are larger than the query-stationary scan's).
 int make_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int64_t bq, int64_t chunks, int flags,
-              int cus, Plan* p, int64_t sample_div = 16, bool allow_tau_in_scan = true, bool allow_gemm = true) {
+              int cus, Plan* p, int64_t sample_div = 16, bool allow_tau_in_scan = true, bool allow_lean = true) {
   if (k < 1 || k > 256) return fail(CVS_ERR_INVALID, "fused_topk supports 1 <= k <= 256");
   if (k > n) return fail(CVS_ERR_INVALID, "k must not exceed the corpus size");
   if (bq < 0) return fail(CVS_ERR_INVALID, "bq must be 0 (auto) or one of 16, 32, 64, 128, 256");
@@ -343,7 +368,7 @@ int make_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int64_t bq, int64_t c
       while (!cfg_for(bq, d, &tmp)) bq >>= 1;
     }
     if (!cfg_for(bq, d, &P.cfg)) return fail(CVS_ERR_INVALID, "bq=%lld is not supported at width %lld", (long long)bq, (long long)d);
-    if (ScanCfg g; allow_gemm && !forced_bq && gemm_cfg(nq, n, d, k, cus, P.cfg, &g)) {
+    if (ScanCfg g; allow_lean && !forced_bq && gemm_cfg(nq, n, d, k, cus, P.cfg, &g)) {
       P.cfg = g;
       bq = g.bq();
     }
@@ -458,6 +483,14 @@ int make_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int64_t bq, int64_t c
     P.sin = false;
   }
   if (P.cap > kMaxCap) return fail(CVS_ERR_INVALID, "internal: list capacity %lld too large", (long long)P.cap);
+  if (allow_lean && !forced_bq && chunks == 0 && (flags & ~CVS_FLAG_IDS_INT64) == 0 &&
+      direct_search(nq, n, d, k, P.prepass)) {
+    P.direct = true;
+    P.sin = P.prepass = P.tau_in_scan = false;
+    P.ws_bytes = align_up(std::max<int64_t>(nq, 1) * n * 4, 256);
+    *p = P;
+    return CVS_OK;
+  }
   const int64_t lists = std::max<int64_t>(nq, 1) * P.nlists;
   int64_t off = 0;
   P.off_lv = off;
@@ -515,12 +548,56 @@ int cvs_fused_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int64_t bq, int6
 
 namespace {
 
+// The score matrix out [nq, n] (fp32 or fp16).  Query blocks and chunking as the
+// fused plan's query-stationary scan.
+hipError_t launch_scores(const _Float16* q, const _Float16* x, int64_t nq, int64_t n, int64_t d, void* out, bool fp32,
+                         int cus, hipStream_t s) {
+  if (nq == 1) {  // one query: the GEMV, 16 waves per CU of at least 16 rows
+    const int64_t waves = std::max<int64_t>(1, std::min<int64_t>((int64_t)cus * 16, ceil_div(n, 16)));
+    GemvArgs g{};
+    g.q = q;
+    g.x = x;
+    g.n = n;
+    g.d = (int)d;
+    g.rows_per_wave = align_up(ceil_div(n, waves), 16);
+    g.mode = fp32 ? kStoreF32 : kStoreF16;
+    g.out = out;
+    return launch_gemv(g, (int)ceil_div(ceil_div(n, g.rows_per_wave), 4), s);
+  }
+  ScanCfg cfg;
+  int64_t bq = nq <= 16 ? 16 : nq <= 32 ? 32 : nq <= 64 ? 64 : (nq <= 128 || d != 384) ? 128 : 256;
+  while (!cfg_for(bq, d, &cfg)) bq >>= 1;
+  const int64_t groups = ceil_div(nq, bq);
+  const int64_t ntiles = ceil_div(n, cfg.tile_rows());
+  const int64_t max_chunks = std::min<int64_t>(ntiles, 65535);
+  const int64_t most = std::min<int64_t>(max_chunks, std::max<int64_t>(1, groups > 1 ? align_up(ntiles / 2, 8) : ntiles / 2));
+  int64_t c = groups == 1 ? std::min<int64_t>(cus, most)
+                          : best_chunks(groups, ntiles, cus, most, qstat_tile_cost(cfg, d));
+  const int64_t tpc = ceil_div(ntiles, c);
+  const int xcd_pair = groups > 1 && c % 8 == 0 ? 1 : 0;
+  if (!xcd_pair) c = ceil_div(ntiles, tpc);
+  if (groups * c > INT_MAX) return hipErrorInvalidValue;
+  ScanArgs a{};
+  a.q = q;
+  a.x = x;
+  a.n = n;
+  a.nq = (int)nq;
+  a.d = (int)d;
+  a.groups = (int)groups;
+  a.nchunks = (int)c;
+  a.ntiles = ntiles;
+  a.tpc = tpc;
+  a.xcd_pair = xcd_pair;
+  a.out = out;
+  return launch_scan(cfg, fp32 ? kStoreF32 : kStoreF16, a, (int)(groups * c), s);
+}
+
 // Records marks[i] after pipeline stage i-1 when marks != nullptr (marks[0]
 // before the first launch).  Stages: 0 sample pass, 1 threshold select, 2 scan
 // or GEMV, 3 final select; skipped stages get back-to-back marks.
 int run_fused(const void* q, const void* x, int64_t nq, int64_t n, int64_t d, int64_t k, int64_t bq,
               int64_t chunks, int flags, void* workspace, int64_t workspace_bytes, float* out_v,
-              void* out_i, int64_t* plan_out, int device, void* stream, hipEvent_t* marks, bool allow_gemm = true) {
+              void* out_i, int64_t* plan_out, int device, void* stream, hipEvent_t* marks, bool allow_lean = true) {
   DevInfo di;
   int rc = dev_info(device, &di);
   if (rc != CVS_OK) return rc;
@@ -528,7 +605,7 @@ int run_fused(const void* q, const void* x, int64_t nq, int64_t n, int64_t d, in
   rc = check_inputs(q, x, nq, n, d);
   if (rc != CVS_OK) return rc;
   Plan P;
-  rc = make_plan(nq, n, d, k, bq, chunks, flags, di.cus, &P, 16, true, allow_gemm);
+  rc = make_plan(nq, n, d, k, bq, chunks, flags, di.cus, &P, 16, true, allow_lean);
   if (rc != CVS_OK) return rc;
   if (plan_out) {
     plan_out[0] = P.bq;
@@ -558,6 +635,25 @@ int run_fused(const void* q, const void* x, int64_t nq, int64_t n, int64_t d, in
   const _Float16* xh = static_cast<const _Float16*>(x);
   hipError_t e;
 
+  if (P.direct) {
+    mark(1);
+    mark(2);
+    e = launch_scores(qh, xh, nq, n, d, lv, true, di.cus, s);
+    if (e != hipSuccess) return hip_fail(e, "score kernel launch");
+    mark(3);
+    RowTopkArgs r{};
+    r.scores = lv;
+    r.n = n;
+    r.k = (int)k;
+    r.out_v = out_v;
+    r.out_i = out_i;
+    r.ids64 = (flags & CVS_FLAG_IDS_INT64) ? 1 : 0;
+    r.skip_nan = 1;
+    e = launch_row_topk(r, (int)nq, s);
+    if (e != hipSuccess) return hip_fail(e, "row top-k launch");
+    mark(4);
+    return CVS_OK;
+  }
   if (P.gemv) {
     GemvArgs g{};
     g.q = qh;
@@ -768,10 +864,10 @@ int cvs_fused_topk_noalloc(const void* q, const void* x, int64_t nq, int64_t n, 
   Plan P;
   rc = make_plan(nq, n, d, k, 0, 0, flags, di.cus, &P);
   if (rc != CVS_OK) return rc;
-  // the tiled-GEMM scan keeps more lists per query: where they do not fit, the
-  // query-stationary one
-  const bool allow_gemm = P.ws_bytes <= kScratchBytes;
-  if (!allow_gemm) {
+  // the tiled-GEMM scan keeps more lists per query, the score-matrix search all
+  // scores: where they do not fit, the query-stationary scan
+  const bool allow_lean = P.ws_bytes <= kScratchBytes;
+  if (!allow_lean) {
     rc = make_plan(nq, n, d, k, 0, 0, flags, di.cus, &P, 16, true, false);
     if (rc != CVS_OK) return rc;
   }
@@ -790,7 +886,7 @@ int cvs_fused_topk_noalloc(const void* q, const void* x, int64_t nq, int64_t n, 
   // The fused path needs no zeroed workspace (every list count and threshold is
   // written before it is read), so nothing is cleared here.
   return run_fused(q, x, nq, n, d, k, 0, 0, flags, ws, kScratchBytes, out_v, out_i, plan_out, device, stream,
-                   nullptr, allow_gemm);
+                   nullptr, allow_lean);
 }
 
 int cvs_fused_topk_marked(const void* q, const void* x, int64_t nq, int64_t n, int64_t d, int64_t k,
@@ -817,45 +913,17 @@ int cvs_scores(const void* q, const void* x, int64_t nq, int64_t n, int64_t d, v
   if (rc != CVS_OK) return rc;
   if (nq == 0 || n == 0) return CVS_OK;
   if (out == nullptr) return fail(CVS_ERR_INVALID, "output pointer must not be null");
-  // Same query blocks and chunking as the fused plan: one workgroup per CU,
-  // chunks a multiple of the 8 XCDs when several query groups share them.
-  ScanCfg cfg;
-  int64_t bq = nq <= 16 ? 16 : nq <= 32 ? 32 : nq <= 64 ? 64 : (nq <= 128 || d != 384) ? 128 : 256;
-  while (!cfg_for(bq, d, &cfg)) bq >>= 1;
-  const int64_t groups = ceil_div(nq, bq);
-  const int64_t ntiles = ceil_div(n, cfg.tile_rows());
-  const int64_t max_chunks = std::min<int64_t>(ntiles, 65535);
-  const int64_t most = std::min<int64_t>(max_chunks, std::max<int64_t>(1, groups > 1 ? align_up(ntiles / 2, 8) : ntiles / 2));
-  int64_t c = groups == 1 ? std::min<int64_t>(di.cus, most)
-                          : best_chunks(groups, ntiles, di.cus, most, qstat_tile_cost(cfg, d));
-  const int64_t tpc = ceil_div(ntiles, c);
-  const int xcd_pair = groups > 1 && c % 8 == 0 ? 1 : 0;
-  if (!xcd_pair) c = ceil_div(ntiles, tpc);
-  if (groups * c > INT_MAX) return fail(CVS_ERR_INVALID, "too many queries");
-
   DeviceGuard guard(device);
   if (guard.err != hipSuccess) return hip_fail(guard.err, "hipSetDevice");
-  ScanArgs a{};
-  a.q = static_cast<const _Float16*>(q);
-  a.x = static_cast<const _Float16*>(x);
-  a.n = n;
-  a.nq = (int)nq;
-  a.d = (int)d;
-  a.groups = (int)groups;
-  a.nchunks = (int)c;
-  a.ntiles = ntiles;
-  a.tpc = tpc;
-  a.xcd_pair = xcd_pair;
-  a.out = out;
-  hipError_t e = launch_scan(cfg, out_fp32 ? kStoreF32 : kStoreF16, a, (int)(groups * c),
-                             reinterpret_cast<hipStream_t>(stream));
+  hipError_t e = launch_scores(static_cast<const _Float16*>(q), static_cast<const _Float16*>(x), nq, n, d, out,
+                               out_fp32 != 0, di.cus, reinterpret_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "score kernel launch");
   return CVS_OK;
 }
 
 namespace {
 
-// Plan of cvs_topk_rows (see cvs_rowtopk.hip); rows of at most kRowCap columns
+// Plan of cvs_topk_rows (see cvs_rowtopk.hip); rows of at most kRowDirect columns
 // need no workspace.  At most kRowBatch rows run in one set of launches, so
 // the candidate arrays stay within 64 MB whatever the batch.
 constexpr int64_t kRowBatch = 1024;
@@ -869,7 +937,7 @@ struct RowPlan {
 RowPlan row_plan(int64_t nq, int64_t n, int64_t k, int cus) {
   RowPlan P;
   P.rows = std::max<int64_t>(1, std::min<int64_t>(nq, kRowBatch));
-  if (n <= kRowCap) return P;
+  if (n <= kRowDirect) return P;
   // The sample: a 32nd of the row, at least 16384 scores (a quarter of a short
   // row), so that about 8 or more of the row's k best are in it for k = 256
   // (30 at k = 1000 over 1M columns); the threshold is the score `rank` from

@@ -14,6 +14,7 @@
 // (v_dot4_i32_i8, exact int32 sums, 128-byte pieces of 128 int8): rows whose
 // score upper bound reaches the threshold are appended, a full list is marked
 // overflowed instead of compacted, and the select recomputes exact scores.
+// kStoreF32 / kStoreF16 write every score (one query's row of the score matrix).
 // kMaxQ8 samples that way: per unit the largest approximate score
 // A = s_q s_b sum(q~ x~) and its row, for the threshold kernel to rescore.
 #include "cvs_common.h"
@@ -54,6 +55,7 @@ __global__ __launch_bounds__(kBlock) void gemv_kernel(GemvArgs a) {
   constexpr bool Q8 = (MODE == kAppendQ8 || MODE == kMaxQ8);
   constexpr bool APP = (MODE == kAppend || MODE == kAppendQ8);
   constexpr bool SMAX = (MODE == kMax || MODE == kMaxQ8);
+  constexpr bool STORE = (MODE == kStoreF32 || MODE == kStoreF16);
   __shared__ uint64_t sortbuf[MODE == kAppend ? 4 * kMaxCap : 1];
   const int lane = lane_id();
   const int w = threadIdx.x >> 6;
@@ -170,7 +172,12 @@ __global__ __launch_bounds__(kBlock) void gemv_kernel(GemvArgs a) {
       }
       const int64_t row = r0 + u * 8 + rg;
       const bool valid = row < r_end;
-      if (MODE == kMax) {
+      if (STORE) {
+        if (valid && sub == 0) {
+          if (MODE == kStoreF32) static_cast<float*>(a.out)[row] = acc;
+          else static_cast<_Float16*>(a.out)[row] = (_Float16)acc;
+        }
+      } else if (MODE == kMax) {
         if (valid) umax = fmaxf(umax, acc);
       } else if (MODE == kMaxQ8) {
         if (valid && acc > umax) {
@@ -249,6 +256,10 @@ hipError_t launch_p(const GemvArgs& a, int grid, hipStream_t s) {
     hipLaunchKernelGGL((gemv_kernel<PMAX, kAppend>), dim3(grid), dim3(kBlock), 0, s, a);
   else if (a.mode == kMax)
     hipLaunchKernelGGL((gemv_kernel<PMAX, kMax>), dim3(grid), dim3(kBlock), 0, s, a);
+  else if (a.mode == kStoreF32)
+    hipLaunchKernelGGL((gemv_kernel<PMAX, kStoreF32>), dim3(grid), dim3(kBlock), 0, s, a);
+  else if (a.mode == kStoreF16)
+    hipLaunchKernelGGL((gemv_kernel<PMAX, kStoreF16>), dim3(grid), dim3(kBlock), 0, s, a);
   else
     return hipErrorInvalidValue;
   return hipGetLastError();

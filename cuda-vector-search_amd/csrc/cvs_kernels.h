@@ -118,7 +118,8 @@ struct GemvArgs {
   int nsample;        // kMax: sampled 64-row blocks (one per wave)
   int upb;            // kMax: units per block, 8 (rows mod 8) or 1 (the block)
   int units;
-  int mode;           // kAppend, kMax, kAppendQ8 or kMaxQ8 (the largest approximate score, int8)
+  int mode;           // kAppend, kMax, kStoreF32, kStoreF16, kAppendQ8 or kMaxQ8 (the largest approximate score, int8)
+  void* out;          // kStore*: [n]
   // kAppendQ8: q and x are int8 rows of d bytes (d = 384, 768 or 1536); the
   // filter uses the score upper bound as the scan's kAppendQ8 does
   const float4* qmeta;  // [1]
@@ -129,7 +130,8 @@ struct GemvArgs {
 // Exact top-k of fp32 score rows (cvs_rowtopk.hip): row r of a launch is row
 // row0 + r of the matrix and of the outputs.
 constexpr int kRowTopkMaxK = 1024;
-constexpr int kRowCap = 8192;  // candidates per row; shorter rows are sorted whole
+constexpr int kRowCap = 8192;      // candidates per row
+constexpr int kRowDirect = 32768;  // rows up to this are cut by one workgroup, without a sampled threshold
 struct RowTopkArgs {
   const float* scores;  // [rows, n] fp32
   int64_t n;
@@ -138,7 +140,8 @@ struct RowTopkArgs {
   float* out_v;         // [rows, k]
   void* out_i;          // [rows, k] int32 column ids (int64 when ids64)
   int ids64;
-  // rows longer than kRowCap
+  int skip_nan;         // 1: NaN scores are no candidates; places left over get (-inf, -1) (n <= kRowDirect only)
+  // rows longer than kRowDirect
   int groups;           // sampled groups of 32 scores per row
   int rank;             // the sample's rank taken as threshold
   int64_t len;          // columns per filter workgroup (a multiple of 4)

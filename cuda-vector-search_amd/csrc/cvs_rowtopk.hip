@@ -16,11 +16,11 @@
 //     fewer than k or more than kRowCap scores reach it, the row is streamed
 //     again here and its top k taken exactly.
 //
-// Rows of at most kRowCap scores need no threshold: step 3 takes the whole row.
+// Rows of at most kRowDirect scores need no threshold: step 3 takes the whole row.
 //
 // Measured against chunk-wise radix selects and a merge of the chunks' top k:
-// 64 rows x 300k, k = 1000: 192 -> 54 us; 1 x 4M, k = 1000: 3378 -> 58 us;
-// 1000 x 8200, k = 300: 132 -> 62 us; whole rows, 1000 x 8000, k = 1000: 78 -> 41 us.
+// 64 rows x 300k, k = 1000: 192 -> 54 us; 1 x 4M, k = 1000: 3378 -> 58 us; whole
+// rows, 1000 x 8000, k = 1000: 78 -> 41 us.
 #include "cvs_common.h"
 #include "cvs_kernels.h"
 
@@ -88,7 +88,8 @@ __device__ __forceinline__ int cut_bin(BinScratch& B, int want, int* above) {
   if (tid % kWave == kWave - 1) B.wsum[tid / kWave] = incl;
   if (tid == 0) B.bin = -1;
   __syncthreads();
-  for (int w = 0; w < tid / kWave; ++w) incl += B.wsum[w];
+#pragma unroll
+  for (int w = 0; w < kFinalWaves; ++w) incl += w < tid / kWave ? B.wsum[w] : 0;
   if (incl - c < want && want <= incl) {
     B.bin = b;
     B.above = incl;
@@ -169,9 +170,38 @@ __device__ __forceinline__ void sort_and_put(int m, int k, uint64_t* lds, Get ge
     if (tid * E + e < top) put(tid * E + e, v[e]);
 }
 
+// The same for m <= 256 keys by rank: G threads count the keys above each (over
+// slices), two barriers where the network takes 55 stages (rows of 3000 scores,
+// k = 10, with their GEMV: 16 -> 8 us).  Equal keys (0: none) rank by position.
+template <class Get, class Put>
+__device__ __forceinline__ void rank_and_put(int m, int k, uint64_t* lds, Get get, Put put) {
+  __shared__ int rank[256];
+  const int tid = threadIdx.x;
+  const int P = m <= 64 ? 64 : 256, G = kFinal / P;
+  const int i = tid & (P - 1), g = tid / P;
+  const uint64_t mine = i < m ? get(i) : 0ull;
+  if (tid < P) rank[tid] = 0;
+  __syncthreads();  // (get() may read from lds)
+  if (g == 0 && i < m) lds[i] = mine;
+  __syncthreads();
+  const int per = (m + G - 1) / G, j1 = min(m, (g + 1) * per);
+  int r = 0;
+  if (i < m)
+#pragma unroll 4
+    for (int j = g * per; j < j1; ++j) {
+      const uint64_t o = lds[j];
+      r += o > mine || (o == mine && j < i) ? 1 : 0;
+    }
+  if (r > 0) atomicAdd(&rank[i], r);
+  __syncthreads();
+  if (g == 0 && i < m && rank[i] < k) put(rank[i], mine);
+}
+
 template <class Get, class Put>
 __device__ __forceinline__ void sort_any(int m, int k, uint64_t* lds, Get get, Put put) {
-  if (m <= kFinal)
+  if (m <= 256)
+    rank_and_put(m, k, lds, get, put);
+  else if (m <= kFinal)
     sort_and_put<1>(m, k, lds, get, put);
   else if (m <= 2 * kFinal)
     sort_and_put<2>(m, k, lds, get, put);
@@ -276,7 +306,7 @@ __global__ __launch_bounds__(kBlock) void row_filter_kernel(RowTopkArgs a) {
   if (nbuf > 0) flush();
 }
 
-// DIRECT: the row's n <= kRowCap scores are the candidates.
+// DIRECT: the row's n <= kRowDirect scores are the candidates.
 template <bool DIRECT>
 __global__ __launch_bounds__(kFinal) void row_final_kernel(RowTopkArgs a) {
   constexpr int E = kRowCap / kFinal;
@@ -290,23 +320,61 @@ __global__ __launch_bounds__(kFinal) void row_final_kernel(RowTopkArgs a) {
   const float* row = a.scores + (a.row0 + r) * a.n;
   const int64_t obase = (a.row0 + r) * (int64_t)k;
   auto put = [&](int i, uint64_t key) {
-    a.out_v[obase + i] = key_score(key);
+    const bool none = key == 0ull;  // (a skipped NaN)
+    a.out_v[obase + i] = none ? -__builtin_inff() : key_score(key);
+    const int id = none ? -1 : key_id(key);
     if (a.ids64)
-      ((int64_t*)a.out_i)[obase + i] = key_id(key);
+      ((int64_t*)a.out_i)[obase + i] = id;
     else
-      ((int*)a.out_i)[obase + i] = key_id(key);
+      ((int*)a.out_i)[obase + i] = id;
   };
   int m = DIRECT ? (int)a.n : a.count[r];
   if (tid == 0) nbuf = 0;
-  if (DIRECT || (m >= k && m <= kRowCap)) {
+  if (DIRECT && m > kRowCap) {
+    // The same cut with the row re-read (from cache) for the range, the
+    // histogram and the keys of its top bins.
+    float lo = __builtin_inff(), hi = -__builtin_inff();
+#pragma unroll 16
+    for (int i = tid; i < m; i += kFinal) {
+      const float v = row[i];
+      lo = fminf(lo, v);
+      hi = fmaxf(hi, v == v || a.skip_nan ? v : __builtin_inff());
+    }
+    Bins bins;
+    if (make_bins(B, lo, hi, &bins)) {  // (uniform)
+#pragma unroll 16
+      for (int i = tid; i < m; i += kFinal) {
+        const float v = row[i];
+        if (v == v) atomicAdd(&B.hist[bins.of(v)], 1);
+      }
+      __syncthreads();
+      int above = 0;
+      const int bstar = cut_bin(B, k, &above);
+      if (bstar >= 0 && above <= kRowCap) {
+#pragma unroll 16
+        for (int i = tid; i < m; i += kFinal) {
+          const float v = row[i];
+          if (v == v && bins.of(v) >= bstar) keys[atomicAdd(&nbuf, 1)] = make_key(v, i);
+        }
+        __syncthreads();
+        sort_any(nbuf, k, keys, [&](int i) { return keys[i]; }, put);
+        return;
+      }
+    }
+    __syncthreads();
+  } else if (DIRECT || (m >= k && m <= kRowCap)) {
     const uint64_t* cand = DIRECT ? nullptr : a.cand + (int64_t)r * kRowCap;
-    auto get = [&](int i) { return DIRECT ? make_key(row[i], i) : cand[i]; };
-    if (m <= 2 * kFinal) {
+    auto get = [&](int i) -> uint64_t {
+      if constexpr (!DIRECT) return cand[i];
+      const float v = row[i];
+      return a.skip_nan && v != v ? 0ull : make_key(v, i);
+    };
+    if (m <= 256 || (m <= 2 * kFinal && 4 * k > m)) {
       sort_any(m, k, keys, get, put);
       return;
     }
-    // cut to the top histogram bins that hold k: a sort of 8192 keys costs
-    // several times one of the ~k that matter
+    // cut to the top histogram bins that hold k: a sort of thousands of keys
+    // costs several times one of the ~k that matter
     uint64_t v[E];
     float lo = __builtin_inff(), hi = -__builtin_inff();
 #pragma unroll
@@ -338,7 +406,7 @@ __global__ __launch_bounds__(kFinal) void row_final_kernel(RowTopkArgs a) {
     sort_any(m, k, keys, [&](int i) { return keys[i]; }, put);
     return;
   }
-  // The threshold missed: the row streamed again, its running k best in LDS.
+  // The threshold missed, or the cut (equal scores, infinities): the row streamed, its running k best in LDS.
   if (tid == 0) kth = 0ull;
   __syncthreads();
   for (int64_t base = 0; base < a.n; base += 4 * kFinal) {
@@ -346,7 +414,8 @@ __global__ __launch_bounds__(kFinal) void row_final_kernel(RowTopkArgs a) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int64_t col = base + u * kFinal + tid;
-      const uint64_t key = col < a.n ? make_key(row[col], (int)col) : 0ull;
+      const float v = col < a.n ? row[col] : 0.f;
+      const uint64_t key = col < a.n && !(a.skip_nan && v != v) ? make_key(v, (int)col) : 0ull;
       if (key > t) keys[atomicAdd(&nbuf, 1)] = key;
     }
     __syncthreads();
@@ -354,6 +423,7 @@ __global__ __launch_bounds__(kFinal) void row_final_kernel(RowTopkArgs a) {
     const bool last = base + 4 * kFinal >= a.n;
     if (last) {
       sort_and_put<E>(nb, k, keys, [&](int i) { return keys[i]; }, put);
+      for (int i = nb + tid; i < k; i += kFinal) put(i, 0ull);  // (NaNs left out)
     } else if (nb > 4 * kFinal) {
       sort_and_put<E>(nb, k, keys, [&](int i) { return keys[i]; }, [&](int i, uint64_t key) {
         keys[i] = key;
@@ -369,7 +439,7 @@ __global__ __launch_bounds__(kFinal) void row_final_kernel(RowTopkArgs a) {
 
 hipError_t launch_row_topk(const RowTopkArgs& a, int rows, hipStream_t s) {
   if (a.k < 1 || a.k > kRowTopkMaxK || a.n < a.k || rows < 1 || a.scores == nullptr) return hipErrorInvalidValue;
-  if (a.n <= kRowCap) {
+  if (a.n <= kRowDirect) {
     hipLaunchKernelGGL(row_final_kernel<true>, dim3(rows), dim3(kFinal), 0, s, a);
     return hipGetLastError();
   }

@@ -642,8 +642,11 @@ def test_topk_rows_with_infinite_scores(eng, nq, n, k):
 
 
 @pytest.mark.parametrize("nq,n,k,data", [
-    (3, 8192, 1024, "normal"), (3, 8193, 1, "normal"), (2, 12289, 1024, "normal"),  # whole rows / filtered, odd strides
-    (1030, 9001, 257, "normal"),           # more rows than one set of launches takes
+    (3, 255, 200, "normal"), (3, 2048, 600, "normal"), (3, 2049, 10, "normal"),  # rank, network, cut
+    (3, 8192, 1024, "normal"), (3, 8193, 1, "normal"), (2, 32768, 1024, "normal"),  # whole rows, re-read past 8192
+    (2, 32768, 100, "nan"), (2, 20000, 1000, "equal"),
+    (2, 32769, 1024, "normal"),            # filtered, odd strides
+    (1030, 33001, 257, "normal"),          # more rows than one set of launches takes
     (2, 70001, 1000, "equal"),             # every score reaches the threshold: streamed again
     (2, 70001, 1000, "burst"),             # the sample sees every high score, too few reach it: streamed again
     (2, 300000, 1000, "block"),            # the best scores side by side in one filter workgroup
@@ -670,6 +673,35 @@ def test_topk_rows_threshold_edges(eng, nq, n, k, data):
     order = np.lexsort((np.broadcast_to(np.arange(n), key.shape), -key), axis=1)[:, :k]
     np.testing.assert_array_equal(i.cpu().numpy(), order)
     np.testing.assert_array_equal(v.cpu().numpy(), np.take_along_axis(s.numpy(), order, axis=1))
+
+
+@pytest.mark.parametrize("nq,n,d,k", [(1, 1, 64, 1), (1, 5003, 384, 5), (16, 8192, 768, 10), (17, 700, 384, 256),
+                                      (300, 8191, 128, 100), (5, 8193, 320, 3), (1, 8192, 1600, 256),
+                                      (9, 32768, 256, 40), (1, 16385, 768, 10), (100, 16000, 768, 200)])
+def test_small_corpus_search_is_exact(eng, nq, n, d, k):
+    """Corpora of few rows searched through a score matrix (and one that is
+    not), against the lists (forced by a flag) and the oracle; exact
+    ties; NaN scores are left out as the lists leave them out."""
+    say(f"small corpus nq={nq} n={n} d={d} k={k}")
+    x, q = make(n, d, nq, seed=n + k)
+    if n > 10:
+        x[n // 2:n // 2 + 5] = x[1]
+        q[0] = x[1]
+    xd, qd = x.cuda(), q.cuda()
+    v, i, _ = eng.fused_topk(qd, xd, k)
+    v2, i2, _ = eng.fused_topk(qd, xd, k, flags=_ext.FLAG_NO_PREPASS)
+    torch.cuda.synchronize()
+    oracle.check_exact(q, x, k, v.cpu().numpy(), i.cpu().numpy())
+    torch.testing.assert_close(v, v2, rtol=0, atol=2 * d * 2.0**-24)  # fp32 sums in two orders
+    assert (i != i2).float().mean().item() < 0.02
+    if n > 10:
+        xd[3::4] = float("nan")
+        v, i, _ = eng.fused_topk(qd, xd, min(k, n))
+        v2, i2, _ = eng.fused_topk(qd, xd, min(k, n), flags=_ext.FLAG_NO_PREPASS | _ext.FLAG_NO_GEMV)
+        torch.cuda.synchronize()
+        assert not torch.isnan(v).any() and torch.equal((i % 4 == 3) & (i >= 0), torch.zeros_like(i, dtype=torch.bool))
+        assert torch.equal(i < 0, i2 < 0)
+        torch.testing.assert_close(v, v2, rtol=0, atol=2 * d * 2.0**-24)
 
 
 def test_topk_rows_errors(eng):
