@@ -1696,3 +1696,50 @@ int cvs_q8_topk_marked(const void* q, const void* x, const void* xq, int64_t xq_
 }
 
 }  // extern "C"
+
+namespace {
+
+// Bytes at the head of cvs_search's workspace for the prepared queries (0: the
+// caller's rows serve as they are).
+int64_t search_query_bytes(int64_t nq, int64_t d, int64_t dim, int normalize) {
+  return normalize || dim != d ? align_up(nq * d * 2, 256) : 0;
+}
+
+}  // namespace
+
+extern "C" {
+
+int cvs_search_plan(int64_t nq, int64_t n, int64_t d, int64_t dim, int64_t k, int normalize, int int8, int flags,
+                    int device, int64_t* workspace_bytes) {
+  int64_t bytes = 0;
+  const int rc = int8 ? cvs_q8_plan(nq, n, d, k, flags, device, nullptr, &bytes)
+                      : cvs_fused_plan(nq, n, d, k, 0, 0, flags, device, nullptr, &bytes);
+  if (rc != CVS_OK) return rc;
+  if (nq < 0 || nq >= INT_MAX) return fail(CVS_ERR_INVALID, "too many queries");
+  if (workspace_bytes) *workspace_bytes = search_query_bytes(nq, d, dim, normalize) + bytes;
+  return CVS_OK;
+}
+
+int cvs_search(const void* q, int64_t dim, int normalize, const void* x, const void* xq, int64_t xq_bytes, int64_t nq,
+               int64_t n, int64_t d, int64_t k, int flags, void* workspace, int64_t workspace_bytes, float* out_v,
+               void* out_i, int device, void* stream) {
+  if (nq < 1 || nq >= INT_MAX) return fail(CVS_ERR_INVALID, "the number of queries must be in [1, 2^31)");
+  if (d <= 0 || d % 64 != 0) return fail(CVS_ERR_INVALID, "width must be a multiple of 64 (zero-pad it)");
+  const int64_t qbytes = search_query_bytes(nq, d, dim, normalize);
+  char* ws = static_cast<char*>(workspace);
+  if (qbytes > 0) {
+    if (ws == nullptr || workspace_bytes < qbytes || reinterpret_cast<uintptr_t>(ws) % 256 != 0)
+      return fail(CVS_ERR_INVALID, "workspace must be 256-byte aligned and hold what cvs_search_plan says");
+    const int rc = cvs_prep_rows(q, ws, nq, dim, dim, d, normalize, device, stream);
+    if (rc != CVS_OK) return rc;
+    q = ws;
+    ws += qbytes;
+    workspace_bytes -= qbytes;
+  }
+  if (xq != nullptr)
+    return run_q8(q, x, xq, xq_bytes, nq, n, d, k, flags, ws, workspace_bytes, out_v, out_i, nullptr, device, stream,
+                  nullptr);
+  return run_fused(q, x, nq, n, d, k, 0, 0, flags, ws, workspace_bytes, out_v, out_i, nullptr, device, stream, nullptr);
+}
+
+}  // extern "C"

@@ -135,6 +135,7 @@ class Index:
         self._xq = None
         self._xq_stamp = None  # (version, data_ptr, shape) of _x when _xq was built
         self._xq_ready = None  # event recorded after the build of _xq
+        self._xq_stream = None  # raw handle of the stream _xq was allocated and built on
         self._xq_lock = threading.Lock()
         if self._use_kernels:
             if not x.is_contiguous():
@@ -189,6 +190,7 @@ class Index:
     def _set_int8(self, xq: torch.Tensor, stamp) -> None:
         ready = torch.cuda.Event()
         ready.record()
+        self._xq_stream = _ext.raw_stream(xq.device.index)
         self._xq, self._xq_stamp, self._xq_ready = xq, stamp, ready
 
     def _int8_companion(self, build: bool):
@@ -204,6 +206,9 @@ class Index:
             if self._xq is None or self._xq_stamp != self._corpus_stamp():
                 self._build_int8()
             xq, ready = self._xq, self._xq_ready
+            same = self._xq_stream == _ext.raw_stream(xq.device.index)
+        if same and ready.query():  # built, and its memory is reused in this stream's order only
+            return xq
         stream = torch.cuda.current_stream(self.device)
         if not ready.query():  # still being built: order this stream after the build
             stream.wait_event(ready)
@@ -231,13 +236,19 @@ class Index:
         """The stored matrix (normalised for cosine), without the padding columns."""
         return self._x[:, :self.dim]
 
-    def _prep_queries(self, queries) -> torch.Tensor:
+    def _query_rows(self, queries) -> torch.Tensor:
+        """The queries as contiguous [b, dim] rows of the stored type on the index's device."""
         q = _as_tensor(queries)
         if q.dim() == 1:
             q = q.unsqueeze(0)
         if q.dim() != 2 or q.shape[1] != self.dim:
             raise ValueError(f"queries must be [b, {self.dim}]")
-        q = q.to(self.device, self._x.dtype).contiguous()
+        if q.dtype != self._x.dtype or q.device != self._x.device:
+            q = q.to(self.device, self._x.dtype)
+        return q if q.is_contiguous() else q.contiguous()
+
+    def _prep_queries(self, queries) -> torch.Tensor:
+        q = self._query_rows(queries)
         width = self._x.shape[1]
         if (self._use_kernels and q.shape[0] > 0
                 and (self.metric == "cosine" or width != q.shape[1])):
@@ -272,30 +283,30 @@ class Index:
         if k < 1:
             raise ValueError("k must be >= 1")
         k = min(k, len(self))
-        q = self._prep_queries(queries)
+        rows = self._query_rows(queries)
         if method == "auto":
             if self._use_kernels and k <= MAX_FUSED_K:
-                method = "int8" if self._int8_wins(q.shape[0], k) else "fused"
+                method = "int8" if self._int8_wins(rows.shape[0], k) else "fused"
             elif self._use_kernels and k <= MAX_EXACT_K:
-                return self._search_large_k(q, k)
+                return self._search_large_k(self._prep_queries(rows), k)
             else:
                 method = "torch"
         if method in ("fused", "twopass", "int8") and not self._use_kernels:
             raise RuntimeError(f"method={method!r} needs an AMD Instinct MI355X (gfx950) GPU")
-        if method == "int8":
+        if method in ("fused", "int8"):
+            xq = None
             if k > MAX_FUSED_K:
-                raise ValueError(f"int8 search supports k <= {MAX_FUSED_K}")
-            if self._x.shape[1] > Q8_MAX_WIDTH:
-                raise ValueError(f"int8 search supports widths up to {Q8_MAX_WIDTH}")
-            xq = self._int8_companion(build=True)
-            v, i, _ = _ext.load().q8_topk(q, self._x, xq, k, flags=_ext.FLAG_IDS_INT64)
-            return v, i
-        if method == "fused":
-            if k > MAX_FUSED_K:
-                raise ValueError(f"fused search supports k <= {MAX_FUSED_K}")
+                raise ValueError(f"{method} search supports k <= {MAX_FUSED_K}")
+            if method == "int8":
+                if self._x.shape[1] > Q8_MAX_WIDTH:
+                    raise ValueError(f"int8 search supports widths up to {Q8_MAX_WIDTH}")
+                xq = self._int8_companion(build=True)
+            if rows.shape[0] == 0:
+                return (torch.empty((0, k), dtype=torch.float32, device=rows.device),
+                        torch.empty((0, k), dtype=torch.int64, device=rows.device))
             # ids come out as int64 directly (index.py:126 widens int32 with .long())
-            v, i, _ = _ext.load().fused_topk(q, self._x, k, flags=_ext.FLAG_IDS_INT64)
-            return v, i
+            return _ext.load().search(rows, self._x, k, self.metric == "cosine", xq)
+        q = self._prep_queries(rows)
         if method == "twopass":
             s = _ext.load().scores(q, self._x, False)
             v, i = torch.topk(s, k, dim=1)

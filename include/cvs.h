@@ -230,6 +230,21 @@ int cvs_q8_topk_marked(const void* q, const void* x, const void* xq, int64_t xq_
                        int64_t d, int64_t k, int flags, void* workspace, int64_t workspace_bytes, float* out_v,
                        void* out_i, int64_t* plan_out, int device, void* stream, void* const* marks);
 
+/*
+ * A whole search in one call (no counterpart in the reference, which chains
+ * index.py:89-131 in Python): the queries q [nq, dim] (fp16, contiguous) as
+ * cvs_prep_rows prepares them for rows of width d (L2-normalised when normalize
+ * != 0, zero-padded when dim < d; used as they are when neither), then
+ * cvs_fused_topk (xq null, auto plan) or cvs_q8_topk with the companion xq.
+ * nq >= 1.  `workspace` (256-byte aligned) holds at least what cvs_search_plan
+ * reports for the same arguments (int8 != 0: with a companion).
+ */
+int cvs_search_plan(int64_t nq, int64_t n, int64_t d, int64_t dim, int64_t k, int normalize, int int8, int flags,
+                    int device, int64_t* workspace_bytes);
+int cvs_search(const void* q, int64_t dim, int normalize, const void* x, const void* xq, int64_t xq_bytes, int64_t nq,
+               int64_t n, int64_t d, int64_t k, int flags, void* workspace, int64_t workspace_bytes, float* out_v,
+               void* out_i, int device, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

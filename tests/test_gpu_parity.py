@@ -704,6 +704,32 @@ def test_small_corpus_search_is_exact(eng, nq, n, d, k):
         torch.testing.assert_close(v, v2, rtol=0, atol=2 * d * 2.0**-24)
 
 
+@pytest.mark.parametrize("metric,d", [("ip", 128), ("ip", 100), ("cosine", 128), ("cosine", 100)])
+def test_search_in_one_call_equals_its_parts(eng, metric, d):
+    """Index.search against prepared queries and the engine's own entry points."""
+    say(f"one-call search {metric} d={d}")
+    x, q = make(3000, d, 7, seed=d)
+    index = Index(x.cuda(), metric=metric, int8_prefilter=True)
+    qp = index._prep_queries(q.cuda())
+    for method, run in (("fused", lambda: eng.fused_topk(qp, index._x, 5, flags=_ext.FLAG_IDS_INT64)),
+                        ("int8", lambda: eng.q8_topk(qp, index._x, index._xq, 5, flags=_ext.FLAG_IDS_INT64))):
+        v, i = index.search(q.cuda(), 5, method=method)
+        v2, i2, _ = run()
+        torch.cuda.synchronize()
+        assert torch.equal(v, v2) and torch.equal(i, i2)
+        side = torch.cuda.Stream()
+        with torch.cuda.stream(side):  # another stream than the companion's
+            v3, i3 = index.search(q.cuda(), 5, method=method)
+        side.synchronize()
+        assert torch.equal(v, v3) and torch.equal(i, i3)
+        assert index.search(q[:0].cuda(), 5, method=method)[1].shape == (0, 5)
+    ws = torch.empty(256, dtype=torch.uint8, device="cuda")
+    args = (qp.data_ptr(), d, 1, index._x.data_ptr(), None, 0, 7, 3000, 128, 5, 0, ws.data_ptr(), 256, v.data_ptr(),
+            i.data_ptr(), 0, None)
+    assert eng.lib.cvs_search(*args) != 0 and b"workspace" in eng.lib.cvs_last_error()
+    assert eng.lib.cvs_search(*args[:6], 0, *args[7:]) != 0
+
+
 def test_topk_rows_errors(eng):
     s = torch.zeros(2, 100, device="cuda")
     with pytest.raises(RuntimeError, match="1 <= k <= 1024"):
