@@ -80,7 +80,7 @@ def build(jobs: int | None = None, verbose: bool = False) -> Path:
         obj = BUILD / (Path(src).stem + ".o")
         objs.append(obj)
         cmds.append([HIPCC, *FLAGS, *EXTRA.get(src, []), "-c", CSRC / src, "-o", obj])
-    # device assembly of the MFMA kernels, for the result-hazard check below
+    # device assembly of the MFMA kernels, for the hazard check below
     asms = []
     for src in MFMA_SOURCES:
         asm = BUILD / (Path(src).stem + ".s")
@@ -90,7 +90,7 @@ def build(jobs: int | None = None, verbose: bool = False) -> Path:
         list(ex.map(lambda c: _run(c, verbose), cmds))
     early = [p for asm in asms for p in hazard_check.check(asm)]
     if early:
-        raise RuntimeError(f"{len(early)} MFMA results read too early in the scan kernels, e.g. " + early[0])
+        raise RuntimeError(f"{len(early)} hazards in the scan kernels, e.g. " + early[0])
     tmp = LIB.with_suffix(".so.tmp")
     _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp], verbose)
     os.replace(tmp, LIB)

@@ -146,12 +146,14 @@ template <bool NT>
 __device__ __forceinline__ void dma_to_lds_16(const void* src, const void* lds_block) {
   const uint32_t base = __builtin_amdgcn_readfirstlane(
       (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)lds_block);
-  // m0 is restored afterwards: the compiler treats it as reserved.
+  // m0 is restored afterwards: the compiler treats it as reserved.  A load into
+  // LDS needs one wait state after the write of m0 (hazard_check.py).
   uint32_t saved;
   if (NT)
     asm volatile(
         "s_mov_b32 %0, m0\n\t"
         "s_mov_b32 m0, %1\n\t"
+        "s_nop 0\n\t"
         "global_load_lds_dwordx4 %2, off nt\n\t"
         "s_mov_b32 m0, %0"
         : "=&s"(saved)
@@ -161,6 +163,7 @@ __device__ __forceinline__ void dma_to_lds_16(const void* src, const void* lds_b
     asm volatile(
         "s_mov_b32 %0, m0\n\t"
         "s_mov_b32 m0, %1\n\t"
+        "s_nop 0\n\t"
         "global_load_lds_dwordx4 %2, off\n\t"
         "s_mov_b32 m0, %0"
         : "=&s"(saved)
@@ -183,6 +186,7 @@ __device__ __forceinline__ void dma16_saddr(uint32_t voff, const void* sbase, ui
   asm volatile(
       "s_mov_b32 %0, m0\n\t"
       "s_mov_b32 m0, %1\n\t"
+      "s_nop 0\n\t"
       "global_load_lds_dwordx4 %2, %3 nt\n\t"
       "s_mov_b32 m0, %0"
       : "=&s"(saved)

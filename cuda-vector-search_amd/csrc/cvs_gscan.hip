@@ -66,6 +66,7 @@ __device__ __forceinline__ void dma16(uint32_t voff, const void* sbase, uint32_t
   asm volatile(
       "s_mov_b32 %0, m0\n\t"
       "s_mov_b32 m0, %1\n\t"
+      "s_nop 0\n\t"
       "global_load_lds_dwordx4 %2, %3\n\t"
       "s_mov_b32 m0, %0"
       : "=&s"(saved)

@@ -1,4 +1,4 @@
-"""Build-time check of MFMA result hazards in the gfx950 scan kernels.
+"""Build-time check of MFMA result and LDS-DMA hazards in the gfx950 scan kernels.
 
     python cuda-vector-search_amd/hazard_check.py cvs_scan.s
 
@@ -13,6 +13,10 @@ every MFMA (fall-through and branch targets, 1 wait state per instruction,
 n + 1 per s_nop n) and fails the build on any read that comes too early, so a
 code change cannot reintroduce the hazard unnoticed.  It reads only assembly
 built in this tree.
+
+A load into LDS takes its LDS address from m0, and needs one wait state after
+the instruction that writes it.  The compiler keeps it for its own loads; the
+kernels' loads are inline asm, where nothing but this check sees it missing.
 """
 
 from __future__ import annotations
@@ -101,9 +105,23 @@ def early_reads(insns, labels):
     return found
 
 
+def early_lds_loads(insns):
+    """Indices of the loads into LDS that directly follow a write of m0."""
+    found = []
+    for i in range(1, len(insns)):
+        op, args = split(insns[i])
+        if "load_lds" in op or (op.startswith("buffer_load") and "lds" in insns[i].split()):
+            before, written = split(insns[i - 1])
+            if before.startswith("s_") and written[:1] == ["m0"]:
+                found.append(i)
+    return found
+
+
 def check(path) -> list[str]:
     problems = []
     for name, (insns, labels) in kernels(Path(path).read_text()).items():
+        for i in early_lds_loads(insns):
+            problems.append(f"{name}: '{insns[i]}' needs a wait state after '{insns[i - 1]}'")
         for i, j, ws, need in early_reads(insns, labels):
             problems.append(f"{name}: '{insns[j]}' reads the result of '{insns[i]}' after {ws} of {need} "
                             "wait states")
@@ -116,7 +134,7 @@ def main(argv):
         bad += check(p)
     for line in bad[:20]:
         print(line)
-    print(f"{len(bad)} early MFMA result reads")
+    print(f"{len(bad)} early MFMA result reads and LDS loads")
     return 1 if bad else 0
 
 

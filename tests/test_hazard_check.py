@@ -60,3 +60,23 @@ def test_built_scans_have_no_early_reads():
         if not asm.exists():
             pytest.skip("library not built in this tree")
         assert hc().check(asm) == []
+
+
+def test_lds_load_right_after_its_m0_is_caught():
+    mod = hc()
+    load = "\tglobal_load_lds_dwordx4 v2, s[4:5] nt\n"
+    for gap, found in (("", [1]), ("\ts_nop 0\n", []), ("\ts_mov_b32 s9, s8\n", [])):
+        asm = kernel("\ts_mov_b32 m0, s8\n" + gap + load)
+        assert mod.early_lds_loads(mod.kernels(asm)["_Z6kernelv"][0]) == found
+
+
+def test_built_lds_loads_wait_for_m0():
+    import pytest
+
+    mod = hc()
+    for name in ("cvs_scan.s", "cvs_scan_q8.s", "cvs_gscan.s"):
+        asm = PKG / "_build" / name
+        if not asm.exists():
+            pytest.skip("library not built in this tree")
+        for insns, _ in mod.kernels(asm.read_text()).values():
+            assert mod.early_lds_loads(insns) == []
