@@ -443,9 +443,13 @@ class Engine:
         import torch
 
         self._check_matrix(x, "corpus")
+        dev = x.device
+        if q.device != dev or q.dtype != x.dtype:  # (Index(device="cuda") under another current device)
+            raise RuntimeError("queries and corpus must be float16 on the same device")
+        if x.shape[0] >= 2**31 - 1:
+            raise RuntimeError("corpus must have fewer than 2^31 rows")
         nq, dim = q.shape
         n, d = x.shape
-        dev = x.device
         index = dev.index
         key = (nq, n, d, dim, k, normalize, xq is None, index)
         ws_bytes = self._search_bytes.get(key)

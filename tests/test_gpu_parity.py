@@ -728,6 +728,8 @@ def test_search_in_one_call_equals_its_parts(eng, metric, d):
             i.data_ptr(), 0, None)
     assert eng.lib.cvs_search(*args) != 0 and b"workspace" in eng.lib.cvs_last_error()
     assert eng.lib.cvs_search(*args[:6], 0, *args[7:]) != 0
+    with pytest.raises(RuntimeError, match="same device"):  # refused before anything is launched
+        eng.search(q.half(), index._x, 5, False)
 
 
 def test_topk_rows_errors(eng):
