@@ -548,8 +548,56 @@ int cvs_fused_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int64_t bq, int6
 
 namespace {
 
-// The score matrix out [nq, n] (fp32 or fp16).  Query blocks and chunking as the
-// fused plan's query-stationary scan.
+// The tiled-GEMM scan for a score matrix (false: the query-stationary scan, cfg
+// unchanged).  Unlike a search it writes 4 or 2 bytes a score, which cost its
+// large tiles the least: 1 KB of a query at a time.  Measured over widths 64
+// to 2048 (us, query-stationary -> tiled, fp32; fp16 gains the same or more):
+//  * small matrices and corpora that the MALL holds: the smallest tiles, two
+//    a CU, fill the GPU soonest (64 x 30000 x 512 16 -> 8.5, 300 x 20000 x 768 25 ->
+//    20, x 1536 45 -> 32, 600 x 50000 x 256 45 -> 36, x 1024 177 -> 83).  Width
+//    384 has the faster query-stationary kernel from 32768 rows on (200 x 50000 22,
+//    22), width 768 from 32M scores (600 x 50000 72 -> 66, 503 x 114000 131 -> 180)
+//    until those of the next line pay (from 100M);
+//  * matrices past 60M scores: 256 x 256 tiles (1000 x 200000 x 256 279 -> 229, small
+//    tiles 354; x 768 435 -> 423; x 1024 1004 -> 514), unless they would pad the
+//    batch by over 15%: then 128 queries a tile where those are the faster (d > 768);
+//    at width 384 262 -> 282, not taken;
+//  * up to 128 queries over a larger corpus both wait for its rows, the
+//    query-stationary scan the same or less (128 x 400000 x 640 156 -> 170, 128 x 128
+//    fp32 63 -> 71, x 768 177 -> 184, 100 x 100000 x 1536 82 -> 85), except past 768
+//    (128 x 400000 x 1024 262 -> 224) and where fp16 stores are cheap (x 64 41 -> 29);
+//  * up to 64 queries over a larger corpus: tiles of 256 rows up to width 256
+//    (64 x 1M x 256 162 -> 155; x 512 264 -> 267, not taken) and past 1536 (x 2048 1004 -> 842).
+bool gemm_scores_cfg(int64_t nq, int64_t n, int64_t d, bool fp32, ScanCfg* cfg) {
+  if (nq <= 32 || n < 2048 || d > kGscanMaxWidth) return false;
+  ScanCfg c{32, 2, 2, 2, -1};  // 128 queries x 128 rows
+  if (nq <= 64) {
+    c.qb = 1;
+    if (n * d > (1 << 26)) {
+      if (d > 256 && d <= 1536) return false;
+      if (d <= 256 || n > (1 << 18)) c.rb = 4;
+    }
+  } else if (nq <= 128) {
+    if (d == 384 || d == 768 || d == 1536) return false;
+    if (n > (1 << 17)) {
+      if (d > 768) c.rb = 4;
+      else if (fp32 || d >= 256) return false;
+    }
+  } else if (nq * n >= (d == 768 ? 100000000 : 60000000)) {
+    if (d == 384) return false;
+    c.rb = 4;
+    if (20 * ceil_div(nq, 256) * 256 <= 23 * ceil_div(nq, 128) * 128) c.qb = 4;
+    else if (d <= 768) return false;
+  } else if ((d == 384 && (n > kRowDirect || nq * n > 20000000)) || (d == 768 && nq * n > 32000000)) {
+    return false;
+  }
+  // (fewer tiles than half the CUs: the query-stationary scan's are smaller)
+  if (ceil_div(nq, c.bq()) * ceil_div(n, c.tile_rows()) < 128) return false;
+  *cfg = c;
+  return true;
+}
+
+// The score matrix out [nq, n] (fp32 or fp16), chunked as the fused plan's scans.
 hipError_t launch_scores(const _Float16* q, const _Float16* x, int64_t nq, int64_t n, int64_t d, void* out, bool fp32,
                          int cus, hipStream_t s) {
   if (nq == 1) {  // one query: the GEMV, 16 waves per CU of at least 16 rows
@@ -567,12 +615,16 @@ hipError_t launch_scores(const _Float16* q, const _Float16* x, int64_t nq, int64
   ScanCfg cfg;
   int64_t bq = nq <= 16 ? 16 : nq <= 32 ? 32 : nq <= 64 ? 64 : (nq <= 128 || d != 384) ? 128 : 256;
   while (!cfg_for(bq, d, &cfg)) bq >>= 1;
-  const int64_t groups = ceil_div(nq, bq);
+  const bool tiled = gemm_scores_cfg(nq, n, d, fp32, &cfg);
+  const int64_t groups = ceil_div(nq, cfg.bq());
   const int64_t ntiles = ceil_div(n, cfg.tile_rows());
   const int64_t max_chunks = std::min<int64_t>(ntiles, 65535);
   const int64_t most = std::min<int64_t>(max_chunks, std::max<int64_t>(1, groups > 1 ? align_up(ntiles / 2, 8) : ntiles / 2));
-  int64_t c = groups == 1 ? std::min<int64_t>(cus, most)
-                          : best_chunks(groups, ntiles, cus, most, qstat_tile_cost(cfg, d));
+  int64_t c;
+  if (tiled)
+    c = best_chunks(groups, ntiles, cus * gemm_per_cu(cfg), max_chunks, gemm_tile_cost(cfg, d, groups, groups * ntiles <= cus));
+  else
+    c = groups == 1 ? std::min<int64_t>(cus, most) : best_chunks(groups, ntiles, cus, most, qstat_tile_cost(cfg, d));
   const int64_t tpc = ceil_div(ntiles, c);
   const int xcd_pair = groups > 1 && c % 8 == 0 ? 1 : 0;
   if (!xcd_pair) c = ceil_div(ntiles, tpc);

@@ -23,6 +23,11 @@
 // the whole scan, tail included, of the query-stationary kernel of that width),
 // 0.86 at width 1664 where the query-stationary scan reached 0.31, and 128 x
 // 128 tiles, two workgroups a CU, 0.76 at width 128 (0.51).
+//
+// kStore* writes the score matrix from the same tiles, straight from the
+// accumulators: lanes swap so that four of them write 64 bytes of a query.
+// (32 bytes by two lanes, without the swaps: 1000 x 1024 over 200k rows, 800 MB of
+// scores, 523 us in fp32 and 453 in fp16, so 497 and 443.)
 #include <type_traits>
 
 #include "cvs_common.h"
@@ -33,6 +38,7 @@ namespace cvs {
 namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
 
 constexpr int kRing = 3;      // corpus stages and query phases in LDS
 constexpr int kStage = 32;    // staged entries per wave
@@ -110,13 +116,34 @@ __device__ __forceinline__ float wave_compact_regs(float* lv, int* li, int count
   return key_score(t);
 }
 
+// Two scores as fp16.
+__device__ __forceinline__ uint32_t pack2(float x, float y) {
+  typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, half2v{(_Float16)x, (_Float16)y});
+}
+
+// The N scores v of rows row, row + 1, ... below n into a query's scores `out`
+// (16 bytes at the element's alignment: n may be odd).
+template <int N, class T, class V>
+__device__ __forceinline__ void store_rows(T* out, int64_t row, int64_t n, V v) {
+  typedef V any __attribute__((aligned(sizeof(T))));
+  if (row + N <= n) {
+    *reinterpret_cast<any*>(out + row) = v;
+  } else {
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      if (row + j < n) out[row + j] = v[j];
+  }
+}
+
 template <int QB, int RB, int MODE>
 __global__ __launch_bounds__(kBlock, QB * RB > 4 ? 1 : 2) void gscan_kernel(ScanArgs a) {
   constexpr int TQ = 64 * QB, TR = 64 * RB;   // queries, rows per workgroup tile
   constexpr int LA = TR / 32, LQ = TQ / 64;   // 1 KiB loads per wave: of a corpus stage, of a query phase
   constexpr int ASTAGE = TR * 128, QPHASE = TQ * 64;
   constexpr bool APP = MODE == kAppend;
-  static_assert(MODE == kAppend || MODE == kMax, "append and sampling");
+  constexpr bool STORE = MODE == kStoreF32 || MODE == kStoreF16;
+  static_assert(APP || STORE || MODE == kMax, "append, sampling and the score matrix");
   __shared__ __attribute__((aligned(1024))) unsigned char sa[kRing * ASTAGE];
   __shared__ __attribute__((aligned(1024))) unsigned char sq[kRing * QPHASE];
   __shared__ int lcnt[APP ? 2 : 1][APP ? TQ : 1];     // entries in each owned list
@@ -405,6 +432,63 @@ __global__ __launch_bounds__(kBlock, QB * RB > 4 ? 1 : 2) void gscan_kernel(Scan
             a.umax[(int64_t)qi * a.units + ((chunk * a.spt + (t - t_begin)) * 2 + wr) * (2 * RB) + 2 * rb + kg] = m;
         }
       }
+    } else if constexpr (STORE) {
+      // Lanes of 16 swap halves of the block, so that 4 lanes write 64 bytes of a
+      // query at once: afterwards a lane holds queries h * 16 + col % 16, h = 0, 1.
+      const int qcol = q0 + wq * QB * 32 + (col & 15);
+      const int up = col >> 4;
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+          asm volatile("" : "+a"(acc[rb][qb]));  // keeps the block's reads here (all 256 would not fit)
+          const f32x16 c = acc[rb][qb];
+          if constexpr (MODE == kStoreF32) {
+#pragma unroll
+            for (int g = 0; g < 4; g += 2) {  // rows 8 g + 4 kg + 0..3, and 8 more
+              f32x4 v[2];
+#pragma unroll
+              for (int j = 0; j < 4; ++j) {
+                const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(c[4 * g + j]),
+                                                                __float_as_uint(c[4 * g + 4 + j]), false, false);
+                v[0][j] = __uint_as_float(r[0]);
+                v[1][j] = __uint_as_float(r[1]);
+              }
+              const int64_t row = rowb + 32 * rb + 8 * (g + up);
+#pragma unroll
+              for (int h = 0; h < 2; ++h) {
+                const int qi = qcol + 32 * qb + 16 * h;
+                if (qi < a.nq) store_rows<4>(static_cast<float*>(a.out) + (int64_t)qi * n, row, n, v[h]);
+              }
+            }
+          } else {
+            uint4v v[2];  // rows 16 p + 8 kg + 0..7: the halves' fours swapped
+#pragma unroll
+            for (int p = 0; p < 2; ++p) {
+#pragma unroll
+              for (int j = 0; j < 2; ++j) {
+                const auto r = __builtin_amdgcn_permlane32_swap(pack2(c[8 * p + 2 * j], c[8 * p + 2 * j + 1]),
+                                                                pack2(c[8 * p + 4 + 2 * j], c[8 * p + 5 + 2 * j]), false, false);
+                v[p][j] = r[0];
+                v[p][2 + j] = r[1];
+              }
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const auto r = __builtin_amdgcn_permlane16_swap(v[0][j], v[1][j], false, false);
+              v[0][j] = r[0];
+              v[1][j] = r[1];
+            }
+            const int64_t row = rowb - 4 * kg + 32 * rb + 16 * up + 8 * kg;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const int qi = qcol + 32 * qb + 16 * h;
+              if (qi < a.nq)
+                store_rows<8>(static_cast<_Float16*>(a.out) + (int64_t)qi * n, row, n, __builtin_bit_cast(half8, v[h]));
+            }
+          }
+        }
+      }
     } else {
       // Stages the passing lanes' scores of half blocks b0, b0 + 1, ... (of half
       // block b0 those of the lanes in `rem`) until the staging area is full
@@ -455,14 +539,14 @@ __global__ __launch_bounds__(kBlock, QB * RB > 4 ? 1 : 2) void gscan_kernel(Scan
   }
   if constexpr (APP) {
     if (st_n > 0) flush();
-  } else if (a.agg) {
+  } else if (MODE == kMax && a.agg) {
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
       const int qi = q0 + (wq * QB + qb) * 32 + col;
       if (qi < a.nq)
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb)
-          a.umax[(int64_t)qi * a.units + (chunk * 2 + wr) * (2 * RB) + 2 * rb + kg] = umx[rb][qb];
+          a.umax[(int64_t)qi * a.units + (chunk * 2 + wr) * (2 * RB) + 2 * rb + kg] = umx[MODE == kMax ? rb : 0][MODE == kMax ? qb : 0];
     }
   }
   // the trailing loads land before this workgroup's LDS can be handed on; counts are final
@@ -480,15 +564,20 @@ template <int QB, int RB>
 hipError_t launch_g(int mode, const ScanArgs& a, int grid, hipStream_t s) {
   if (mode == kAppend)
     hipLaunchKernelGGL((gscan_kernel<QB, RB, kAppend>), dim3(grid), dim3(kBlock), 0, s, a);
-  else
+  else if (mode == kMax)
     hipLaunchKernelGGL((gscan_kernel<QB, RB, kMax>), dim3(grid), dim3(kBlock), 0, s, a);
+  else if (mode == kStoreF32)
+    hipLaunchKernelGGL((gscan_kernel<QB, RB, kStoreF32>), dim3(grid), dim3(kBlock), 0, s, a);
+  else
+    hipLaunchKernelGGL((gscan_kernel<QB, RB, kStoreF16>), dim3(grid), dim3(kBlock), 0, s, a);
   return hipGetLastError();
 }
 
 }  // namespace
 
 hipError_t launch_gscan(const ScanCfg& c, int mode, const ScanArgs& a, int grid, hipStream_t s) {
-  if ((mode != kAppend && mode != kMax) || a.d < 64 || a.d % 64 != 0 || a.d > kGscanMaxWidth || a.nq < 1 || a.ntiles < 1 ||
+  const bool store = mode == kStoreF32 || mode == kStoreF16;
+  if ((mode != kAppend && mode != kMax && !store) || (store && a.out == nullptr) || a.d < 64 || a.d % 64 != 0 || a.d > kGscanMaxWidth || a.nq < 1 || a.ntiles < 1 ||
       a.umax_in != nullptr || a.qq_out != nullptr || (mode == kMax && (a.umax == nullptr || a.agg > 1)) ||
       (mode == kAppend && (a.cap > kMaxCap || a.k > a.cap || a.nlists != a.nchunks * 2)))
     return hipErrorInvalidValue;

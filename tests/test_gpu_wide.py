@@ -52,6 +52,40 @@ def test_wide_scores_match_oracle(eng, nq, n, d):
     np.testing.assert_allclose(s16.float().cpu().numpy(), ref, rtol=0, atol=3e-3)
 
 
+# The tiled-GEMM scan's tiles of 64 to 256 queries and 128 or 256 rows: batches a
+# query past and short of them, odd row counts (stores off 16-byte alignment, a
+# last tile of few rows), the narrowest width and ones past 1536; and sizes
+# either side of where the query-stationary scan takes over.
+TILED_SCORES = [(33, 60001, 64), (64, 50003, 512), (48, 16387, 1024), (64, 9001, 2048),  # 64 x 128
+                (40, 270001, 256), (33, 263001, 1600),                                   # 64 x 256
+                (65, 30005, 128), (255, 20002, 1088), (257, 30007, 192), (300, 8193, 384), (512, 40003, 640),
+                (300, 8192, 1536), (129, 25007, 768), (513, 4101, 2048),                 # 128 x 128
+                (100, 131077, 832), (300, 200003, 832),                                  # 128 x 256
+                (256, 240001, 64), (512, 200003, 768),                                   # 256 x 256
+                (128, 2049, 64), (200, 32770, 384), (300, 200003, 128), (128, 131077, 128)]
+
+
+@pytest.mark.parametrize("nq,n,d", TILED_SCORES)
+def test_tiled_scores_match_fp64(eng, nq, n, d):
+    """The whole matrix, and nothing past its ends."""
+    say(f"tiled scores nq={nq} n={n} d={d}")
+    x, q = make(n, d, nq, seed=n + d)
+    x, q = x.cuda(), q.cuda()
+    ref = torch.cat([q.double() @ r.double().T for r in x.split(1 << 14)], 1)
+    guard = 64
+    for dtype in (torch.float32, torch.float16):
+        buf = torch.full((nq * n + 2 * guard,), 7.0, dtype=dtype, device="cuda")
+        out = buf[guard:guard + nq * n]
+        rc = eng.lib.cvs_scores(q.data_ptr(), x.data_ptr(), nq, n, d, out.data_ptr(), int(dtype == torch.float32), 0, None)
+        torch.cuda.synchronize()
+        assert rc == 0, eng.lib.cvs_last_error()
+        # unit rows: a sum of d products in fp32 is off by at most d 2^-24 (1 + rounding of the
+        # norms); fp16 rounds scores below 1.01 by 2^-11 at most
+        bound = 1.1 * d * 2.0**-24 + (2.0**-11 if dtype == torch.float16 else 0.0)
+        assert float((out.view(nq, n).double() - ref).abs().max()) <= bound
+        assert bool((buf[:guard] == 7).all()) and bool((buf[guard + nq * n:] == 7).all())
+
+
 WIDE_FUSED = [
     (20000, 1600, 1, 10),     # batch-1 GEMV
     (20000, 2048, 16, 10),    # 16-query block (16x16x32 MFMA)
