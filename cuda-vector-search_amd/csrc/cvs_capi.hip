@@ -282,11 +282,19 @@ bool gemm_cfg(int64_t nq, int64_t n, int64_t d, int64_t k, int cus, const ScanCf
 // 32000 40 / 34, 40 x 384 26 / 35); short ones while few scores are stored, more of
 // them where the scans are slow (1 x 384 over 5000, k = 10 19 / 9, over 32000
 // 20 / 24; 200 x 384 over 8000 28 / 26, 1000 x 384 42 / 50; 200 x 768 over
-// 16000 39 / 34).
+// 16000 39 / 34).  From width 512, where the matrix comes from the tiled-GEMM scan
+// (40 x 768 over 24000 36 / 25, 200 x 512 37 / 32, but over 12000 and fewer the lists
+// as often; 84 x 640 over 32000 33 / 36; from 1024 up to 10M scores: 300 over 24000 94 / 67,
+// over 32000 92 / 80, 600 over 24000 76 / 89; k = 1 104 x 1280 over 32500 42 / 49).
+// (Width 1536 has query-stationary kernels for both; not measured.)
 constexpr int64_t kDirectBytes = 256ll << 20;  // of scores (the MALL holds them)
 bool direct_search(int64_t nq, int64_t n, int64_t d, int64_t k, bool sampled) {
   if (n > kRowDirect || nq * n * 4 > kDirectBytes) return false;
   if (!sampled) return true;
+  if (nq > 32 && k >= 4 && d >= 512 && d != 1536 &&
+      (d >= 1024 ? nq * n <= 10000000
+                 : n > (d < 768 ? 16384 : 0) && n <= 24576 && nq <= 256 && nq * n <= 5000000))
+    return true;
   if (k >= 32) return nq <= 16 || (n <= 16384 && nq * n <= 8000000);
   if (nq == 1) return n <= 16384 || d >= 768;
   return d >= 768 ? n <= 16384 && nq * n <= 3300000 : n <= 8192 && nq * n <= 1700000;

@@ -677,7 +677,9 @@ def test_topk_rows_threshold_edges(eng, nq, n, k, data):
 
 @pytest.mark.parametrize("nq,n,d,k", [(1, 1, 64, 1), (1, 5003, 384, 5), (16, 8192, 768, 10), (17, 700, 384, 256),
                                       (300, 8191, 128, 100), (5, 8193, 320, 3), (1, 8192, 1600, 256),
-                                      (9, 32768, 256, 40), (1, 16385, 768, 10), (100, 16000, 768, 200)])
+                                      (9, 32768, 256, 40), (1, 16385, 768, 10), (100, 16000, 768, 200),
+                                      (33, 24577, 512, 10), (200, 24576, 768, 10), (300, 32768, 1024, 100),
+                                      (34, 32767, 2048, 1)])
 def test_small_corpus_search_is_exact(eng, nq, n, d, k):
     """Corpora of few rows searched through a score matrix (and one that is
     not), against the lists (forced by a flag) and the oracle; exact
