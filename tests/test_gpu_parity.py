@@ -565,6 +565,60 @@ def test_prep_rows_matches_oracle(eng, n, d, width):
         np.testing.assert_array_equal(inplace.cpu().numpy(), got)
 
 
+def fp32_normalized(x):
+    """fp16 rows as the stored format defines them: fp32 sums of the squares over the
+    columns of equal index mod 64 in ascending order, a tree over the 64 sums
+    (32, 16, ... 1 apart), the fp32 norm clamped at 1e-12, the fp32 quotient, fp16."""
+    n, d = x.shape
+    xf = np.zeros((n, -(-d // 64), 64), dtype=np.float32)
+    xf.reshape(n, -1)[:, :d] = x
+    s = np.zeros((n, 64), dtype=np.float32)
+    with np.errstate(all="ignore"):
+        for m in range(xf.shape[1]):
+            s = s + xf[:, m] * xf[:, m]  # (the squares are exact)
+        for off in (32, 16, 8, 4, 2, 1):
+            s = s[:, :off] + s[:, off:]
+        return (x.astype(np.float32) / np.fmax(np.sqrt(s), np.float32(1e-12))).astype(np.float16)
+
+
+@pytest.mark.parametrize("n,d,width", [(1, 1, 64), (3000, 64, 64), (257, 100, 128), (300, 129, 192), (2000, 384, 384),
+                                       (65, 387, 448), (2000, 768, 768), (33, 769, 832), (513, 1536, 1536),
+                                       (129, 1537, 1600), (500, 2048, 2048), (31, 4096, 4096), (65, 4100, 4160),
+                                       (9, 9001, 9024)])
+def test_prep_rows_stores_the_same_bits(eng, n, d, width):
+    """Normalised rows bit for bit, out of place from an unaligned source, in place
+    and with rows of zeros, subnormals, infinities and NaNs."""
+    say(f"prep_rows bits n={n} d={d} width={width}")
+    g = torch.Generator().manual_seed(n + d)
+    x = (torch.randn(n, d + 1, generator=g) * torch.rand(n, 1, generator=g) * 4).half()[:, 1:]
+    if n > 8:
+        x[0] = 0.0
+        x[1] = -0.0
+        x[2] *= 2.0**-20
+        x[3] = 0.0
+        x[3, d // 2] = -(2.0**-24)
+        x[4, d - 1] = float("inf")
+        x[5, 0] = float("nan")
+        x[6, 0], x[6, d - 1] = float("nan"), float("-inf")
+        x[7] = 65504.0
+    want = fp32_normalized(x.numpy())
+    src = torch.zeros(n, d + 1, dtype=torch.float16, device="cuda")[:, 1:]
+    src.copy_(x)
+    out = torch.full((n, width), 7.0, dtype=torch.float16, device="cuda")
+    eng.prep_rows(src, out, True)
+    got = [out[:, :d]]
+    inplace = torch.empty(n, d, dtype=torch.float16, device="cuda").copy_(x)
+    eng.prep_rows(inplace, inplace, True)
+    got.append(inplace)
+    torch.cuda.synchronize()
+    assert not out[:, d:].any()
+    nan = np.isnan(want)
+    for t in got:
+        t = t.cpu().numpy()
+        assert np.array_equal(np.isnan(t), nan)
+        assert np.array_equal(t.view(np.int16)[~nan], want.view(np.int16)[~nan])
+
+
 def test_prep_rows_errors(eng):
     x = torch.zeros(4, 64, dtype=torch.float16, device="cuda")
     with pytest.raises(RuntimeError, match="destination width"):
