@@ -20,6 +20,12 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kWave = 64;
 constexpr int kBlock = 256;  // 4 waves, one per SIMD
 
+// Filter threshold (m >= threshold passes) of a query tile's columns past the
+// batch, which load the last query again: NaN, which nothing reaches.  A score of
+// +inf (an fp16 element overflowed) reaches +inf, and its row would be appended
+// to lists that the workspace does not hold.
+constexpr float kNoThreshold = __builtin_nanf("");
+
 // ---- 64-bit search keys ----------------------------------------------------
 
 __device__ __forceinline__ uint32_t float_order(float v) {

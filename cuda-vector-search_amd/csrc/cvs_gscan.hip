@@ -254,13 +254,13 @@ __global__ __launch_bounds__(kBlock, QB * RB > 4 ? 1 : 2) void gscan_kernel(Scan
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) {
     const int qi = q0 + (wq * QB + qb) * 32 + col;
-    thr[qb] = qi >= a.nq ? __builtin_inff() : (APP && a.tau ? a.tau[qi] : -__builtin_inff());
+    thr[qb] = qi >= a.nq ? kNoThreshold : (APP && a.tau ? a.tau[qi] : -__builtin_inff());
   }
   if constexpr (APP) {
     for (int i = tid; i < 2 * TQ; i += kBlock) {
       (&lcnt[0][0])[i] = 0;
       const int qi = q0 + i % TQ;
-      (&thr_s[0][0])[i] = qi >= a.nq ? __builtin_inff() : (a.tau ? a.tau[qi] : -__builtin_inff());
+      (&thr_s[0][0])[i] = qi >= a.nq ? kNoThreshold : (a.tau ? a.tau[qi] : -__builtin_inff());
     }
   }
   wait_vmcnt<0>();  // retires the threshold loads: the compiler then waits on no vector load inside the loop

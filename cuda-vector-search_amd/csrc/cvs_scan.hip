@@ -453,7 +453,7 @@ __global__ __launch_bounds__(scan_waves(QS) * kWave, 1) void scan_kernel(ScanArg
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) {
     const int qi = qwave0 + qb * MS + col;
-    thr[qb] = (qi >= a.nq) ? __builtin_inff() : (a.tau ? a.tau[qi] : -__builtin_inff());
+    thr[qb] = (qi >= a.nq) ? kNoThreshold : (a.tau ? a.tau[qi] : -__builtin_inff());
   }
   // kAppendQ8: this lane's queries' (s_q, |q^|, |e|), for the score bound.
   float4 qm[QB];
@@ -482,7 +482,7 @@ __global__ __launch_bounds__(scan_waves(QS) * kWave, 1) void scan_kernel(ScanArg
     for (int i = tid; i < RS * BQ; i += NT) {
       (&lcnt[0][0])[i] = 0;
       const int qi = grp * BQ + i % BQ;
-      if (!thr_in) (&thr_s[0][0])[i] = (qi >= a.nq) ? __builtin_inff() : (a.tau ? a.tau[qi] : -__builtin_inff());
+      if (!thr_in) (&thr_s[0][0])[i] = (qi >= a.nq) ? kNoThreshold : (a.tau ? a.tau[qi] : -__builtin_inff());
     }
   }
   // kTopK: this lane's running top-k of each query block in the last k of
@@ -665,7 +665,7 @@ __global__ __launch_bounds__(scan_waves(QS) * kWave, 1) void scan_kernel(ScanArg
           if (sum8_i32(c) >= a.k) tk = cand;
         }
       }
-      const float tv = qi >= a.nq ? __builtin_inff() : (a.units_in >= a.k ? order_threshold(tk) : -__builtin_inff());
+      const float tv = qi >= a.nq ? kNoThreshold : (a.units_in >= a.k ? order_threshold(tk) : -__builtin_inff());
       if (g8 == 0)
 #pragma unroll
         for (int r = 0; r < RS; ++r) thr_s[r][ql] = tv;
@@ -903,7 +903,7 @@ __global__ __launch_bounds__(scan_waves(QS) * kWave, 1) void scan_kernel(ScanArg
   auto wait_thresholds = [&]() {
     for (int i = tid; i < BQ; i += NT) {
       const int qi = grp * BQ + i;
-      const float tv = qi >= a.nq ? __builtin_inff() : tau_wait(a.tauw, qi, wait_ticks);
+      const float tv = qi >= a.nq ? kNoThreshold : tau_wait(a.tauw, qi, wait_ticks);
 #pragma unroll
       for (int r = 0; r < RS; ++r) thr_s[r][i] = tv;
     }

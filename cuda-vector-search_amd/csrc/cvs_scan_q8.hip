@@ -151,13 +151,13 @@ __global__ __launch_bounds__(kQ8Waves * kWave, 1) void q8scan384_kernel(ScanArgs
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
       const int qi = grp * kQ8Bq + qgw * 64 + qb * 32 + col;
-      const int qc = min(qi, a.nq - 1);  // columns past nq load the last query; their threshold is +inf
+      const int qc = min(qi, a.nq - 1);  // columns past nq load the last query; kNoThreshold drops them
       i32x4 ld[kQ8Ks];
 #pragma unroll
       for (int ks = 0; ks < kQ8Ks; ++ks) ld[ks] = *(const i32x4*)(a.qf + q8_frag_offset(qc, ks, kg, kQ8Ks));
 #pragma unroll
       for (int ks = 0; ks < kQ8Ks; ++ks) qf[qb][ks] = pin_agpr(ld[ks]);
-      thr[qb] = (qi >= a.nq) ? __builtin_inff() : (a.tau ? a.tau[qi] : -__builtin_inff());
+      thr[qb] = (qi >= a.nq) ? kNoThreshold : (a.tau ? a.tau[qi] : -__builtin_inff());
       qm[qb] = a.qmeta[qc];
     }
   };
@@ -180,7 +180,7 @@ __global__ __launch_bounds__(kQ8Waves * kWave, 1) void q8scan384_kernel(ScanArgs
   for (int i = tid; i < kQ8Bq; i += kQ8Waves * kWave) {
     const int qi = grp * kQ8Bq + i;
     lcnt[i] = 0;
-    if (!fused) thr_s[i] = (qi >= a.nq) ? __builtin_inff() : (a.tau ? a.tau[qi] : -__builtin_inff());
+    if (!fused) thr_s[i] = (qi >= a.nq) ? kNoThreshold : (a.tau ? a.tau[qi] : -__builtin_inff());
   }
   int st_n = 0;  // wave-uniform count of staged entries
 
@@ -405,7 +405,7 @@ __global__ __launch_bounds__(kQ8Waves * kWave, 1) void q8scan384_kernel(ScanArgs
       // the first scanned tile's MFMAs run
       for (int i = tid; i < kQ8Bq; i += kQ8Waves * kWave) {
         const int qi = grp * kQ8Bq + i;
-        thr_s[i] = qi >= a.nq ? __builtin_inff() : tau_wait(a.tauw, qi, wait_ticks);
+        thr_s[i] = qi >= a.nq ? kNoThreshold : tau_wait(a.tauw, qi, wait_ticks);
       }
       __syncthreads();
 #pragma unroll

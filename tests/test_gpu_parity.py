@@ -14,6 +14,7 @@ the k-th score, scores within 1e-3 (oracle.check_exact); score matrices within
 
 from __future__ import annotations
 
+import ctypes
 import sys
 from pathlib import Path
 
@@ -786,6 +787,68 @@ def test_search_in_one_call_equals_its_parts(eng, metric, d):
     assert eng.lib.cvs_search(*args[:6], 0, *args[7:]) != 0
     with pytest.raises(RuntimeError, match="same device"):  # refused before anything is launched
         eng.search(q.half(), index._x, 5, False)
+
+
+# Query tiles with columns past the batch, of every filtering scan: the
+# query-stationary ones (16 to 256 queries a tile, thresholds from a launch, from
+# the scan itself and none), the tiled ones (64, 128 and 256 queries) and the int8
+# ones (general and 8-wave).
+INF_CASES = [(5, 40001, 384, 10, "fused"), (20, 40001, 384, 10, "fused"), (100, 40001, 384, 10, "fused"),
+             (200, 100001, 384, 10, "fused"), (300, 60001, 384, 100, "fused"), (5, 40001, 768, 10, "fused"),
+             (33, 40001, 768, 10, "fused"), (129, 40001, 768, 10, "fused"), (9, 40001, 1536, 10, "fused"),
+             (20, 40001, 2048, 10, "fused"), (50, 40001, 1536, 10, "fused"),
+             (33, 40001, 128, 10, "fused"), (40, 40001, 1024, 10, "fused"), (100, 40001, 1024, 10, "fused"),
+             (129, 200001, 1024, 10, "fused"), (192, 200001, 1024, 10, "fused"), (300, 200001, 640, 200, "fused"),
+             (5, 40001, 384, 10, "int8"), (40, 40001, 384, 10, "int8"), (200, 60001, 384, 10, "int8"),
+             (300, 60001, 384, 10, "int8"), (33, 40001, 768, 100, "int8"), (100, 40001, 1024, 10, "int8")]
+
+
+@pytest.mark.parametrize("nq,n,d,k,path", INF_CASES)
+@pytest.mark.parametrize("flags", [0, _ext.FLAG_NO_PREPASS], ids=["auto", "nosample"])
+def test_infinite_scores_stay_in_their_lists(eng, nq, n, d, k, path, flags):
+    """Rows with an infinite element (an fp32 value past 65504 stored as fp16) that
+    the last query scores +inf: nothing is written past the workspace, and the
+    fp16 path ranks them first."""
+    say(f"infinite scores nq={nq} n={n} d={d} k={k} {path} flags={flags}")
+    x, q = make(n, d, nq, seed=n + d + nq)
+    rows = torch.tensor([3, n // 3, n // 2, n - 1])
+    x[rows, 7] = float("inf")
+    q[:, 7] = -0.5 * q[:, 7].abs() - 2.0**-10
+    q[0, 7] = q[-1, 7] = 0.25
+    xd, qd = x.cuda(), q.cuda()
+    if path == "int8":
+        xq = eng.q8_build(xd)
+        _, need = eng.q8_plan(nq, n, d, k, flags)
+    else:
+        _, need = eng.plan(nq, n, d, k, flags=flags)
+    guard = 1 << 20
+    buf = torch.full((need + 2 * guard,), 0x5A, dtype=torch.uint8, device="cuda")
+    v = torch.full((nq + 2, k), 7.0, device="cuda")
+    i = torch.full((nq + 2, k), 7, dtype=torch.int32, device="cuda")
+    ws, vp, ip = buf.data_ptr() + guard, v[1:].data_ptr(), i[1:].data_ptr()
+    plan = (ctypes.c_int64 * 2)()
+    if path == "int8":
+        rc = eng.lib.cvs_q8_topk(qd.data_ptr(), xd.data_ptr(), xq.data_ptr(), xq.numel(), nq, n, d, k, flags, ws, need,
+                                 vp, ip, plan, 0, eng._stream(qd.device))
+    else:
+        rc = eng.lib.cvs_fused_topk(qd.data_ptr(), xd.data_ptr(), nq, n, d, k, 0, 0, flags, ws, need, vp, ip, plan, 0,
+                                    eng._stream(qd.device))
+    torch.cuda.synchronize()
+    assert rc == 0, eng.lib.cvs_last_error()
+    assert bool((buf[:guard] == 0x5A).all()) and bool((buf[guard + need:] == 0x5A).all())
+    assert bool((v[[0, -1]] == 7).all()) and bool((i[[0, -1]] == 7).all())
+    if path == "int8":  # (an infinite scale leaves the pre-filter's bounds undefined)
+        return
+    v, i = v[1:-1].cpu(), i[1:-1].cpu().long()
+    for b in (0, nq - 1):
+        assert torch.isinf(v[b, :4]).all() and torch.equal(i[b, :4], rows)
+    finite = q.double() @ x.double().clamp(-65504, 65504).T
+    finite[:, rows] = -float("inf")
+    finite[[0, -1]] = torch.where(finite[[0, -1]] == -float("inf"), float("inf"), finite[[0, -1]])
+    want = torch.topk(finite, k, dim=1).values
+    # unit rows, fp32 sums of d products: off by at most d 2^-24 each
+    torch.testing.assert_close(v.double(), want, rtol=0, atol=2 * d * 2.0**-24)
+    torch.testing.assert_close(torch.gather(finite, 1, i), want, rtol=0, atol=2 * d * 2.0**-24)
 
 
 def test_topk_rows_errors(eng):
