@@ -172,6 +172,18 @@ double scan_cost(int64_t groups, int64_t ntiles, int64_t chunks, int64_t slots, 
   return (double)rounds * ((double)tpc * tile + 860.0);
 }
 
+// Entries of a candidate list.
+int64_t list_cap(int64_t k) { return std::max<int64_t>(128, pow2_at_least(k + 64)); }
+
+// The most chunks, rs lists per query each, whose lists stay within 512 MB (a
+// single chunk's may not).  A search allocates them per call; without the bound
+// several rounds of chunks took 1.5 GB (700 queries, k = 256, width 1024, 2M rows)
+// and 8 chunks of 100000 queries 3.3.
+constexpr int64_t kListBytes = 512ll << 20;
+int64_t list_chunks(int64_t nq, int64_t rs, int64_t k) {
+  return std::max<int64_t>(1, kListBytes / (std::max<int64_t>(nq, 1) * rs * list_cap(k) * 8));
+}
+
 // Chunks of a scan, one workgroup per (group, chunk): the count that ends
 // soonest, the most chunks among equals (more CUs pull the corpus from
 // HBM: 256 x 1024 over 200k rows with 128 chunks 178 us, with 112 202).  With
@@ -180,19 +192,25 @@ double scan_cost(int64_t groups, int64_t ntiles, int64_t chunks, int64_t slots, 
 // 6 and 7 groups and left a second round nearly empty: 600 x 384 over 1M rows
 // through the int8 path 522 us, now 425; 700 x 768 over 200k 461 -> 316; 700 x 768,
 // k = 100, over 1M 1404 -> 986; scores of 300 x 768 over 100k 137 -> 87.)
-int64_t best_chunks(int64_t groups, int64_t ntiles, int64_t slots, int64_t max_chunks, double tile) {
+// few: fewer than 8 too, where the groups alone nearly fill the GPU (9000 x 384
+// over 200k: 7 chunks 1477 us, 8 in two rounds 1796); not for the int8 scan,
+// whose lists are not cut when they fill (there 5306 and 1423).
+int64_t best_chunks(int64_t groups, int64_t ntiles, int64_t slots, int64_t max_chunks, double tile, bool few = false) {
   if (groups == 1) return std::max<int64_t>(1, std::min<int64_t>({slots, ntiles, max_chunks}));
   const int64_t step = ntiles >= 8 && max_chunks >= 8 ? 8 : 1;
   const int64_t most = std::min<int64_t>(max_chunks, align_up(ntiles, step)) / step * step;
   int64_t best = step;
   double cost = -1;
-  for (int r = 1; r <= 3; ++r) {  // the most chunks that r rounds hold
-    const int64_t c = std::max<int64_t>(step, std::min<int64_t>(most, r * slots / (groups * step) * step));
+  auto consider = [&](int64_t c) {
     const double t = scan_cost(groups, ntiles, c, slots, tile);
     if (cost < 0 || t < cost || (t == cost && c > best)) {
       cost = t;
       best = c;
     }
+  };
+  for (int r = 1; r <= 3; ++r) {  // the most chunks that r rounds hold
+    consider(std::max<int64_t>(step, std::min<int64_t>(most, r * slots / (groups * step) * step)));
+    if (const int64_t c = r * slots / groups; few && c >= 1 && c < step) consider(c);
   }
   return best;
 }
@@ -262,7 +280,8 @@ bool gemm_cfg(int64_t nq, int64_t n, int64_t d, int64_t k, int cus, const ScanCf
     const int64_t groups = ceil_div(nq, c.bq()), ntiles = ceil_div(n, c.tile_rows());
     const int64_t slots = cus * gemm_per_cu(c);
     const double tile = gemm_tile_cost(c, d, groups, groups * ntiles <= cus);
-    const double t = scan_cost(groups, ntiles, best_chunks(groups, ntiles, slots, kSelectMaxLists / 2, tile), slots, tile);
+    const int64_t max_chunks = std::min<int64_t>(kSelectMaxLists / 2, list_chunks(nq, 2, k));
+    const double t = scan_cost(groups, ntiles, best_chunks(groups, ntiles, slots, max_chunks, tile, true), slots, tile);
     if (t < (found ? cost : 0.85 * cost)) {  // (15%: the model's error)
       cost = t;
       *out = c;
@@ -385,7 +404,8 @@ int make_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int64_t bq, int64_t c
     P.tile_rows = P.cfg.tile_rows();
     P.ntiles = ceil_div(n, P.tile_rows);
     const int64_t rs = P.cfg.rs();
-    const int64_t max_chunks = std::min<int64_t>({P.ntiles, 65535, kSelectMaxLists / rs});
+    int64_t max_chunks = std::min<int64_t>({P.ntiles, 65535, kSelectMaxLists / rs});
+    if (chunks == 0) max_chunks = std::min(max_chunks, list_chunks(nq, rs, k));
     int64_t c;
     if (chunks > 0) {
       c = std::max<int64_t>(1, std::min<int64_t>(chunks, max_chunks));
@@ -393,20 +413,20 @@ int make_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int64_t bq, int64_t c
       c = ceil_div(P.ntiles, P.tpc);
     } else if (P.cfg.gemm()) {
       c = best_chunks(P.groups, P.ntiles, cus * gemm_per_cu(P.cfg), max_chunks,
-                      gemm_tile_cost(P.cfg, d, P.groups, P.groups * P.ntiles <= cus));
+                      gemm_tile_cost(P.cfg, d, P.groups, P.groups * P.ntiles <= cus), true);
       P.tpc = ceil_div(P.ntiles, c);
-      if (P.groups == 1) c = ceil_div(P.ntiles, P.tpc);
+      if (P.groups == 1 || c % 8 != 0) c = ceil_div(P.ntiles, P.tpc);
     } else {
       const int64_t most = std::min<int64_t>(max_chunks, std::max<int64_t>(1, P.groups > 1 ? align_up(P.ntiles / 2, 8) : P.ntiles / 2));
       c = P.groups == 1 ? std::min<int64_t>(cus, most)
-                        : best_chunks(P.groups, P.ntiles, cus, most, qstat_tile_cost(P.cfg, d));
+                        : best_chunks(P.groups, P.ntiles, cus, most, qstat_tile_cost(P.cfg, d), true);
       P.tpc = ceil_div(P.ntiles, c);
       if (P.groups == 1 || c % 8 != 0) c = ceil_div(P.ntiles, P.tpc);
     }
     P.chunks = c;
     P.xcd_pair = (P.groups > 1 && c % 8 == 0) ? 1 : 0;
     P.nlists = c * rs;
-    P.cap = std::max<int64_t>(128, pow2_at_least(k + 64));
+    P.cap = list_cap(k);
     // Sampling pre-pass: about 1/16 of the tiles, and at least 8k/upt of them
     // but at most a quarter (its threshold is the k-th best of ~upt*s unit
     // maxima, so the expected number of candidates that pass it is about
@@ -657,7 +677,8 @@ hipError_t launch_scores(const _Float16* q, const _Float16* x, int64_t nq, int64
 // or GEMV, 3 final select; skipped stages get back-to-back marks.
 int run_fused(const void* q, const void* x, int64_t nq, int64_t n, int64_t d, int64_t k, int64_t bq,
               int64_t chunks, int flags, void* workspace, int64_t workspace_bytes, float* out_v,
-              void* out_i, int64_t* plan_out, int device, void* stream, hipEvent_t* marks, bool allow_lean = true) {
+              void* out_i, int64_t* plan_out, int device, void* stream, hipEvent_t* marks,
+              const Plan* given = nullptr) {  // (made for these sizes, instead of the automatic one)
   DevInfo di;
   int rc = dev_info(device, &di);
   if (rc != CVS_OK) return rc;
@@ -665,7 +686,10 @@ int run_fused(const void* q, const void* x, int64_t nq, int64_t n, int64_t d, in
   rc = check_inputs(q, x, nq, n, d);
   if (rc != CVS_OK) return rc;
   Plan P;
-  rc = make_plan(nq, n, d, k, bq, chunks, flags, di.cus, &P, 16, true, allow_lean);
+  if (given)
+    P = *given;
+  else
+    rc = make_plan(nq, n, d, k, bq, chunks, flags, di.cus, &P);
   if (rc != CVS_OK) return rc;
   if (plan_out) {
     plan_out[0] = P.bq;
@@ -926,9 +950,16 @@ int cvs_fused_topk_noalloc(const void* q, const void* x, int64_t nq, int64_t n, 
   if (rc != CVS_OK) return rc;
   // the tiled-GEMM scan keeps more lists per query, the score-matrix search all
   // scores: where they do not fit, the query-stationary scan
-  const bool allow_lean = P.ws_bytes <= kScratchBytes;
-  if (!allow_lean) {
+  if (P.ws_bytes > kScratchBytes) {
     rc = make_plan(nq, n, d, k, 0, 0, flags, di.cus, &P, 16, true, false);
+    if (rc != CVS_OK) return rc;
+  }
+  // ... and where several rounds of its chunks, each with its lists, do not: one
+  // workgroup per CU, rounded up
+  if (P.ws_bytes > kScratchBytes && P.groups > 1) {
+    int64_t c = std::min<int64_t>(ceil_div(di.cus, P.groups), std::max<int64_t>(1, P.ntiles / 2));
+    if (c >= 8) c = align_up(c, 8);
+    rc = make_plan(nq, n, d, k, 0, c, flags, di.cus, &P, 16, true, false);
     if (rc != CVS_OK) return rc;
   }
   if (P.ws_bytes > kScratchBytes)
@@ -946,7 +977,7 @@ int cvs_fused_topk_noalloc(const void* q, const void* x, int64_t nq, int64_t n, 
   // The fused path needs no zeroed workspace (every list count and threshold is
   // written before it is read), so nothing is cleared here.
   return run_fused(q, x, nq, n, d, k, 0, 0, flags, ws, kScratchBytes, out_v, out_i, plan_out, device, stream,
-                   nullptr, allow_lean);
+                   nullptr, &P);
 }
 
 int cvs_fused_topk_marked(const void* q, const void* x, int64_t nq, int64_t n, int64_t d, int64_t k,
@@ -1233,7 +1264,7 @@ int make_q8_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int flags, int cus
     P.groups = ceil_div(std::max<int64_t>(nq, 1), P.bq);
     P.ntiles = ceil_div(n, P.cfg.tile_rows());
     const int64_t rs = P.cfg.rs();
-    const int64_t max_chunks = std::min<int64_t>({P.ntiles, 65535, kSelectMaxLists / rs});
+    const int64_t max_chunks = std::min<int64_t>({P.ntiles, 65535, kSelectMaxLists / rs, list_chunks(nq, rs, k)});
     const int64_t most = std::min<int64_t>(max_chunks, std::max<int64_t>(1, P.groups > 1 ? align_up(P.ntiles / 2, 8) : P.ntiles / 2));
     int64_t c = P.groups == 1 ? std::min<int64_t>(cus, most)  // (an int8 column's time is half an fp16 one's)
                               : best_chunks(P.groups, P.ntiles, cus, most, 0.5 * qstat_tile_cost(P.cfg, P.dq));
@@ -1270,7 +1301,7 @@ int make_q8_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int flags, int cus
     P.s8_nsample = P.sample.nsample;
     P.s8_units = P.sample.units;
   }
-  P.cap = std::max<int64_t>(128, pow2_at_least(k + 64));
+  P.cap = list_cap(k);
   if (P.groups * P.chunks > INT_MAX) return fail(CVS_ERR_INVALID, "too many queries");
   if (!P.gemv) {
     const ScanCfg c384{32, 8, 1, 2, 12};

@@ -81,7 +81,9 @@ int cvs_scores(const void* q, const void* x, int64_t nq, int64_t n, int64_t d, v
  * Plan of cvs_fused_topk for these sizes, without running it.
  * plan_out[0] = query-block size (the reference's bq; 1 for the batch-1 GEMV
  * path), plan_out[1] = corpus chunks (lists per query for the GEMV path);
- * *workspace_bytes = device scratch the call needs.  Replaces the plan
+ * *workspace_bytes = device scratch the call needs: up to 512 MB of candidate
+ * lists (more where one list per query of the batch takes more), or at most
+ * 256 MB of scores for small corpora, and some KB per query.  Replaces the plan
  * heuristic of kernels.cu:499-536.  bq = 0 / chunks = 0 mean "auto"; a forced
  * bq must be 16, 32, 64, 128 or 256 and, as in the reference, satisfy
  * bq * slots(k) <= 256 with slots(k) = 1/2/4/8 for k <= 32/64/128/256; a forced
@@ -139,8 +141,10 @@ int cvs_fused_topk_marked(const void* q, const void* x, int64_t nq, int64_t n, i
  * arguments, results and errors as cvs_fused_topk with bq = chunks = 0 (the
  * auto plan), but the workspace is a library-owned device array of
  * CVS_NOALLOC_SCRATCH_BYTES per GPU (set up on the first call on a device,
- * held until the process ends); calls whose plan needs more (cvs_fused_plan's
- * workspace_bytes) fail with CVS_ERR_INVALID.  It calls no hipMalloc/hipFree.
+ * held until the process ends).  Where the automatic plan (cvs_fused_plan's
+ * workspace_bytes) needs more, the query-stationary scan is planned, at last
+ * with one workgroup per CU; calls that need more even so fail with
+ * CVS_ERR_INVALID.  It calls no hipMalloc/hipFree.
  * Every call on one GPU shares that array: calls that overlap in time on one
  * GPU (other streams, other threads) race and must be serialised by the caller.
  * Covers the headline shapes (1M x 384, batch 256, k 10: 67.1 MB).

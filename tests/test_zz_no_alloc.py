@@ -62,3 +62,31 @@ def test_noalloc_refuses_a_plan_larger_than_its_scratch(eng):
     assert ws > _ext.NOALLOC_SCRATCH_BYTES
     rc, _, _, _ = noalloc(eng, q, x, 100)
     assert rc == 1 and b"allocation-free" in eng.lib.cvs_last_error()
+
+
+@pytest.mark.parametrize("nq,n,d,k", [(20000, 20000, 384, 10), (640, 1_000_000, 384, 1), (1300, 50_000, 64, 100)])
+def test_noalloc_takes_fewer_chunks_where_the_automatic_plan_does_not_fit(eng, nq, n, d, k):
+    """Large batches whose candidate lists fit with one workgroup per CU."""
+    print(f"noalloc n={n} d={d} b={nq} k={k}", flush=True)
+    x = synthetic.unit_corpus(n, d, seed=11, device="cuda")
+    q = synthetic.unit_queries(nq, d, seed=12, device="cuda")
+    rc, v, i, plan = noalloc(eng, q, x, k)
+    assert rc == 0, eng.lib.cvs_last_error()
+    vf, i_f, _ = eng.fused_topk(q, x, k)
+    torch.cuda.synchronize()
+    torch.testing.assert_close(v, vf, rtol=0, atol=2 * d * 2.0**-24)  # fp32 sums in two orders
+    assert (i != i_f).float().mean().item() < 0.001
+
+
+@pytest.mark.parametrize("nq,n,d,k,chunks", [(100_000, 1_000_000, 768, 256, 1), (20_000, 1_000_000, 768, 256, 6),
+                                             (700, 2_000_000, 1024, 256, 88), (128, 1_000_000, 1024, 256, 512),
+                                             (3000, 4_000_000, 384, 200, 64), (4000, 300_000, 2048, 100, 256)])
+def test_candidate_lists_are_bounded(eng, nq, n, d, k, chunks):
+    """512 MB of (query, chunk) lists at most, or one chunk's; the sampling maxima
+    (2048 a query) and list counts come on top."""
+    plan, ws = eng.plan(nq, n, d, k)
+    assert plan[1] <= chunks
+    one = nq * 8 * (128 if k <= 64 else 256 if k <= 192 else 512)
+    assert ws <= max(512 << 20, one) + nq * 4 * (2048 + 2 * plan[1] + 1) + (1 << 16)
+    _, ws = eng.q8_plan(nq, n, min(d, 1536), k)
+    assert ws <= max(512 << 20, one) + nq * (8 * 4096 + 4 * 512 + 2 * 1536 + 64) + (1 << 17)
