@@ -242,15 +242,35 @@ double gemm_tile_cost(const ScanCfg& c, int64_t d, int64_t groups, bool alone) {
   return stream && !alone ? 2.9 * (double)d : 2 * blocks * 1.15 * (double)d * (alone ? 0.85 : 1.0);
 }
 
+// Chunks of a search's scan in an automatic plan, and the time of that scan as
+// scan_cost has it.
+struct ScanPlan {
+  int64_t chunks = 0;
+  double cost = 0;
+};
+
+ScanPlan plan_scan(const ScanCfg& c, int64_t nq, int64_t n, int64_t d, int64_t k, int cus) {
+  const int64_t groups = ceil_div(std::max<int64_t>(nq, 1), c.bq()), ntiles = ceil_div(n, c.tile_rows());
+  // (a chunk's groups share an XCD in multiples of 8, the last ones perhaps empty)
+  const int64_t max_chunks = std::min<int64_t>({groups > 1 ? align_up(ntiles, 8) : ntiles, 65535, kSelectMaxLists / c.rs(),
+                                                list_chunks(nq, c.rs(), k)});
+  const int64_t slots = cus * (c.gemm() ? gemm_per_cu(c) : 1);
+  const double tile = c.gemm() ? gemm_tile_cost(c, d, groups, groups * ntiles <= cus) : qstat_tile_cost(c, d);
+  // (the query-stationary scan's workgroups take at least two tiles)
+  const int64_t most = c.gemm() ? max_chunks
+                                : std::min<int64_t>(max_chunks, std::max<int64_t>(1, groups > 1 ? align_up(ntiles / 2, 8) : ntiles / 2));
+  ScanPlan p;
+  p.chunks = best_chunks(groups, ntiles, slots, most, tile, true);
+  p.cost = scan_cost(groups, ntiles, p.chunks, slots, tile);
+  return p;
+}
+
 // The tiled-GEMM scan for an automatic plan (false: the query-stationary scan).
 // Never up to 32 queries (both are bound by the corpus stream, within 5% of
 // each other), nor where the query-stationary scan has a kernel of exactly this
 // width with enough queries per wave: 384 and 768 (1000 x 384 over 100k rows:
 // 142 us against 167-173; 256 x 768, k = 100, over 200k: 146 against 175), and up
-// to 64 queries 1536 (64 over 100k: 82 against 90-97).  Otherwise the kernel
-// whose rounds end soonest: the query-stationary scan's tiles take longer but
-// are as small as 64 x 32, which fill the GPU on small corpora (156 x 1536 over
-// 7730 rows: 45 us against 53-71).
+// to 64 queries 1536 (64 over 100k: 82 against 90-97).
 // Whole searches, query-stationary -> tiled (us): 794 x 1664 over 276k rows
 // 2455 -> 960, 645 x 1536 over 32k 246 -> 139, 300 x 2048 over 50k 292 -> 130,
 // 100 x 1024 over 600k 433 -> 277, 1000 x 128 over 1M 573 -> 386, 231 x 256 over 1M
@@ -268,22 +288,18 @@ bool gemm_cfg(int64_t nq, int64_t n, int64_t d, int64_t k, int cus, const ScanCf
   // scan a little better (100 x 512, k = 100, over 1M rows: 269 us
   // against 287; over 100k rows 56 against 49)
   if (nq > 64 && nq <= 128 && d > 384 && d < 768 && n >= (1 << 19)) return false;
-  const int64_t qgroups = ceil_div(nq, qstat.bq()), qtiles = ceil_div(n, qstat.tile_rows());
-  const int64_t qchunks = std::max<int64_t>(1, std::min<int64_t>(ceil_div(cus, qgroups), qtiles / 2));
-  double cost = scan_cost(qgroups, qtiles, qchunks, cus, qstat_tile_cost(qstat, d));
+  // Several query groups: always (over 267 random sizes of 65 to 2500 queries and
+  // 1500 to 120000 rows 0.70 of the query-stationary scan's time, 1.05 at worst).  One: the model
+  // decides, within its error of 15%.
+  double limit = nq > qstat.bq() ? HUGE_VAL : 0.85 * plan_scan(qstat, nq, n, d, k, cus).cost;
   const ScanCfg small[1] = {{32, 2, 1, d < 1024 ? 2 : 4, -1}};
   const ScanCfg large[3] = {{32, 2, 4, 4, -1}, {32, 2, 2, 4, -1}, {32, 2, 2, 2, -1}};
-  const ScanCfg* cfgs = nq <= 64 ? small : large;
   bool found = false;
   for (int i = 0; i < (nq <= 64 ? 1 : 3); ++i) {
-    const ScanCfg& c = cfgs[i];
-    const int64_t groups = ceil_div(nq, c.bq()), ntiles = ceil_div(n, c.tile_rows());
-    const int64_t slots = cus * gemm_per_cu(c);
-    const double tile = gemm_tile_cost(c, d, groups, groups * ntiles <= cus);
-    const int64_t max_chunks = std::min<int64_t>(kSelectMaxLists / 2, list_chunks(nq, 2, k));
-    const double t = scan_cost(groups, ntiles, best_chunks(groups, ntiles, slots, max_chunks, tile, true), slots, tile);
-    if (t < (found ? cost : 0.85 * cost)) {  // (15%: the model's error)
-      cost = t;
+    const ScanCfg& c = nq <= 64 ? small[i] : large[i];
+    const double t = plan_scan(c, nq, n, d, k, cus).cost;
+    if (t < limit) {
+      limit = t;
       *out = c;
       found = true;
     }
@@ -306,10 +322,14 @@ bool gemm_cfg(int64_t nq, int64_t n, int64_t d, int64_t k, int cus, const ScanCf
 // as often; 84 x 640 over 32000 33 / 36; from 1024 up to 10M scores: 300 over 24000 94 / 67,
 // over 32000 92 / 80, 600 over 24000 76 / 89; k = 1 104 x 1280 over 32500 42 / 49).
 // (Width 1536 has query-stationary kernels for both; not measured.)
+// sampled: the plan's scan samples; qstat_sampled: the query-stationary scan, with
+// half the units a row, would too (where only the tiled one does: 208 x 1972
+// lists / matrix 31 / 19, 392 x 21173 79 / 57, but 1083 x 5449 0.89 of the matrix's
+// time and past it less).
 constexpr int64_t kDirectBytes = 256ll << 20;  // of scores (the MALL holds them)
-bool direct_search(int64_t nq, int64_t n, int64_t d, int64_t k, bool sampled) {
+bool direct_search(int64_t nq, int64_t n, int64_t d, int64_t k, bool sampled, bool qstat_sampled) {
   if (n > kRowDirect || nq * n * 4 > kDirectBytes) return false;
-  if (!sampled) return true;
+  if (!sampled || (!qstat_sampled && nq * n <= 4500000)) return true;
   if (nq > 32 && k >= 4 && d >= 512 && d != 1536 &&
       (d >= 1024 ? nq * n <= 10000000
                  : n > (d < 768 ? 16384 : 0) && n <= 24576 && nq <= 256 && nq * n <= 5000000))
@@ -317,6 +337,20 @@ bool direct_search(int64_t nq, int64_t n, int64_t d, int64_t k, bool sampled) {
   if (k >= 32) return nq <= 16 || (n <= 16384 && nq * n <= 8000000);
   if (nq == 1) return n <= 16384 || d >= 768;
   return d >= 768 ? n <= 16384 && nq * n <= 3300000 : n <= 8192 && nq * n <= 1700000;
+}
+
+// Tiles of the sampling pre-pass of a scan in configuration c: about
+// 1/sample_div of them, and at least 8k/units-per-tile (the tiled scan 4) but at
+// most a quarter (its threshold is the k-th best of the unit maxima, so the
+// expected number of candidates that pass it is about k * ntiles / tiles); 0
+// where that leaves too few units.
+int64_t sample_tiles(const ScanCfg& c, int64_t n, int64_t k, int flags, int64_t sample_div) {
+  if (flags & CVS_FLAG_NO_PREPASS) return 0;
+  const bool force = flags & CVS_FLAG_FORCE_PREPASS;
+  const int64_t ntiles = ceil_div(n, c.tile_rows()), upt = c.units_per_tile();
+  int64_t s = std::min<int64_t>(16384 / sample_div, std::max<int64_t>({ntiles / sample_div, ceil_div(8 * k, upt), c.gemm() ? 4 : 0}));
+  s = std::min<int64_t>(s, force ? ntiles : ntiles / 4);
+  return (force && s >= 1) || (s >= 4 && s * upt >= 2 * k) ? s : 0;
 }
 
 struct Plan {
@@ -366,6 +400,7 @@ int make_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int64_t bq, int64_t c
     if (bq * slots_per_lane(k) > 256) return fail(CVS_ERR_INVALID, "bq * ceil(k/32) must be <= 256");
   }
   Plan P;
+  bool qstat_sampled = true;
   P.gemv = (nq == 1 && !forced_bq && !(flags & CVS_FLAG_NO_GEMV));
   if (P.gemv) {
     int64_t waves = chunks > 0 ? chunks : (int64_t)cus * 16;
@@ -395,6 +430,7 @@ int make_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int64_t bq, int64_t c
       while (!cfg_for(bq, d, &tmp)) bq >>= 1;
     }
     if (!cfg_for(bq, d, &P.cfg)) return fail(CVS_ERR_INVALID, "bq=%lld is not supported at width %lld", (long long)bq, (long long)d);
+    qstat_sampled = sample_tiles(P.cfg, n, k, flags, sample_div) > 0;
     if (ScanCfg g; allow_lean && !forced_bq && gemm_cfg(nq, n, d, k, cus, P.cfg, &g)) {
       P.cfg = g;
       bq = g.bq();
@@ -404,22 +440,13 @@ int make_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int64_t bq, int64_t c
     P.tile_rows = P.cfg.tile_rows();
     P.ntiles = ceil_div(n, P.tile_rows);
     const int64_t rs = P.cfg.rs();
-    int64_t max_chunks = std::min<int64_t>({P.ntiles, 65535, kSelectMaxLists / rs});
-    if (chunks == 0) max_chunks = std::min(max_chunks, list_chunks(nq, rs, k));
     int64_t c;
     if (chunks > 0) {
-      c = std::max<int64_t>(1, std::min<int64_t>(chunks, max_chunks));
+      c = std::max<int64_t>(1, std::min<int64_t>({chunks, P.ntiles, 65535, kSelectMaxLists / rs}));
       P.tpc = ceil_div(P.ntiles, c);
       c = ceil_div(P.ntiles, P.tpc);
-    } else if (P.cfg.gemm()) {
-      c = best_chunks(P.groups, P.ntiles, cus * gemm_per_cu(P.cfg), max_chunks,
-                      gemm_tile_cost(P.cfg, d, P.groups, P.groups * P.ntiles <= cus), true);
-      P.tpc = ceil_div(P.ntiles, c);
-      if (P.groups == 1 || c % 8 != 0) c = ceil_div(P.ntiles, P.tpc);
     } else {
-      const int64_t most = std::min<int64_t>(max_chunks, std::max<int64_t>(1, P.groups > 1 ? align_up(P.ntiles / 2, 8) : P.ntiles / 2));
-      c = P.groups == 1 ? std::min<int64_t>(cus, most)
-                        : best_chunks(P.groups, P.ntiles, cus, most, qstat_tile_cost(P.cfg, d), true);
+      c = plan_scan(P.cfg, nq, n, d, k, cus).chunks;
       P.tpc = ceil_div(P.ntiles, c);
       if (P.groups == 1 || c % 8 != 0) c = ceil_div(P.ntiles, P.tpc);
     }
@@ -427,23 +454,16 @@ int make_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int64_t bq, int64_t c
     P.xcd_pair = (P.groups > 1 && c % 8 == 0) ? 1 : 0;
     P.nlists = c * rs;
     P.cap = list_cap(k);
-    // Sampling pre-pass: about 1/16 of the tiles, and at least 8k/upt of them
-    // but at most a quarter (its threshold is the k-th best of ~upt*s unit
-    // maxima, so the expected number of candidates that pass it is about
-    // k * ntiles / s), run by at most one workgroup per CU, each on spt
-    // consecutive tiles.
-    // (The tiled-GEMM scan samples in its smallest tiles: more workgroups for the
-    // same sample; 645 x 1536 over 32k rows: sampling 42 -> 19 us.)
+    // Sampling pre-pass, run by at most one workgroup per CU, each on spt
+    // consecutive tiles.  (The tiled-GEMM scan samples in its smallest tiles: more
+    // workgroups for the same sample; 645 x 1536 over 32k rows: sampling 42 -> 19 us.)
     P.scfg = P.cfg;
     if (P.cfg.gemm()) P.scfg = {32, 2, nq > 64 ? 2 : 1, 2, -1};
     P.s_groups = ceil_div(std::max<int64_t>(nq, 1), P.scfg.bq());
     P.s_ntiles = ceil_div(n, P.scfg.tile_rows());
     const int64_t upt = P.scfg.units_per_tile();  // sampling units per tile
-    int64_t s = std::min<int64_t>(16384 / sample_div, std::max<int64_t>({P.s_ntiles / sample_div, ceil_div(8 * k, upt),
-                                                                         P.scfg.gemm() ? 4 : 0}));
-    s = std::min<int64_t>(s, (flags & CVS_FLAG_FORCE_PREPASS) ? P.s_ntiles : P.s_ntiles / 4);
-    P.prepass = !(flags & CVS_FLAG_NO_PREPASS) &&
-                (((flags & CVS_FLAG_FORCE_PREPASS) && s >= 1) || (s >= 4 && s * upt >= 2 * k));
+    const int64_t s = sample_tiles(P.scfg, n, k, flags, sample_div);
+    P.prepass = s > 0;
     if (P.prepass) {
       const int64_t s_slots = cus * (P.scfg.gemm() ? gemm_per_cu(P.scfg) : 1);
       const int64_t wgs = std::max<int64_t>(1, std::min<int64_t>(s, s_slots / P.s_groups));
@@ -512,7 +532,7 @@ int make_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int64_t bq, int64_t c
   }
   if (P.cap > kMaxCap) return fail(CVS_ERR_INVALID, "internal: list capacity %lld too large", (long long)P.cap);
   if (allow_lean && !forced_bq && chunks == 0 && (flags & ~CVS_FLAG_IDS_INT64) == 0 &&
-      direct_search(nq, n, d, k, P.prepass)) {
+      direct_search(nq, n, d, k, P.prepass, qstat_sampled)) {
     P.direct = true;
     P.sin = P.prepass = P.tau_in_scan = false;
     P.ws_bytes = align_up(std::max<int64_t>(nq, 1) * n * 4, 256);

@@ -257,6 +257,21 @@ def test_tiled_scan_cuts_full_lists(eng, nq, n, d, k):
     oracle.check_exact(q, x, k, v.cpu().numpy(), i.cpu().numpy())
 
 
+@pytest.mark.parametrize("nq,n,d,k,bq,chunks", [
+    (176, 29864, 448, 2, 128, 240), (256, 27757, 704, 1, 128, 224),  # 234, 217 tiles: one per workgroup, the last chunks
+    (480, 21729, 448, 12, 256, 88), (2002, 7654, 512, 11, 256, 32),  # empty; 85, 30 tiles of 256 rows
+    (192, 18339, 832, 2, 128, 144), (112, 16857, 832, 1, 128, 132)])  # several groups: no longer the 64-query scan
+def test_tiles_are_chosen_by_the_plan_that_runs(eng, nq, n, d, k, bq, chunks):
+    """The costs compared are those of the chunk counts that are then run."""
+    say(f"tile choice nq={nq} n={n} d={d} k={k}")
+    plan, _ = eng.plan(nq, n, d, k)
+    assert plan == [bq, chunks]
+    x, q = make(n, d, nq, seed=nq)
+    v, i, _ = eng.fused_topk(q.cuda(), x.cuda(), k)
+    torch.cuda.synchronize()
+    oracle.check_exact(q, x, k, v.cpu().numpy(), i.cpu().numpy())
+
+
 def test_noalloc_keeps_what_its_scratch_held(eng):
     """The allocation-free search of sizes whose tiled plan outgrows its scratch
     runs the query-stationary plan, as it did."""
