@@ -1035,8 +1035,8 @@ int cvs_scores(const void* q, const void* x, int64_t nq, int64_t n, int64_t d, v
 namespace {
 
 // Plan of cvs_topk_rows (see cvs_rowtopk.hip); rows of at most kRowDirect columns
-// need no workspace.  At most kRowBatch rows run in one set of launches, so
-// the candidate arrays stay within 64 MB whatever the batch.
+// need no workspace.  Of longer ones at most kRowBatch run in one set of
+// launches, so the candidate arrays stay within 64 MB whatever the batch.
 constexpr int64_t kRowBatch = 1024;
 
 struct RowPlan {
@@ -1047,8 +1047,9 @@ struct RowPlan {
 
 RowPlan row_plan(int64_t nq, int64_t n, int64_t k, int cus) {
   RowPlan P;
-  P.rows = std::max<int64_t>(1, std::min<int64_t>(nq, kRowBatch));
+  P.rows = std::max<int64_t>(1, nq);
   if (n <= kRowDirect) return P;
+  P.rows = std::min<int64_t>(P.rows, kRowBatch);
   // The sample: a 32nd of the row, at least 16384 scores (a quarter of a short
   // row), so that about 8 or more of the row's k best are in it for k = 256
   // (30 at k = 1000 over 1M columns); the threshold is the score `rank` from

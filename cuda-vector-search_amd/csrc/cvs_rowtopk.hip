@@ -440,8 +440,14 @@ __global__ __launch_bounds__(kFinal) void row_final_kernel(RowTopkArgs a) {
 hipError_t launch_row_topk(const RowTopkArgs& a, int rows, hipStream_t s) {
   if (a.k < 1 || a.k > kRowTopkMaxK || a.n < a.k || rows < 1 || a.scores == nullptr) return hipErrorInvalidValue;
   if (a.n <= kRowDirect) {
-    hipLaunchKernelGGL(row_final_kernel<true>, dim3(rows), dim3(kFinal), 0, s, a);
-    return hipGetLastError();
+    constexpr int64_t kMost = 1 << 21;  // workgroups of a launch: fewer than 2^32 threads
+    for (int64_t r = 0; r < rows; r += kMost) {
+      RowTopkArgs b = a;
+      b.row0 = a.row0 + r;
+      hipLaunchKernelGGL(row_final_kernel<true>, dim3((unsigned)(rows - r < kMost ? rows - r : kMost)), dim3(kFinal), 0, s, b);
+      if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    }
+    return hipSuccess;
   }
   if (a.tau == nullptr || a.count == nullptr || a.cand == nullptr || a.groups < 1 || 32 * (int64_t)a.groups > a.n ||
       a.chunks < 1 || a.len < 1 || a.len * a.chunks < a.n || (int64_t)rows * a.chunks > 0x7fffffff)

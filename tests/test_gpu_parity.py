@@ -789,6 +789,23 @@ def test_search_in_one_call_equals_its_parts(eng, metric, d):
         eng.search(q.half(), index._x, 5, False)
 
 
+def test_small_corpus_search_of_millions_of_queries(eng):
+    """More queries than one launch of the whole-row top k has workgroups for."""
+    nq, n, d, k = 4_300_000, 8, 64, 4
+    say(f"millions of queries nq={nq} n={n}")
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(n, d, generator=g, device="cuda").half()
+    q = torch.randn(nq, d, generator=g, device="cuda").half()
+    v, i, _ = eng.fused_topk(q, x, k)
+    s = torch.cat([c.float() @ x.float().T for c in q.split(1 << 20)])
+    # |q||x| < 200 here: fp32 sums of 64 products are off by less than 64 2^-24 200 each
+    torch.testing.assert_close(v, torch.topk(s, k, dim=1).values, rtol=0, atol=2 * 64 * 2.0**-24 * 200)
+    torch.testing.assert_close(torch.gather(s, 1, i.long()), v, rtol=0, atol=2 * 64 * 2.0**-24 * 200)
+    w, j = eng.topk_rows(s, k)
+    torch.testing.assert_close(w, torch.topk(s, k, dim=1).values, rtol=0, atol=0)
+    assert bool((torch.gather(s, 1, j.long()) == w).all())
+
+
 # Query tiles with columns past the batch, of every filtering scan: the
 # query-stationary ones (16 to 256 queries a tile, thresholds from a launch, from
 # the scan itself and none), the tiled ones (64, 128 and 256 queries) and the int8
