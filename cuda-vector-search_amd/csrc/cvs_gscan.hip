@@ -564,12 +564,14 @@ template <int QB, int RB>
 hipError_t launch_g(int mode, const ScanArgs& a, int grid, hipStream_t s) {
   if (mode == kAppend)
     hipLaunchKernelGGL((gscan_kernel<QB, RB, kAppend>), dim3(grid), dim3(kBlock), 0, s, a);
-  else if (mode == kMax)
-    hipLaunchKernelGGL((gscan_kernel<QB, RB, kMax>), dim3(grid), dim3(kBlock), 0, s, a);
   else if (mode == kStoreF32)
     hipLaunchKernelGGL((gscan_kernel<QB, RB, kStoreF32>), dim3(grid), dim3(kBlock), 0, s, a);
-  else
+  else if (mode == kStoreF16)
     hipLaunchKernelGGL((gscan_kernel<QB, RB, kStoreF16>), dim3(grid), dim3(kBlock), 0, s, a);
+  else if constexpr (RB == 2)  // sampling: the smallest tiles of a batch only
+    hipLaunchKernelGGL((gscan_kernel<QB, RB, kMax>), dim3(grid), dim3(kBlock), 0, s, a);
+  else
+    return hipErrorInvalidValue;
   return hipGetLastError();
 }
 

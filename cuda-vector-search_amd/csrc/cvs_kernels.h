@@ -259,7 +259,8 @@ constexpr int64_t kGscanMaxWidth = 1 << 16;  // (32-bit byte offsets within a ti
 
 // Returns hipErrorInvalidValue when no kernel is instantiated for (cfg, mode).
 hipError_t launch_scan(const ScanCfg& cfg, int mode, const ScanArgs& a, int grid, hipStream_t s);
-// cfg.gemm(): modes kAppend, kMax, kStoreF32 and kStoreF16 of the configs of launch_gscan.
+// cfg.gemm(): modes kAppend, kStoreF32 and kStoreF16 of the configs of launch_gscan,
+// kMax of those with rb = 2 (sampling takes the smallest tiles).
 hipError_t launch_gscan(const ScanCfg& cfg, int mode, const ScanArgs& a, int grid, hipStream_t s);
 // Mode kTopK: instantiated for cfg {32, 1, 1, 1, 24} only (batches <= 32, width <= 384).
 bool scan_topk_available(const ScanCfg& cfg, int64_t d, int64_t k);

@@ -80,3 +80,19 @@ def test_built_lds_loads_wait_for_m0():
             pytest.skip("library not built in this tree")
         for insns, _ in mod.kernels(asm.read_text()).values():
             assert mod.early_lds_loads(insns) == []
+
+
+def test_tiled_scan_samples_in_its_smallest_tiles_only():
+    """The plans sample in tiles of 128 rows: no other sampling kernel is built."""
+    import re
+
+    import pytest
+
+    asm = PKG / "_build" / "cvs_gscan.s"
+    if not asm.exists():
+        pytest.skip("library not built in this tree")
+    built = set(re.findall(r"gscan_kernelILi(\d)ELi(\d)ELi(\d+)E", asm.read_text()))
+    assert len({m for _, _, m in built}) == 4 and len({(q, r) for q, r, _ in built}) == 5
+    per_mode = {m: {(q, r) for q, r, mm in built if mm == m} for _, _, m in built}
+    assert sorted(map(len, per_mode.values())) == [2, 5, 5, 5]
+    assert {"12", "22"} == {q + r for q, r in min(per_mode.values(), key=len)}
