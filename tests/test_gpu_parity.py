@@ -706,6 +706,10 @@ def test_topk_rows_with_infinite_scores(eng, nq, n, k):
     (2, 70001, 1000, "burst"),             # the sample sees every high score, too few reach it: streamed again
     (2, 300000, 1000, "block"),            # the best scores side by side in one filter workgroup
     (2, 40000, 300, "nan"),                # NaN above +inf, as the keys order them
+    (3, 8192, 1024, "outlier"), (3, 2500, 10, "outlier"), (2, 32768, 100, "outlier"), (2, 9000, 1, "outlier"),
+    (2, 70001, 1000, "outlier"),           # all others in one bin: cut again
+    (2, 8192, 40, "nested"), (2, 32768, 700, "nested"), (2, 32768, 3, "nested"),  # and again, more often than it is
+    (2, 32768, 300, "steps"),              # ties at the k-th place within the bin
 ])
 def test_topk_rows_threshold_edges(eng, nq, n, k, data):
     say(f"topk_rows nq={nq} n={n} k={k} {data}")
@@ -718,6 +722,15 @@ def test_topk_rows_threshold_edges(eng, nq, n, k, data):
         s[:, 60:60 + 136 * 500:136] += 9.0
     elif data == "block":
         s[:, 100000:103000] += 50.0
+    elif data == "outlier":
+        s[:, 11] = 3e4
+        s[0, 12] = -3e4
+        s[1, 13:15] = float("inf")
+    elif data == "nested":
+        s[:, 100:140] += 10.0 ** torch.arange(40, dtype=torch.float64).sub(4).float()
+    elif data == "steps":
+        s = torch.round(s * 8) / 8
+        s[:, 7] = 1e6
     elif data == "nan":
         s[0, 17::911] = float("nan")
         s[1, 5] = float("inf")
@@ -787,6 +800,35 @@ def test_search_in_one_call_equals_its_parts(eng, metric, d):
     assert eng.lib.cvs_search(*args[:6], 0, *args[7:]) != 0
     with pytest.raises(RuntimeError, match="same device"):  # refused before anything is launched
         eng.search(q.half(), index._x, 5, False)
+
+
+@pytest.mark.parametrize("nq,n,d,k", [(200, 16000, 768, 10), (100, 24000, 1024, 10), (40, 8000, 384, 10)])
+def test_one_long_row_does_not_slow_small_corpora(eng, nq, n, d, k):
+    """A row of 3000 times the others' norm: within twice the plain corpus's time (it
+    took 3.5 to 5 times while the whole-row top k had one level of bins)."""
+    say(f"one long row nq={nq} n={n} d={d}")
+    x, q = make(n, d, nq, seed=1)
+    y = x.clone()
+    y[n // 3] *= 3000
+
+    def best(c):
+        c, qd, out = c.cuda(), q.cuda(), []
+        for _ in range(8):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            torch.cuda.synchronize()
+            a.record()
+            for _ in range(20):
+                r = eng.fused_topk(qd, c, k)
+            b.record()
+            torch.cuda.synchronize()
+            out.append(a.elapsed_time(b))
+        return min(out), r
+
+    plain, _ = best(x)
+    slow, (v, i, _) = best(y)
+    assert slow < 2 * plain
+    s = q.double() @ y.double().T
+    torch.testing.assert_close(v.cpu().double(), torch.topk(s, k, dim=1).values, rtol=2 * d * 2.0**-24, atol=2 * d * 2.0**-24)
 
 
 def test_small_corpus_search_of_millions_of_queries(eng):
