@@ -257,6 +257,40 @@ def test_tiled_scan_cuts_full_lists(eng, nq, n, d, k):
     oracle.check_exact(q, x, k, v.cpu().numpy(), i.cpu().numpy())
 
 
+@pytest.mark.parametrize("nq,n,d,k,zeros,bq", [(64, 100000, 512, 10, 1, 64), (64, 100000, 512, 10, 8, 64),
+                                               (48, 60001, 1024, 100, 2, 16), (300, 60001, 192, 200, 3, 16),
+                                               (130, 40001, 640, 10, 40, 64)])
+def test_tiled_scan_of_queries_of_zeros(eng, nq, n, d, k, zeros, bq):
+    """Queries (padding) whose scores all tie: the smallest ids, the other queries'
+    results as without them, and no longer than the query-stationary scan."""
+    say(f"queries of zeros nq={nq} n={n} d={d} k={k} zeros={zeros}")
+    x, q = make(n, d, nq, seed=n + d)
+    q[:: nq // zeros][:zeros] = 0
+    empty = (q == 0).all(1)
+    xd, qd = x.cuda(), q.cuda()
+
+    def best(**kw):
+        out = []
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            torch.cuda.synchronize()
+            a.record()
+            for _ in range(3):
+                r = eng.fused_topk(qd, xd, k, **kw)
+            b.record()
+            torch.cuda.synchronize()
+            out.append(a.elapsed_time(b))
+        return min(out), r[0].cpu(), r[1].cpu()
+
+    tiled, v, i = best()
+    qstat, v2, i2 = best(bq=bq)
+    assert int(empty.sum()) == zeros
+    assert torch.equal(i[empty], torch.arange(k, dtype=i.dtype).expand(zeros, k)) and not v[empty].any()
+    oracle.check_exact(q[~empty], x, k, v[~empty].numpy(), i[~empty].numpy())
+    torch.testing.assert_close(v, v2, rtol=0, atol=2 * d * 2.0**-24)
+    assert tiled < 1.3 * qstat
+
+
 @pytest.mark.parametrize("nq,n,d,k,bq,chunks", [
     (176, 29864, 448, 2, 128, 240), (256, 27757, 704, 1, 128, 224),  # 234, 217 tiles: one per workgroup, the last chunks
     (480, 21729, 448, 12, 256, 88), (2002, 7654, 512, 11, 256, 32),  # empty; 85, 30 tiles of 256 rows
