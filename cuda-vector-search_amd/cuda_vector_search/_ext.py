@@ -232,13 +232,18 @@ class Engine:
         if not dst.is_contiguous():
             raise RuntimeError("prep_rows needs a contiguous destination")
 
+    @staticmethod
+    def _row_stride(src, dst) -> int:
+        """src's row stride; a single row's may be anything, and does not matter."""
+        return src.stride(0) if src.shape[0] > 1 else dst.shape[1]
+
     def prep_rows(self, src, dst, normalize: bool) -> None:
         """dst[:, :d] = src (L2-normalised when `normalize`), dst[:, d:] = 0, in one
         kernel.  src: [n, d] fp16 CUDA rows with unit column stride; dst: [n, w]
         contiguous fp16, w >= d; dst may be src itself (in place, w == d)."""
         self._check_prep(src, dst)
         n, d = src.shape
-        rc = self.lib.cvs_prep_rows(src.data_ptr(), dst.data_ptr(), n, d, src.stride(0), dst.shape[1],
+        rc = self.lib.cvs_prep_rows(src.data_ptr(), dst.data_ptr(), n, d, self._row_stride(src, dst), dst.shape[1],
                                     1 if normalize else 0, src.device.index, self._stream(src.device))
         if rc != 0:
             raise self._error(rc)
@@ -376,7 +381,7 @@ class Engine:
         self._check_matrix(dst, "corpus")
         n, d = src.shape
         xq = torch.empty(self.q8_corpus_bytes(n, dst.shape[1]), dtype=torch.uint8, device=dst.device)
-        rc = self.lib.cvs_q8_prep_build(src.data_ptr(), dst.data_ptr(), n, d, src.stride(0), dst.shape[1],
+        rc = self.lib.cvs_q8_prep_build(src.data_ptr(), dst.data_ptr(), n, d, self._row_stride(src, dst), dst.shape[1],
                                         1 if normalize else 0, xq.data_ptr(), xq.numel(), dst.device.index,
                                         self._stream(dst.device))
         if rc != 0:

@@ -620,6 +620,27 @@ def test_prep_rows_stores_the_same_bits(eng, n, d, width):
         assert np.array_equal(t.view(np.int16)[~nan], want.view(np.int16)[~nan])
 
 
+@pytest.mark.parametrize("d", [384, 100])
+@pytest.mark.parametrize("metric", ["ip", "cosine"])
+@pytest.mark.parametrize("copy", [True, False])
+def test_index_of_one_row_of_any_stride(eng, d, metric, copy):
+    """A [1, d] tensor is contiguous whatever its row stride (a transposed column has
+    1, a slice of wider rows theirs)."""
+    say(f"one row d={d} {metric} copy={copy}")
+    g = torch.Generator().manual_seed(d)
+    col = torch.randn(d, 1, generator=g).half()
+    wide = torch.zeros(3, d + 9, dtype=torch.float16)
+    wide[0, :d] = col[:, 0]
+    want = fp32_normalized(col.t().numpy()) if metric == "cosine" else col.t().numpy()
+    for row in (col.cuda().t(), wide.cuda()[:1, :d]):
+        assert row.is_contiguous() and row.stride(0) != d
+        for int8 in (False, True):
+            index = Index(row.clone(memory_format=torch.preserve_format), metric=metric, copy=copy, int8_prefilter=int8)
+            assert np.array_equal(index.embeddings.cpu().numpy().view(np.int16), want.view(np.int16))
+            v, i = index.search(col[:, 0].cuda(), 1)
+            assert i.tolist() == [[0]]
+
+
 def test_prep_rows_errors(eng):
     x = torch.zeros(4, 64, dtype=torch.float16, device="cuda")
     with pytest.raises(RuntimeError, match="destination width"):
