@@ -540,17 +540,18 @@ __global__ __launch_bounds__(kBlock, QB * RB > 4 ? 1 : 2) void gscan_kernel(Scan
   if constexpr (APP) {
     if (st_n > 0) flush();
     // The lists of a few queries that stayed half full (scores that tie by the
-    // thousand, as a query of zeros has) are cut to their k best: the select reads
-    // all lists of a query in one workgroup (64 x 512 over 100k rows with one query of zeros:
-    // 398 us, 252 with the query-stationary scan's fewer lists, so 131).  Where
-    // most queries have such lists, their selects run side by side (rows stored by ascending score:
-    // 53 us, with every list cut 127).
+    // thousand, as a query of zeros has) are cut to their k best where that takes
+    // most of them away: the select reads all lists of a query in one workgroup
+    // (64 x 512 over 100k rows, k = 10, with one query of zeros: 398 us, 252 with the
+    // query-stationary scan's fewer lists, so 131; with 8 405, 312 and 225).  Where
+    // most queries have such lists their selects run side by side, and the cuts
+    // would not (rows stored by ascending score 53 us, every list cut 127).
 #pragma unroll 1
     for (int i = 0; i < 32 * QB; i += kWave) {
       const int ql = wq * QB * 32 + i + lane;
       const int c = i + lane < 32 * QB ? lcnt[wr][ql] : 0;
-      uint64_t om = __ballot(2 * c >= a.cap && c > a.k);
-      if (__popcll(om) > 16) om = 0;
+      uint64_t om = __ballot(2 * c >= a.cap && c >= 4 * a.k);
+      if (__popcll(om) > 8) om = 0;
 #pragma unroll 1
       while (om) {
         const int l = __ffsll((unsigned long long)om) - 1;
