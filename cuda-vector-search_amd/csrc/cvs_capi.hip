@@ -592,6 +592,24 @@ int cvs_fused_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int64_t bq, int6
   return CVS_OK;
 }
 
+int cvs_fused_path(int64_t nq, int64_t n, int64_t d, int64_t k, int64_t bq, int64_t chunks, int flags,
+                   int device, int64_t* path_out) {
+  DevInfo di;
+  int rc = dev_info(device, &di);
+  if (rc != CVS_OK) return rc;
+  if (path_out == nullptr) return fail(CVS_ERR_INVALID, "path pointer must not be null");
+  if (d <= 0 || d % 64 != 0) return fail(CVS_ERR_INVALID, "width must be a multiple of 64 (zero-pad it)");
+  if (d >= INT_MAX / 2) return fail(CVS_ERR_INVALID, "width %lld is too large", (long long)d);
+  Plan P;
+  rc = make_plan(nq, n, d, k, bq, chunks, flags, di.cus, &P);
+  if (rc != CVS_OK) return rc;
+  path_out[0] = P.direct ? 3 : P.gemv ? 0 : P.cfg.gemm() ? 2 : 1;
+  const bool scan = !P.direct && !P.gemv;
+  path_out[1] = scan ? P.cfg.bq() : 0;
+  path_out[2] = scan ? P.cfg.tile_rows() : 0;
+  return CVS_OK;
+}
+
 }  // extern "C"
 
 namespace {

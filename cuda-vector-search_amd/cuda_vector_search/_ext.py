@@ -127,6 +127,8 @@ def _bind(lib: ctypes.CDLL) -> ctypes.CDLL:
     lib.cvs_fused_plan.restype = i32
     lib.cvs_fused_plan.argtypes = [i64, i64, i64, i64, i64, i64, i32, i32,
                                    ctypes.POINTER(i64), ctypes.POINTER(i64)]
+    lib.cvs_fused_path.restype = i32
+    lib.cvs_fused_path.argtypes = [i64, i64, i64, i64, i64, i64, i32, i32, ctypes.POINTER(i64)]
     lib.cvs_fused_topk.restype = i32
     lib.cvs_fused_topk.argtypes = [vp, vp, i64, i64, i64, i64, i64, i64, i32, vp, i64,
                                    vp, vp, ctypes.POINTER(i64), i32, vp]
@@ -296,6 +298,15 @@ class Engine:
         if rc != 0:
             raise self._error(rc)
         return [int(plan[0]), int(plan[1])], int(ws.value)
+
+    def search_path(self, nq: int, n: int, d: int, k: int, bq: int = 0, chunks: int = 0, flags: int = 0, device: int = 0):
+        """Which kernels a search of these sizes runs: ("gemv", "scan", "tiled" or
+        "matrix", queries per tile, rows per tile; 0, 0 without a scan)."""
+        out = (ctypes.c_int64 * 3)()
+        rc = self.lib.cvs_fused_path(nq, n, d, k, bq, chunks, flags, device, out)
+        if rc != 0:
+            raise self._error(rc)
+        return ("gemv", "scan", "tiled", "matrix")[out[0]], int(out[1]), int(out[2])
 
     def fused_topk(self, q, x, k: int, bq: int = 0, chunks: int = 0, flags: int = 0):
         return self._fused(q, x, k, bq, chunks, flags, None)

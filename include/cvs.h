@@ -93,6 +93,16 @@ int cvs_fused_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int64_t bq, int6
                    int flags, int device, int64_t* plan_out, int64_t* workspace_bytes);
 
 /*
+ * Which kernels cvs_fused_topk runs for these sizes (no counterpart in the
+ * reference; for tests and diagnostics), path_out[0]: 0 the batch-1 GEMV, 1 the
+ * query-stationary scan, 2 the tiled-GEMM scan, 3 the score matrix and the
+ * whole-row top-k (plan_out of cvs_fused_plan then holds the scan that it
+ * replaces).  path_out[1], [2]: queries and corpus rows of a scan's tile, 0 otherwise.
+ */
+int cvs_fused_path(int64_t nq, int64_t n, int64_t d, int64_t k, int64_t bq, int64_t chunks, int flags,
+                   int device, int64_t* path_out);
+
+/*
  * Exact top-k by inner product: for each query, the k rows with the largest
  * fp32-accumulated score, sorted by score descending and then row id
  * ascending.  out_v is [nq, k] fp32, out_i is [nq, k] int32 (int64 with

@@ -764,16 +764,21 @@ def test_topk_rows_threshold_edges(eng, nq, n, k, data):
     np.testing.assert_array_equal(v.cpu().numpy(), np.take_along_axis(s.numpy(), order, axis=1))
 
 
-@pytest.mark.parametrize("nq,n,d,k", [(1, 1, 64, 1), (1, 5003, 384, 5), (16, 8192, 768, 10), (17, 700, 384, 256),
-                                      (300, 8191, 128, 100), (5, 8193, 320, 3), (1, 8192, 1600, 256),
-                                      (9, 32768, 256, 40), (1, 16385, 768, 10), (100, 16000, 768, 200),
-                                      (33, 24577, 512, 10), (200, 24576, 768, 10), (300, 32768, 1024, 100),
-                                      (34, 32767, 2048, 1)])
-def test_small_corpus_search_is_exact(eng, nq, n, d, k):
-    """Corpora of few rows searched through a score matrix (and one that is
+@pytest.mark.parametrize("nq,n,d,k,path", [
+    (1, 1, 64, 1, "matrix"), (1, 5003, 384, 5, "matrix"), (16, 8192, 768, 10, "matrix"), (17, 700, 384, 256, "matrix"),
+    (300, 8191, 128, 100, "matrix"), (5, 8193, 320, 3, "scan"), (1, 8192, 1600, 256, "matrix"),
+    (9, 32768, 256, 40, "matrix"), (1, 16385, 768, 10, "matrix"), (100, 16000, 768, 200, "matrix"),
+    (33, 24577, 512, 10, "tiled"), (200, 24576, 768, 10, "matrix"), (300, 32768, 1024, 100, "matrix"),
+    (34, 32767, 2048, 1, "scan"), (33, 4097, 64, 1, "matrix"), (64, 20001, 128, 100, "tiled"),
+    (40, 9000, 1024, 10, "matrix"), (65, 30001, 256, 10, "tiled"), (513, 20000, 2048, 5, "tiled"),
+    (300, 20000, 128, 200, "matrix"), (200, 30000, 1024, 10, "matrix")])
+def test_small_corpus_search_is_exact(eng, nq, n, d, k, path):
+    """Corpora of few rows searched through a score matrix (and some that are
     not), against the lists (forced by a flag) and the oracle; exact
     ties; NaN scores are left out as the lists leave them out."""
     say(f"small corpus nq={nq} n={n} d={d} k={k}")
+    assert eng.search_path(nq, n, d, k)[0] == path
+    assert eng.search_path(nq, n, d, k, flags=_ext.FLAG_NO_PREPASS)[0] in ("gemv", "scan", "tiled")
     x, q = make(n, d, nq, seed=n + k)
     if n > 10:
         x[n // 2:n // 2 + 5] = x[1]

@@ -213,25 +213,28 @@ def test_wide_int8_is_refused_by_the_engine(eng):
         eng.q8_plan(4, 128, 2048, 10)
 
 
-# The tiled-GEMM scan (every auto plan past 32 queries at widths other than 384
-# and 768, once the corpus is large enough): each tile shape, widths of one
-# stage and up, partial tiles and query blocks, a chunk of one tile, several
+# The tiled-GEMM scan (auto plans past 32 queries at widths other than 384 and
+# 768, once the corpus is too large for the score matrix): each tile shape,
+# widths of one stage and up, partial tiles and query blocks, several
 # groups, ties and lists that fill.
-@pytest.mark.parametrize("nq,n,d,k", [
-    (33, 4097, 64, 1), (64, 20001, 128, 100), (40, 9000, 1024, 10),          # 64-query tiles, 128 and 256 rows
-    (65, 30001, 256, 10), (128, 70000, 1024, 64), (100, 33000, 1600, 256),   # 128-query tiles
-    (257, 40003, 192, 17), (600, 50000, 1088, 100), (513, 20000, 2048, 5),   # several groups
+@pytest.mark.parametrize("nq,n,d,k,tile", [
+    (33, 50001, 64, 1, (64, 128)), (64, 40001, 128, 100, (64, 128)), (60, 33001, 960, 10, (64, 128)),
+    (40, 90001, 1024, 10, (64, 256)), (64, 70003, 1600, 64, (64, 256)),
+    (257, 40003, 192, 17, (128, 128)), (600, 50000, 1088, 100, (128, 128)), (1000, 200001, 64, 10, (128, 128)),
+    (65, 50001, 256, 10, (128, 256)), (128, 70000, 1024, 64, (128, 256)), (100, 33000, 1600, 256, (128, 256)),
+    (300, 33001, 2048, 5, (128, 256)),
+    (200, 33000, 640, 256, (256, 256)), (512, 60000, 1088, 100, (256, 256)), (256, 50000, 1088, 3, (256, 256)),
 ])
-def test_tiled_scan_is_exact(eng, nq, n, d, k):
+def test_tiled_scan_is_exact(eng, nq, n, d, k, tile):
     say(f"tiled scan nq={nq} n={n} d={d} k={k}")
     x, q = make(n, d, nq, seed=n + d + k)
     x[n // 2:n // 2 + 40] = x[3]  # exact ties
     q[1] = x[3]
-    plan, _ = eng.plan(nq, n, d, k)
-    assert plan[0] in (64, 128, 256)
+    assert eng.search_path(nq, n, d, k) == ("tiled", *tile)
     xd, qd = x.cuda(), q.cuda()
     v, i, _ = eng.fused_topk(qd, xd, k)
-    forced = 16 if d > 768 or k > 128 else 32  # the query-stationary scan
+    forced = 16 if d > 768 or k > 128 else 32
+    assert eng.search_path(nq, n, d, k, bq=forced)[0] == "scan"  # the query-stationary scan
     v2, i2, p2 = eng.fused_topk(qd, xd, k, bq=forced)
     torch.cuda.synchronize()
     assert p2.tolist()[0] == forced
@@ -241,20 +244,33 @@ def test_tiled_scan_is_exact(eng, nq, n, d, k):
     assert (i != i2).float().mean().item() < 0.02
 
 
-@pytest.mark.parametrize("nq,n,d,k", [(200, 30000, 1024, 10), (300, 20000, 128, 200)])
-def test_tiled_scan_cuts_full_lists(eng, nq, n, d, k):
-    """Rows in ascending order of their scores fill every list many times over
+# Rows per list of 3 to 7 times its capacity (the last rows all pass), every tile
+# and lists of 128, 256 and 512 entries.
+@pytest.mark.parametrize("nq,n,d,k,tile", [(64, 400000, 64, 10, (64, 128)), (33, 300000, 1024, 10, (64, 256)),
+                                           (1000, 100000, 128, 100, (128, 128)), (300, 340000, 576, 200, (128, 128)),
+                                           (128, 200000, 1024, 10, (128, 256)), (256, 300000, 1024, 10, (256, 256))])
+def test_tiled_scan_cuts_full_lists(eng, nq, n, d, k, tile):
+    """Rows in ascending order of their scores fill every list several times over
     (no sampling), so that lists are cut to their k best as they go."""
     say(f"tiled scan, full lists nq={nq} n={n} d={d} k={k}")
-    g = torch.Generator().manual_seed(5)
-    base = torch.nn.functional.normalize(torch.randn(1, d, generator=g), dim=1)
-    x = (base * torch.linspace(0.1, 1.0, n)[:, None] + 0.001 * torch.randn(n, d, generator=g)).half()
-    q = (base + 0.01 * torch.randn(nq, d, generator=g)).half()
-    v, i, _ = eng.fused_topk(q.cuda(), x.cuda(), k, flags=_ext.FLAG_NO_PREPASS)
-    v2, i2, _ = eng.fused_topk(q.cuda(), x.cuda(), k)
+    flags = _ext.FLAG_NO_PREPASS
+    assert eng.search_path(nq, n, d, k) == eng.search_path(nq, n, d, k, flags=flags) == ("tiled", *tile)
+    plan, _ = eng.plan(nq, n, d, k, flags=flags)
+    cap = 128 if k <= 64 else 256 if k <= 192 else 512
+    assert n / (2 * plan[1]) > 1.9 * cap
+    g = torch.Generator(device="cuda").manual_seed(5)
+    base = torch.nn.functional.normalize(torch.randn(1, d, generator=g, device="cuda"), dim=1)
+    x = torch.empty(n, d, dtype=torch.float16, device="cuda")
+    for lo in range(0, n, 1 << 16):
+        r = torch.arange(lo, min(n, lo + (1 << 16)), device="cuda")
+        x[r] = (base * (0.1 + 0.9 * r[:, None] / n) + 0.001 * torch.randn(len(r), d, generator=g, device="cuda")).half()
+    q = (base + 0.01 * torch.randn(nq, d, generator=g, device="cuda")).half()
+    v, i, _ = eng.fused_topk(q, x, k, flags=flags)
+    v2, i2, _ = eng.fused_topk(q, x, k)
     torch.cuda.synchronize()
     assert torch.equal(v, v2) and torch.equal(i, i2)
-    oracle.check_exact(q, x, k, v.cpu().numpy(), i.cpu().numpy())
+    sel = torch.arange(0, nq, max(1, nq // 8))
+    oracle.check_exact(q[sel].cpu(), x.cpu(), k, v[sel].cpu().numpy(), i[sel].cpu().numpy())
 
 
 @pytest.mark.parametrize("nq,n,d,k,zeros,bq", [(64, 100000, 512, 10, 1, 64), (64, 100000, 512, 10, 8, 64),
@@ -267,6 +283,7 @@ def test_tiled_scan_of_queries_of_zeros(eng, nq, n, d, k, zeros, bq):
     x, q = make(n, d, nq, seed=n + d)
     q[:: nq // zeros][:zeros] = 0
     empty = (q == 0).all(1)
+    assert eng.search_path(nq, n, d, k)[0] == "tiled" and eng.search_path(nq, n, d, k, bq=bq)[0] == "scan"
     xd, qd = x.cuda(), q.cuda()
 
     def best(**kw):
@@ -299,7 +316,7 @@ def test_tiles_are_chosen_by_the_plan_that_runs(eng, nq, n, d, k, bq, chunks):
     """The costs compared are those of the chunk counts that are then run."""
     say(f"tile choice nq={nq} n={n} d={d} k={k}")
     plan, _ = eng.plan(nq, n, d, k)
-    assert plan == [bq, chunks]
+    assert plan == [bq, chunks] and eng.search_path(nq, n, d, k)[0] == "tiled"
     x, q = make(n, d, nq, seed=nq)
     v, i, _ = eng.fused_topk(q.cuda(), x.cuda(), k)
     torch.cuda.synchronize()
@@ -310,6 +327,7 @@ def test_noalloc_keeps_what_its_scratch_held(eng):
     """The allocation-free search of sizes whose tiled plan outgrows its scratch
     runs the query-stationary plan, as it did."""
     nq, n, d, k = 1000, 200000, 128, 10
+    assert eng.search_path(nq, n, d, k)[0] == "tiled"
     _, ws = eng.plan(nq, n, d, k)
     assert ws > _ext.NOALLOC_SCRATCH_BYTES
     x, q = make(n, d, nq, seed=9)
