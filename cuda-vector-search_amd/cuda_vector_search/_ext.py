@@ -462,10 +462,13 @@ class Engine:
         dev = x.device
         if q.device != dev or q.dtype != x.dtype:  # (Index(device="cuda") under another current device)
             raise RuntimeError("queries and corpus must be float16 on the same device")
+        if q.dim() != 2 or not q.is_contiguous():
+            raise RuntimeError("queries must be contiguous [nq, dim] rows")
         if x.shape[0] >= 2**31 - 1:
             raise RuntimeError("corpus must have fewer than 2^31 rows")
         nq, dim = q.shape
         n, d = x.shape
+        k = int(k)  # (a float or a 0-d tensor from the caller)
         index = dev.index
         key = (nq, n, d, dim, k, normalize, xq is None, index)
         ws_bytes = self._search_bytes.get(key)

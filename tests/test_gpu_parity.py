@@ -826,6 +826,12 @@ def test_search_in_one_call_equals_its_parts(eng, metric, d):
     assert eng.lib.cvs_search(*args[:6], 0, *args[7:]) != 0
     with pytest.raises(RuntimeError, match="same device"):  # refused before anything is launched
         eng.search(q.half(), index._x, 5, False)
+    with pytest.raises(RuntimeError, match="contiguous"):
+        eng.search(q.cuda()[:, :64], index._x, 5, False)
+    for k in (5.0, np.int64(5), torch.tensor(5)):  # whatever int() takes
+        for method in ("fused", "int8", "auto"):
+            w, j = index.search(q.cuda(), k, method=method)
+            assert w.shape == (7, 5) and torch.equal(j, i)
 
 
 @pytest.mark.parametrize("nq,n,d,k", [(200, 16000, 768, 10), (100, 24000, 1024, 10), (40, 8000, 384, 10)])
