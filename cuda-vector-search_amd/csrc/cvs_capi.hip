@@ -666,7 +666,12 @@ bool gemm_scores_cfg(int64_t nq, int64_t n, int64_t d, bool fp32, ScanCfg* cfg) 
 // The score matrix out [nq, n] (fp32 or fp16), chunked as the fused plan's scans.
 hipError_t launch_scores(const _Float16* q, const _Float16* x, int64_t nq, int64_t n, int64_t d, void* out, bool fp32,
                          int cus, hipStream_t s) {
-  if (nq == 1) {  // one query: the GEMV, 16 waves per CU of at least 16 rows
+  // One query: the GEMV, 16 waves per CU of at least 16 rows, for small corpora and
+  // past the MALL (5000 x 384 5.5 -> 4.5 us, 8000 x 2048 25 -> 10, 1M x 384 132 -> 118, 400k x
+  // 768 107 -> 94); between them the scan reads the MALL faster (117k x 1024 36, GEMV 45;
+  // 1M x 128 41, 47; 70k x 384 10.8, 11.6).
+  const int64_t corpus_bytes = 2 * n * d;
+  if (nq == 1 && (corpus_bytes <= (48 << 20) || corpus_bytes >= (512 << 20))) {
     const int64_t waves = std::max<int64_t>(1, std::min<int64_t>((int64_t)cus * 16, ceil_div(n, 16)));
     GemvArgs g{};
     g.q = q;

@@ -86,6 +86,35 @@ def test_tiled_scores_match_fp64(eng, nq, n, d):
         assert bool((buf[:guard] == 7).all()) and bool((buf[guard + nq * n:] == 7).all())
 
 
+@pytest.mark.parametrize("n,d", [(1, 64), (5003, 384), (32768, 768), (32769, 768), (117022, 1024), (300007, 1024)])
+def test_one_query_scores_match_fp64(eng, n, d):
+    """The GEMV below 48 MB of corpus and from 512 MB on, the scan between them."""
+    say(f"one-query scores n={n} d={d}")
+    g = torch.Generator(device="cuda").manual_seed(n + d)
+    x = torch.nn.functional.normalize(torch.randn(n, d, generator=g, device="cuda"), dim=1).half()
+    q = torch.nn.functional.normalize(torch.randn(2, d, generator=g, device="cuda"), dim=1).half()
+    ref = torch.cat([q[:1].double() @ r.double().T for r in x.split(1 << 16)], 1)
+    for fp32 in (True, False):
+        bound = 1.1 * d * 2.0**-24 + (0.0 if fp32 else 2.0**-11)
+        assert float((eng.scores(q[:1], x, fp32).double() - ref).abs().max()) <= bound
+
+    def best(rows):
+        out = []
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            torch.cuda.synchronize()
+            a.record()
+            for _ in range(20):
+                eng.scores(q[:rows], x)
+            b.record()
+            torch.cuda.synchronize()
+            out.append(a.elapsed_time(b))
+        return min(out)
+
+    if n > 100000:  # (a second query costs the scan nothing; the GEMV took 1.25 times its time out of the MALL)
+        assert best(1) < 1.15 * best(2)
+
+
 WIDE_FUSED = [
     (20000, 1600, 1, 10),     # batch-1 GEMV
     (20000, 2048, 16, 10),    # 16-query block (16x16x32 MFMA)
