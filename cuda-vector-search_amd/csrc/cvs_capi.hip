@@ -1072,19 +1072,20 @@ RowPlan row_plan(int64_t nq, int64_t n, int64_t k, int cus) {
   RowPlan P;
   P.rows = std::max<int64_t>(1, nq);
   if (n <= kRowDirect) return P;
-  P.rows = std::min<int64_t>(P.rows, kRowBatch);
-  // The sample: a 32nd of the row, at least 16384 scores (a quarter of a short
-  // row), so that about 8 or more of the row's k best are in it for k = 256
-  // (30 at k = 1000 over 1M columns); the threshold is the score `rank` from
-  // the top of the sample, 15% and five standard deviations (and 5) past where
-  // the k-th best is expected, so that fewer than k scores practically never
+  P.rows = ceil_div(P.rows, ceil_div(P.rows, kRowBatch));
+  // The sample: a 32nd of the row, at least 16384 scores (8192 in batches past one row a
+  // CU; a quarter of a short row), so that about 8 or more of the row's k best are
+  // in it for k = 256 (30 at k = 1000 over 1M columns); the threshold is the score
+  // `rank` from the top of the sample, 15% and five standard deviations (and 5)
+  // past where the k-th best is expected, so that fewer than k scores practically never
   // reach it and at most a few thousand do (kRowCap = 8192 fit).
-  P.groups = std::min<int64_t>(n / 128, std::max<int64_t>(512, n / 1024));
+  P.groups = std::min<int64_t>(n / 128, std::max<int64_t>(P.rows > cus ? 256 : 512, n / 1024));
   const double mu = (double)k * 32.0 * (double)P.groups / (double)n;
   P.rank = (int64_t)(1.15 * mu + 5.0 * std::sqrt(mu) + 5.0);
   // about 8 filter workgroups per CU, of 1 to 16 rounds of 4096 columns
   const int64_t want = ceil_div(P.rows * n, 8 * (int64_t)cus);
   P.len = std::max<int64_t>(4096, std::min<int64_t>(65536, align_up(want, 4096)));
+  P.len = align_up(ceil_div(n, ceil_div(n, P.len)), 4096);  // even chunks
   P.chunks = ceil_div(n, P.len);
   P.off_count = align_up(P.rows * 4, 256);
   P.off_cand = P.off_count + align_up(P.rows * 4, 256);
