@@ -274,7 +274,7 @@ ScanPlan plan_scan(const ScanCfg& c, int64_t nq, int64_t n, int64_t d, int64_t k
 // Whole searches, query-stationary -> tiled (us): 794 x 1664 over 276k rows
 // 2455 -> 960, 645 x 1536 over 32k 246 -> 139, 300 x 2048 over 50k 292 -> 130,
 // 100 x 1024 over 600k 433 -> 277, 1000 x 128 over 1M 573 -> 386, 231 x 256 over 1M
-// 256 -> 220, 48 x 1024 over 600k 302 -> 250, 64 x 256 over 300k 62 -> 50.
+// 256 -> 220, 64 x 256 over 300k 62 -> 50.
 // Up to 64 queries the corpus stream decides between the tiles: 128 rows, two
 // a CU, below d = 1024 (64 x 256: 50 us against 55 with 256 rows), 256
 // rows from there (48 x 1024: 250 against 257).
@@ -289,9 +289,21 @@ bool gemm_cfg(int64_t nq, int64_t n, int64_t d, int64_t k, int cus, const ScanCf
   // against 287; over 100k rows 56 against 49)
   if (nq > 64 && nq <= 128 && d > 384 && d < 768 && n >= (1 << 19)) return false;
   // Several query groups: always (over 267 random sizes of 65 to 2500 queries and
-  // 1500 to 120000 rows 0.70 of the query-stationary scan's time, 1.05 at worst).  One: the model
-  // decides, within its error of 15%.
-  double limit = nq > qstat.bq() ? HUGE_VAL : 0.85 * plan_scan(qstat, nq, n, d, k, cus).cost;
+  // 1500 to 120000 rows 0.70 of the query-stationary scan's time, 1.05 at worst).
+  // One: unless the corpus stream decides, which the query-stationary scan's finer
+  // tiles share out better.  Over 371 random sizes of up to 64 queries two were
+  // slower by more than 3% (by the costs alone 35), over 150 of up to 128 six (13).
+  double limit = HUGE_VAL;
+  if (nq <= qstat.bq()) {
+    if (d >= 1024) {  // the last round of its large tiles nearly empty (55 x 1408 over 136k rows 95 us, 126)
+      const int64_t tiles = ceil_div(n, 256), slots = 2 * (int64_t)cus;
+      if (tiles > slots && 10 * tiles < 9 * align_up(tiles, slots)) return false;
+    } else if (d >= 576) {  // past the MALL (62 x 896 over 799k 277, 307)
+      if (n * d > 150000000) return false;
+    } else if (nq > 64 && k >= 75 && d > 64 && d <= 192) {  // its lists cost the select (82 x 128, k = 80, over 197k 53, 60)
+      limit = 0.65 * plan_scan(qstat, nq, n, d, k, cus).cost;
+    }
+  }
   const ScanCfg small[1] = {{32, 2, 1, d < 1024 ? 2 : 4, -1}};
   const ScanCfg large[3] = {{32, 2, 4, 4, -1}, {32, 2, 2, 4, -1}, {32, 2, 2, 2, -1}};
   bool found = false;

@@ -275,7 +275,7 @@ def test_tiled_scan_is_exact(eng, nq, n, d, k, tile):
 
 # Rows per list of 3 to 7 times its capacity (the last rows all pass), every tile
 # and lists of 128, 256 and 512 entries.
-@pytest.mark.parametrize("nq,n,d,k,tile", [(64, 400000, 64, 10, (64, 128)), (33, 300000, 1024, 10, (64, 256)),
+@pytest.mark.parametrize("nq,n,d,k,tile", [(64, 400000, 64, 10, (64, 128)), (33, 260000, 1024, 10, (64, 256)),
                                            (1000, 100000, 128, 100, (128, 128)), (300, 340000, 576, 200, (128, 128)),
                                            (128, 200000, 1024, 10, (128, 256)), (256, 300000, 1024, 10, (256, 256))])
 def test_tiled_scan_cuts_full_lists(eng, nq, n, d, k, tile):
@@ -350,6 +350,14 @@ def test_tiles_are_chosen_by_the_plan_that_runs(eng, nq, n, d, k, bq, chunks):
     v, i, _ = eng.fused_topk(q.cuda(), x.cuda(), k)
     torch.cuda.synchronize()
     oracle.check_exact(q, x, k, v.cpu().numpy(), i.cpu().numpy())
+
+
+@pytest.mark.parametrize("nq,n,d,k,path", [
+    (55, 135823, 1408, 1, "scan"), (36, 218849, 2048, 5, "scan"), (62, 799357, 896, 3, "scan"),
+    (81, 485581, 576, 254, "scan"), (82, 197167, 128, 80, "scan"),  # 7 to 33% slower through the tiles
+    (46, 120242, 1792, 5, "tiled"), (64, 300000, 256, 10, "tiled"), (100, 600000, 1024, 50, "tiled")])
+def test_one_query_group_takes_the_tiles_where_they_are_faster(eng, nq, n, d, k, path):
+    assert eng.search_path(nq, n, d, k)[0] == path
 
 
 def test_noalloc_keeps_what_its_scratch_held(eng):
