@@ -705,9 +705,9 @@ hipError_t launch_scores(const _Float16* q, const _Float16* x, int64_t nq, int64
   const int64_t most = std::min<int64_t>(max_chunks, std::max<int64_t>(1, groups > 1 ? align_up(ntiles / 2, 8) : ntiles / 2));
   int64_t c;
   if (tiled)
-    c = best_chunks(groups, ntiles, cus * gemm_per_cu(cfg), max_chunks, gemm_tile_cost(cfg, d, groups, groups * ntiles <= cus));
+    c = best_chunks(groups, ntiles, cus * gemm_per_cu(cfg), max_chunks, gemm_tile_cost(cfg, d, groups, groups * ntiles <= cus), true);
   else
-    c = groups == 1 ? std::min<int64_t>(cus, most) : best_chunks(groups, ntiles, cus, most, qstat_tile_cost(cfg, d));
+    c = best_chunks(groups, ntiles, cus, most, qstat_tile_cost(cfg, d), true);
   const int64_t tpc = ceil_div(ntiles, c);
   const int xcd_pair = groups > 1 && c % 8 == 0 ? 1 : 0;
   if (!xcd_pair) c = ceil_div(ntiles, tpc);
