@@ -1323,8 +1323,20 @@ int make_q8_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int flags, int cus
     const int64_t rs = P.cfg.rs();
     const int64_t max_chunks = std::min<int64_t>({P.ntiles, 65535, kSelectMaxLists / rs, list_chunks(nq, rs, k)});
     const int64_t most = std::min<int64_t>(max_chunks, std::max<int64_t>(1, P.groups > 1 ? align_up(P.ntiles / 2, 8) : P.ntiles / 2));
-    int64_t c = P.groups == 1 ? std::min<int64_t>(cus, most)  // (an int8 column's time is half an fp16 one's)
-                              : best_chunks(P.groups, P.ntiles, cus, most, 0.5 * qstat_tile_cost(P.cfg, P.dq));
+    // (an int8 column's time is half an fp16 one's)
+    int64_t c = best_chunks(P.groups, P.ntiles, cus, most, 0.5 * qstat_tile_cost(P.cfg, P.dq));
+    // Without a sample every row passes, and a list that fills is scanned again:
+    // chunks of no more rows than a list holds (2316 x 1472, k = 45, over 1153 rows: 8 chunks 814 us,
+    // 16 299).
+    const int64_t upt = P.cfg.units_per_tile();
+    int64_t s = std::min<int64_t>(16384 / kQ8SampleDiv, std::max<int64_t>(P.ntiles / kQ8SampleDiv, ceil_div(8 * k, upt)));
+    s = std::min<int64_t>(s, (flags & CVS_FLAG_FORCE_PREPASS) ? P.ntiles : P.ntiles / 4);
+    P.s8 = !(flags & CVS_FLAG_NO_PREPASS) &&
+           (((flags & CVS_FLAG_FORCE_PREPASS) && s >= 1) || (s >= 4 && s * upt >= 2 * k));
+    if (!P.s8) {
+      const int64_t fit = ceil_div(P.ntiles, std::max<int64_t>(1, list_cap(k) / P.cfg.tile_rows()));
+      c = std::max(c, std::min<int64_t>(P.groups > 1 ? align_up(fit, 8) : fit, max_chunks));
+    }
     P.tpc = ceil_div(P.ntiles, c);
     if (P.groups == 1 || c % 8 != 0) c = ceil_div(P.ntiles, P.tpc);
     P.chunks = c;
@@ -1338,11 +1350,6 @@ int make_q8_plan(int64_t nq, int64_t n, int64_t d, int64_t k, int flags, int cus
     // (per-tile units for k = 100 at 1M x 768 cost 7 us more in the scattered
     // stores and in the threshold select than the looser threshold costs
     // later).  At most 16 * 256 units per query (the threshold kernel's limit).
-    const int64_t upt = P.cfg.units_per_tile();
-    int64_t s = std::min<int64_t>(16384 / kQ8SampleDiv, std::max<int64_t>(P.ntiles / kQ8SampleDiv, ceil_div(8 * k, upt)));
-    s = std::min<int64_t>(s, (flags & CVS_FLAG_FORCE_PREPASS) ? P.ntiles : P.ntiles / 4);
-    P.s8 = !(flags & CVS_FLAG_NO_PREPASS) &&
-           (((flags & CVS_FLAG_FORCE_PREPASS) && s >= 1) || (s >= 4 && s * upt >= 2 * k));
     if (P.s8) {
       P.s8_tiles = s;
       const int64_t wgs = std::max<int64_t>(1, std::min<int64_t>({s, cus / P.groups, (16 * 256) / upt}));

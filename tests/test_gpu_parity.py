@@ -721,6 +721,7 @@ def test_topk_rows_with_infinite_scores(eng, nq, n, k):
     (3, 255, 200, "normal"), (3, 2048, 600, "normal"), (3, 2049, 10, "normal"),  # rank, network, cut
     (3, 8192, 1024, "normal"), (3, 8193, 1, "normal"), (2, 32768, 1024, "normal"),  # whole rows, re-read past 8192
     (2, 32768, 100, "nan"), (2, 20000, 1000, "equal"),
+    (3, 16384, 1024, "normal"), (3, 16385, 40, "outlier"), (2, 12000, 600, "nan"), (700, 9001, 500, "normal"),
     (2, 32769, 1024, "normal"),            # filtered, odd strides
     (1030, 33001, 257, "normal"),          # more rows than one set of launches takes
     (2, 70001, 1000, "equal"),             # every score reaches the threshold: streamed again
@@ -769,7 +770,7 @@ def test_topk_rows_threshold_edges(eng, nq, n, k, data):
     (300, 8191, 128, 100, "matrix"), (5, 8193, 320, 3, "scan"), (1, 8192, 1600, 256, "matrix"),
     (9, 32768, 256, 40, "matrix"), (1, 16385, 768, 10, "matrix"), (100, 16000, 768, 200, "matrix"),
     (33, 24577, 512, 10, "tiled"), (200, 24576, 768, 10, "matrix"), (300, 32768, 1024, 100, "matrix"),
-    (34, 32767, 2048, 1, "scan"), (33, 4097, 64, 1, "matrix"), (64, 20001, 128, 100, "tiled"),
+    (34, 32767, 2048, 1, "tiled"), (33, 4097, 64, 1, "matrix"), (64, 20001, 128, 100, "tiled"),
     (40, 9000, 1024, 10, "matrix"), (65, 30001, 256, 10, "tiled"), (513, 20000, 2048, 5, "tiled"),
     (300, 20000, 128, 200, "matrix"), (200, 30000, 1024, 10, "matrix")])
 def test_small_corpus_search_is_exact(eng, nq, n, d, k, path):
@@ -832,6 +833,22 @@ def test_search_in_one_call_equals_its_parts(eng, metric, d):
         for method in ("fused", "int8", "auto"):
             w, j = index.search(q.cuda(), k, method=method)
             assert w.shape == (7, 5) and torch.equal(j, i)
+
+
+def test_int8_lists_of_unsampled_corpora_hold_their_rows(eng):
+    """Without a sample every row passes: a chunk of more rows than its list holds is
+    scanned again by the select (2.7 times the search's time)."""
+    nq, n, d, k = 2316, 1153, 1472, 45
+    say(f"int8 lists nq={nq} n={n} d={d} k={k}")
+    plan, _ = eng.q8_plan(nq, n, d, k)
+    assert -(-n // plan[1]) <= 128
+    x, q = make(n, d, nq, seed=4)
+    xd, qd = x.cuda(), q.cuda()
+    v, i, _ = eng.q8_topk(qd, xd, eng.q8_build(xd), k)
+    v2, i2, _ = eng.fused_topk(qd, xd, k)
+    torch.cuda.synchronize()
+    torch.testing.assert_close(v, v2, rtol=0, atol=2 * d * 2.0**-24)
+    assert (i != i2).float().mean().item() < 0.001
 
 
 @pytest.mark.parametrize("nq,n,d,k", [(200, 16000, 768, 10), (100, 24000, 1024, 10), (40, 8000, 384, 10)])
