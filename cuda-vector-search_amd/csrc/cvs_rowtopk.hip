@@ -364,8 +364,9 @@ __global__ __launch_bounds__(kBlock) void row_filter_kernel(RowTopkArgs a) {
 
 // kCandidates: the filter's; kShortRow: the row's n <= kRowCap scores; either in 64
 // registers a thread, so that two rows share a CU (1130 rows of 1721, k = 278 63 -> 43 us);
+// kMidRow: its n <= 2 kRowCap scores, likewise (2386 rows of 10020, k = 2 76 -> 46 us);
 // kRow: its n <= kRowDirect scores.
-enum Source { kCandidates, kShortRow, kRow };
+enum Source { kCandidates, kShortRow, kMidRow, kRow };
 template <Source SRC>
 __global__ __launch_bounds__(kFinal, SRC == kRow ? 1 : 8) void row_final_kernel(RowTopkArgs a) {
   constexpr bool DIRECT = SRC != kCandidates;
@@ -449,8 +450,8 @@ __global__ __launch_bounds__(kFinal, SRC == kRow ? 1 : 8) void row_final_kernel(
   };
   const int m = DIRECT ? (int)a.n : a.count[r];
   if (tid == 0) nbuf = 0;
-  if constexpr (SRC == kRow) {
-    constexpr int R = kRowDirect / kFinal;
+  if constexpr (SRC == kMidRow || SRC == kRow) {
+    constexpr int R = (SRC == kMidRow ? 2 * kRowCap : kRowDirect) / kFinal;
     float v[R];
 #pragma unroll
     for (int e = 0; e < R; ++e) v[e] = e * kFinal < m ? row[min(e * kFinal + tid, m - 1)] : 0.f;
@@ -539,6 +540,8 @@ hipError_t launch_row_topk(const RowTopkArgs& a, int rows, hipStream_t s) {
       const dim3 grid((unsigned)(rows - r < kMost ? rows - r : kMost));
       if (a.n <= kRowCap)
         hipLaunchKernelGGL(row_final_kernel<kShortRow>, grid, dim3(kFinal), 0, s, b);
+      else if (a.n <= 2 * kRowCap)
+        hipLaunchKernelGGL(row_final_kernel<kMidRow>, grid, dim3(kFinal), 0, s, b);
       else
         hipLaunchKernelGGL(row_final_kernel<kRow>, grid, dim3(kFinal), 0, s, b);
       if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
