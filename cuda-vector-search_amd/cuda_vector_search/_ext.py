@@ -468,7 +468,6 @@ class Engine:
             raise RuntimeError("corpus must have fewer than 2^31 rows")
         nq, dim = q.shape
         n, d = x.shape
-        k = int(k)  # (a float or a 0-d tensor from the caller)
         index = dev.index
         key = (nq, n, d, dim, k, normalize, xq is None, index)
         ws_bytes = self._search_bytes.get(key)

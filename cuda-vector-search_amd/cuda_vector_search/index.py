@@ -165,19 +165,21 @@ class Index:
         if shared and not copy and cosine and width != d:
             eng.prep_rows(x, x, True)
             cosine = False
+        int8 = (int8_prefilter is not False and width <= Q8_MAX_WIDTH
+                and (int8_prefilter or int8_builds(n, width)))
+        if not (cosine or int8) and width == d:  # nothing to prepare
+            self._x = x.clone() if shared and copy else x
+            return
         if (shared and copy) or width != d:
             out = torch.empty((n, width), dtype=x.dtype, device=x.device)
         else:
             out = x
-        int8 = (int8_prefilter is not False and width <= Q8_MAX_WIDTH
-                and (int8_prefilter or int8_builds(n, width)))
         self._x = out
         if out is x and not cosine:
-            if int8:
-                self._build_int8()
+            self._build_int8()
         elif int8:
             self._set_int8(eng.q8_prep_build(x, out, cosine), self._corpus_stamp())
-        elif n > 0:
+        else:
             eng.prep_rows(x, out, cosine)
 
     def _corpus_stamp(self):
@@ -248,7 +250,10 @@ class Index:
         return q if q.is_contiguous() else q.contiguous()
 
     def _prep_queries(self, queries) -> torch.Tensor:
-        q = self._query_rows(queries)
+        return self._prep_rows(self._query_rows(queries))
+
+    def _prep_rows(self, q: torch.Tensor) -> torch.Tensor:
+        """_query_rows as the engine takes them: normalised (cosine) and zero-padded."""
         width = self._x.shape[1]
         if (self._use_kernels and q.shape[0] > 0
                 and (self.metric == "cosine" or width != q.shape[1])):
@@ -288,7 +293,7 @@ class Index:
             if self._use_kernels and k <= MAX_FUSED_K:
                 method = "int8" if self._int8_wins(rows.shape[0], k) else "fused"
             elif self._use_kernels and k <= MAX_EXACT_K:
-                return self._search_large_k(self._prep_queries(rows), k)
+                return self._search_large_k(self._prep_rows(rows), k)
             else:
                 method = "torch"
         if method in ("fused", "twopass", "int8") and not self._use_kernels:
@@ -306,7 +311,7 @@ class Index:
                         torch.empty((0, k), dtype=torch.int64, device=rows.device))
             # ids come out as int64 directly (index.py:126 widens int32 with .long())
             return _ext.load().search(rows, self._x, k, self.metric == "cosine", xq)
-        q = self._prep_queries(rows)
+        q = self._prep_rows(rows)
         if method == "twopass":
             s = _ext.load().scores(q, self._x, False)
             v, i = torch.topk(s, k, dim=1)
