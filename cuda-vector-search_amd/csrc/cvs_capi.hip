@@ -324,7 +324,7 @@ bool gemm_cfg(int64_t nq, int64_t n, int64_t d, int64_t k, int cus, const ScanCf
 // filtering into lists and selecting (three to five).  Measured (us, GPU time,
 // lists / matrix): always where the corpus is too small to sample for this k,
 // whose lists then fill and are cut over and over (1000 x 768 over 16000 rows, k =
-// 100 988 / 100; 40 x 384 over 1000, k = 10 29 / 16); long results up to 16k rows
+// 100 988 / 74; 40 x 384 over 1000, k = 10 29 / 16); long results up to 16k rows
 // (200 x 384 over 16000, k = 100 111 / 36; past it only small batches: 8 x 768 over
 // 32000 40 / 34, 40 x 384 26 / 35); short ones while few scores are stored, more of
 // them where the scans are slow (1 x 384 over 5000, k = 10 19 / 9, over 32000

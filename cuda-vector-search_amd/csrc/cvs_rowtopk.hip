@@ -11,16 +11,16 @@
 //     proportion);
 //  2. row_filter_kernel, one workgroup per (row, chunk): the scores at or above
 //     the threshold into the row's candidate array;
-//  3. row_final_kernel, one workgroup per row: sorts the candidates and writes
-//     the k best.  The threshold is a guess and never decides the result: when
+//  3. row_final_kernel, one workgroup per row: cuts the candidates to few more
+//     than k, ranks those and writes the k best.  The threshold is a guess and never decides the result: when
 //     fewer than k or more than kRowCap scores reach it, the row is streamed
 //     again here and its top k taken exactly.
 //
 // Rows of at most kRowDirect scores need no threshold: step 3 takes the whole row.
 //
 // Measured against chunk-wise radix selects and a merge of the chunks' top k:
-// 64 rows x 300k, k = 1000: 192 -> 54 us; 1 x 4M, k = 1000: 3378 -> 58 us; whole
-// rows, 1000 x 8000, k = 1000: 78 -> 41 us.
+// 64 rows x 300k, k = 1000: 189 -> 49 us; 1 x 4M, k = 1000: 3380 -> 60 us; whole
+// rows, 1000 x 8000, k = 1000: 77 -> 45 us.
 #include "cvs_common.h"
 #include "cvs_kernels.h"
 
