@@ -1076,6 +1076,7 @@ constexpr int64_t kRowBatch = 1024;
 
 struct RowPlan {
   int64_t rows = 0;  // rows per set of launches
+  bool narrow = false;  // one workgroup a row, no workspace
   int64_t groups = 0, rank = 0, len = 0, chunks = 1;
   int64_t off_count = 0, off_cand = 0, ws_bytes = 0;
 };
@@ -1084,16 +1085,31 @@ RowPlan row_plan(int64_t nq, int64_t n, int64_t k, int cus) {
   RowPlan P;
   P.rows = std::max<int64_t>(1, nq);
   if (n <= kRowDirect) return P;
-  P.rows = ceil_div(P.rows, ceil_div(P.rows, kRowBatch));
   // The sample: a 32nd of the row, at least 16384 scores (8192 in batches past one row a
   // CU; a quarter of a short row), so that about 8 or more of the row's k best are
   // in it for k = 256 (30 at k = 1000 over 1M columns); the threshold is the score
   // `rank` from the top of the sample, 15% and five standard deviations (and 5)
   // past where the k-th best is expected, so that fewer than k scores practically never
-  // reach it and at most a few thousand do (kRowCap = 8192 fit).
-  P.groups = std::min<int64_t>(n / 128, std::max<int64_t>(P.rows > cus ? 256 : 512, n / 1024));
-  const double mu = (double)k * 32.0 * (double)P.groups / (double)n;
-  P.rank = (int64_t)(1.15 * mu + 5.0 * std::sqrt(mu) + 5.0);
+  // reach it and at most a few thousand do (kRowCap = 8192 fit); never past k, which
+  // as many of the sample itself reach.
+  auto sample = [&](int64_t least) {
+    P.groups = std::min<int64_t>(n / 128, std::max<int64_t>(least, n / 1024));
+    const double mu = (double)k * 32.0 * (double)P.groups / (double)n;
+    P.rank = std::min<int64_t>(k, (int64_t)(1.15 * mu + 5.0 * std::sqrt(mu) + 5.0));
+  };
+  // Two or more rows a CU: each row's whole work in one small workgroup, from a smaller
+  // sample, where about 1200 candidates are expected at most (2048 fit).  us, launches of
+  // all rows / one workgroup a row: 520 x 33000, k = 1 33 / 26; 1000 x 60000, k = 100
+  // 95 / 63; 2048 x 130000, k = 300 300 / 252; about equal over 130k to 250k columns
+  // (1200 x 130000, k = 1 0.82 at worst), past that better from 1000 rows (800 x 262145,
+  // k = 10 184 / 183, 520 127 / 146; 2048 465 / 419; 1500 x 520000 658 / 708).
+  if (nq > kNarrowRows && n <= (nq < 1000 ? 1 << 18 : 3 << 17)) {
+    sample(std::clamp<int64_t>(k, 64, 256));
+    P.narrow = P.rank * n <= 32 * P.groups * 1200;
+    if (P.narrow) return P;
+  }
+  P.rows = ceil_div(P.rows, ceil_div(P.rows, kRowBatch));
+  sample(P.rows > cus ? 256 : 512);
   // about 8 filter workgroups per CU, of 1 to 16 rounds of 4096 columns
   const int64_t want = ceil_div(P.rows * n, 8 * (int64_t)cus);
   P.len = std::max<int64_t>(4096, std::min<int64_t>(65536, align_up(want, 4096)));
@@ -1153,9 +1169,10 @@ int cvs_topk_rows(const float* scores, int64_t nq, int64_t n, int64_t k, int fla
   r.out_v = out_v;
   r.out_i = out_i;
   r.ids64 = (flags & CVS_FLAG_IDS_INT64) ? 1 : 0;
+  r.groups = (int)P.groups;
+  r.rank = (int)P.rank;
+  r.narrow = P.narrow ? 1 : 0;
   if (P.ws_bytes > 0) {
-    r.groups = (int)P.groups;
-    r.rank = (int)P.rank;
     r.len = P.len;
     r.chunks = (int)P.chunks;
     r.tau = reinterpret_cast<uint32_t*>(ws);

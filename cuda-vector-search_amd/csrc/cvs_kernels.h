@@ -131,6 +131,7 @@ struct GemvArgs {
 // row0 + r of the matrix and of the outputs.
 constexpr int kRowTopkMaxK = 1024;
 constexpr int kRowCap = 8192;      // candidates per row
+constexpr int kNarrowRows = 512;   // rows past which small workgroups take them (two rows a CU)
 constexpr int kRowDirect = 32768;  // rows up to this are cut by one workgroup, without a sampled threshold
 struct RowTopkArgs {
   const float* scores;  // [rows, n] fp32
@@ -146,6 +147,7 @@ struct RowTopkArgs {
   int rank;             // the sample's rank taken as threshold
   int64_t len;          // columns per filter workgroup (a multiple of 4)
   int chunks;           // ceil(n / len)
+  int narrow;           // 1: one small workgroup a row, without tau, count and cand
   uint32_t* tau;        // [rows of a launch] threshold order keys
   int* count;           // [rows of a launch] scores that reached them
   uint64_t* cand;       // [rows of a launch, kRowCap] their keys

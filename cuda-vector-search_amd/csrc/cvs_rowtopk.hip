@@ -17,10 +17,12 @@
 //     again here and its top k taken exactly.
 //
 // Rows of at most kRowDirect scores need no threshold: step 3 takes the whole row.
+// With two or more rows a CU, one workgroup of 256 threads does a long row's three
+// steps (kStream), the candidates in LDS.
 //
 // Measured against chunk-wise radix selects and a merge of the chunks' top k:
 // 64 rows x 300k, k = 1000: 189 -> 49 us; 1 x 4M, k = 1000: 3380 -> 60 us; whole
-// rows, 1000 x 8000, k = 1000: 77 -> 45 us.
+// rows, 1000 x 8000, k = 1000: 77 -> 46 us; 4000 x 40000, k = 100: 258 -> 188.
 #include "cvs_common.h"
 #include "cvs_kernels.h"
 
@@ -28,8 +30,9 @@ namespace cvs {
 
 namespace {
 
-constexpr int kFinal = 1024;              // threads of the sample and final kernels
-constexpr int kFinalWaves = kFinal / kWave;
+// T below: threads of a row's workgroup, 1024, or 256 and 512 where there are
+// several rows a CU (barriers then wait for fewer waves, and 7 or 4 rows share a CU).
+constexpr int kNarrow = 256;
 constexpr int kBins = 1024;
 constexpr int kFilterU = 16;              // scores per thread and round of the filter
 constexpr int kFilterFlush = 512;         // candidates in LDS that trigger a write-out
@@ -45,16 +48,18 @@ struct Bins {
   }
 };
 
+template <int T>
 struct BinScratch {
-  float mm[2][kFinalWaves];
+  float mm[2][T / kWave];
   int hist[kBins];
-  int wsum[kFinalWaves];
+  int wsum[T / kWave];
   int bin, above;
 };
 
 // The block's bins over the [min, max] of every thread's (lo, hi), an empty
 // histogram, and false when that range is empty or not finite.  Whole block.
-__device__ __forceinline__ bool make_bins(BinScratch& B, float lo, float hi, Bins* bins) {
+template <int T>
+__device__ __forceinline__ bool make_bins(BinScratch<T>& B, float lo, float hi, Bins* bins) {
   const int tid = threadIdx.x;
   lo = wave_min_f32(lo);
   hi = wave_max_f32(hi);
@@ -62,12 +67,13 @@ __device__ __forceinline__ bool make_bins(BinScratch& B, float lo, float hi, Bin
     B.mm[0][tid / kWave] = lo;
     B.mm[1][tid / kWave] = hi;
   }
-  B.hist[tid] = 0;  // kBins == kFinal
+#pragma unroll
+  for (int i = 0; i < kBins / T; ++i) B.hist[i * T + tid] = 0;
   __syncthreads();
   lo = B.mm[0][0];
   hi = B.mm[1][0];
 #pragma unroll
-  for (int i = 1; i < kFinalWaves; ++i) {
+  for (int i = 1; i < T / kWave; ++i) {
     lo = fminf(lo, B.mm[0][i]);
     hi = fmaxf(hi, B.mm[1][i]);
   }
@@ -80,19 +86,30 @@ __device__ __forceinline__ bool make_bins(BinScratch& B, float lo, float hi, Bin
 // The highest bin b with at least `want` counts in bins >= b (bin 0 when there
 // are fewer in all), and that count.  Whole block, after a barrier that made
 // the histogram complete.
-__device__ __forceinline__ int cut_bin(BinScratch& B, int want, int* above) {
+template <int T>
+__device__ __forceinline__ int cut_bin(BinScratch<T>& B, int want, int* above) {
+  constexpr int Q = kBins / T;  // bins a thread, descending
   const int tid = threadIdx.x;
-  const int b = kBins - 1 - tid;  // descending
-  const int c = B.hist[b];
-  int incl = wave_incl_sum_i32(c);
+  int c[Q], sum = 0;
+#pragma unroll
+  for (int i = 0; i < Q; ++i) {
+    c[i] = B.hist[kBins - 1 - tid * Q - i];
+    sum += c[i];
+  }
+  int incl = wave_incl_sum_i32(sum);
   if (tid % kWave == kWave - 1) B.wsum[tid / kWave] = incl;
   if (tid == 0) B.bin = -1;
   __syncthreads();
 #pragma unroll
-  for (int w = 0; w < kFinalWaves; ++w) incl += w < tid / kWave ? B.wsum[w] : 0;
-  if (incl - c < want && want <= incl) {
-    B.bin = b;
-    B.above = incl;
+  for (int w = 0; w < T / kWave; ++w) incl += w < tid / kWave ? B.wsum[w] : 0;
+  int run = incl - sum;
+#pragma unroll
+  for (int i = 0; i < Q; ++i) {
+    if (run < want && want <= run + c[i]) {
+      B.bin = kBins - 1 - tid * Q - i;
+      B.above = run + c[i];
+    }
+    run += c[i];
   }
   __syncthreads();
   *above = B.above;
@@ -114,8 +131,8 @@ struct Cut {
 // values, all equal, NaNs that count).  each(f) calls f(v) for the thread's
 // values.  Whole block.
 constexpr int kNoCut = 0x7fffffff;
-template <class Each>
-__device__ __forceinline__ int find_cut(BinScratch& B, int k, int want, bool skip_nan, Each each, Cut* cut) {
+template <int T, class Each>
+__device__ __forceinline__ int find_cut(BinScratch<T>& B, int k, int want, bool skip_nan, Each each, Cut* cut) {
   float lo = __builtin_inff(), hi = -__builtin_inff();
   each([&](float v) {
     if (__builtin_isfinite(v)) {  // (infinities fall into the outer bins)
@@ -154,15 +171,15 @@ __device__ __forceinline__ int find_cut(BinScratch& B, int k, int want, bool ski
   return count;
 }
 
-// Descending bitonic sort of N = kFinal * E keys, key i = tid * E + e in v[e] of
+// Descending bitonic sort of N = T * E keys, key i = tid * E + e in v[e] of
 // thread tid.  Strides below E stay in the thread, those below 64 E in the wave
-// (shuffles), the rest (10 stages of 66 at E = 2) cross waves through `lds`
+// (shuffles), the rest (10 stages of 66 at T = 1024, E = 2) cross waves through `lds`
 // (N keys).  Whole block.
-template <int E>
+template <int T, int E>
 __device__ __forceinline__ void block_bitonic_desc(uint64_t (&v)[E], uint64_t* lds) {
   const int tid = threadIdx.x;
 #pragma unroll 1
-  for (int size = 2; size <= kFinal * E; size <<= 1) {
+  for (int size = 2; size <= T * E; size <<= 1) {
 #pragma unroll 1
     for (int stride = size >> 1; stride >= E; stride >>= 1) {
       const int ls = stride / E;  // partner thread: tid ^ ls
@@ -170,10 +187,10 @@ __device__ __forceinline__ void block_bitonic_desc(uint64_t (&v)[E], uint64_t* l
       if (ls >= kWave) {
         __syncthreads();
 #pragma unroll
-        for (int e = 0; e < E; ++e) lds[e * kFinal + tid] = v[e];
+        for (int e = 0; e < E; ++e) lds[e * T + tid] = v[e];
         __syncthreads();
 #pragma unroll
-        for (int e = 0; e < E; ++e) o[e] = lds[e * kFinal + (tid ^ ls)];
+        for (int e = 0; e < E; ++e) o[e] = lds[e * T + (tid ^ ls)];
       } else {
 #pragma unroll
         for (int e = 0; e < E; ++e) o[e] = __shfl_xor(v[e], ls);
@@ -204,20 +221,20 @@ __device__ __forceinline__ void block_bitonic_desc(uint64_t (&v)[E], uint64_t* l
   }
 }
 
-// Sorts the m <= kFinal * E keys get(i) and calls put(i, key) for the first
-// min(k, m) of them in descending order.  Whole block; `lds` holds kFinal * E keys
+// Sorts the m <= T * E keys get(i) and calls put(i, key) for the first
+// min(k, m) of them in descending order.  Whole block; `lds` holds T * E keys
 // and may be what get() reads.
-template <int E, class Get, class Put>
+template <int T, int E, class Get, class Put>
 __device__ __forceinline__ void sort_and_put(int m, int k, uint64_t* lds, Get get, Put put) {
   const int tid = threadIdx.x;
   uint64_t v[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) {
-    const int i = e * kFinal + tid;
+    const int i = e * T + tid;
     v[e] = i < m ? get(i) : 0ull;  // key 0: below every real key
   }
   __syncthreads();
-  block_bitonic_desc<E>(v, lds);
+  block_bitonic_desc<T, E>(v, lds);
   __syncthreads();  // put() may write to lds
   const int top = min(k, m);
 #pragma unroll
@@ -228,11 +245,11 @@ __device__ __forceinline__ void sort_and_put(int m, int k, uint64_t* lds, Get ge
 // The same for m <= 256 keys by rank: G threads count the keys above each (over
 // slices), two barriers where the network takes 55 stages (rows of 3000 scores,
 // k = 10, with their GEMV: 16 -> 8 us).  Equal keys (0: none) rank by position.
-template <class Get, class Put>
+template <int T, class Get, class Put>
 __device__ __forceinline__ void rank_and_put(int m, int k, uint64_t* lds, Get get, Put put) {
   __shared__ int rank[256];
   const int tid = threadIdx.x;
-  const int P = m <= 64 ? 64 : 256, G = kFinal / P;
+  const int P = m <= 64 ? 64 : 256, G = T / P;
   const int i = tid & (P - 1), g = tid / P;
   const uint64_t mine = i < m ? get(i) : 0ull;
   if (tid < P) rank[tid] = 0;
@@ -252,31 +269,31 @@ __device__ __forceinline__ void rank_and_put(int m, int k, uint64_t* lds, Get ge
   if (g == 0 && i < m && rank[i] < k) put(rank[i], mine);
 }
 
-template <class Get, class Put>
+template <int T, class Get, class Put>
 __device__ __forceinline__ void sort_any(int m, int k, uint64_t* lds, Get get, Put put) {
   if (m <= 256)
-    rank_and_put(m, k, lds, get, put);
-  else if (m <= kFinal)
-    sort_and_put<1>(m, k, lds, get, put);
-  else if (m <= 2 * kFinal)
-    sort_and_put<2>(m, k, lds, get, put);
-  else if (m <= 4 * kFinal)
-    sort_and_put<4>(m, k, lds, get, put);
+    rank_and_put<T>(m, k, lds, get, put);
+  else if (m <= T)
+    sort_and_put<T, 1>(m, k, lds, get, put);
+  else if (m <= 2 * T)
+    sort_and_put<T, 2>(m, k, lds, get, put);
+  else if (m <= 4 * T)
+    sort_and_put<T, 4>(m, k, lds, get, put);
   else
-    sort_and_put<8>(m, k, lds, get, put);
+    sort_and_put<T, 8>(m, k, lds, get, put);
 }
 
-__global__ __launch_bounds__(kFinal) void row_sample_kernel(RowTopkArgs a) {
-  __shared__ BinScratch B;
+// The order key of a row's sampled threshold; ~0u: no guess (equal or no finite
+// samples).  Whole block.
+template <int T>
+__device__ __forceinline__ uint32_t sample_threshold(BinScratch<T>& B, const RowTopkArgs& a, const float* src) {
   const int tid = threadIdx.x;
-  const int r = blockIdx.x;
-  const float* src = a.scores + (a.row0 + r) * a.n;
   const int64_t S = 32 * (int64_t)a.groups;  // group g: 32 scores centred in the row's g-th of `groups` parts
   const int64_t step = a.n / a.groups;
   auto at = [&](int64_t i) { return src[(i >> 5) * step + ((step - 32) >> 1) + (i & 31)]; };
   float lo = __builtin_inff(), hi = -__builtin_inff();
 #pragma unroll 8
-  for (int64_t i = tid; i < S; i += kFinal) {
+  for (int64_t i = tid; i < S; i += T) {
     const float v = at(i);
     if (__builtin_isfinite(v)) {
       lo = fminf(lo, v);
@@ -286,14 +303,59 @@ __global__ __launch_bounds__(kFinal) void row_sample_kernel(RowTopkArgs a) {
   Bins bins;
   const bool ok = make_bins(B, lo, hi, &bins);
 #pragma unroll 8
-  for (int64_t i = tid; i < S; i += kFinal) atomicAdd(&B.hist[bins.of(at(i))], 1);  // (re-read: in cache)
+  for (int64_t i = tid; i < S; i += T) atomicAdd(&B.hist[bins.of(at(i))], 1);  // (re-read: in cache)
   __syncthreads();
   int above;
   const int b = cut_bin(B, a.rank, &above);
-  if (tid == 0) {
-    // (equal or no finite samples: no guess, and no candidates; step 3 streams the row)
-    a.tau[r] = ok ? float_order(bins.lo + (float)b / bins.scale) : ~0u;
+  return ok ? float_order(bins.lo + (float)b / bins.scale) : ~0u;
+}
+
+__global__ __launch_bounds__(1024) void row_sample_kernel(RowTopkArgs a) {
+  __shared__ BinScratch<1024> B;
+  const int r = blockIdx.x;
+  const uint32_t tau = sample_threshold(B, a, a.scores + (a.row0 + r) * a.n);
+  if (threadIdx.x == 0) {
+    a.tau[r] = tau;  // (~0u: no candidates; step 3 streams the row)
     a.count[r] = 0;
+  }
+}
+
+// Appends the keys of the columns [c0, c1) whose order keys reach tk, kFilterU of
+// each of T threads from `base` on: 16-byte loads from the aligned addresses at
+// or below each four columns (a row's first column sits `off` floats past one; base =
+// c0 - off + a multiple of kFilterU T).  A quad that is not wholly inside the
+// range loads its columns one by one.
+template <int T, class Put>
+__device__ __forceinline__ void filter_round(const float* row, int64_t base, int64_t c0, int64_t c1, uint32_t tk,
+                                             int* nbuf, Put put) {
+  const int tid = threadIdx.x;
+  f32x4 v[kFilterU / 4];
+#pragma unroll
+  for (int u = 0; u < kFilterU / 4; ++u) {
+    const int64_t col = base + (u * T + tid) * 4;
+    v[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (col >= c0 && col + 4 <= c1) {
+      v[u] = *(const f32x4*)(row + col);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (col + j >= c0 && col + j < c1) v[u][j] = row[col + j];
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < kFilterU / 4; ++u) {
+    const int64_t col = base + (u * T + tid) * 4;
+    unsigned pass = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      pass |= (col + j >= c0 && col + j < c1 && float_order(v[u][j]) >= tk ? 1u : 0u) << j;
+    if (__ballot(pass != 0) == 0) continue;
+    if (pass) {
+      int p = atomicAdd(nbuf, __popc(pass));
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if ((pass >> j) & 1u) put(p++, make_key(v[u][j], (int)(col + j)));
+    }
   }
 }
 
@@ -306,10 +368,7 @@ __global__ __launch_bounds__(kBlock) void row_filter_kernel(RowTopkArgs a) {
   const int64_t c0 = (int64_t)c * a.len;
   const int64_t c1 = min<int64_t>(c0 + a.len, a.n);
   const float* row = a.scores + (a.row0 + r) * a.n;
-  // 16-byte loads from the aligned addresses at or below each four columns: a
-  // row's first column sits `off` floats past one.  A quad that is not wholly
-  // inside the chunk loads its columns one by one.
-  const int off = (int)((reinterpret_cast<uintptr_t>(row) >> 2) & 3);
+  const int off = (int)((reinterpret_cast<uintptr_t>(row) >> 2) & 3);  // (c0: a multiple of 4)
   const uint32_t tk = a.tau[r];
   if (tid == 0) nbuf = 0;
   __syncthreads();
@@ -326,34 +385,7 @@ __global__ __launch_bounds__(kBlock) void row_filter_kernel(RowTopkArgs a) {
     __syncthreads();
   };
   for (int64_t base = c0 - off; base < c1; base += kFilterRound) {
-    f32x4 v[kFilterU / 4];
-#pragma unroll
-    for (int u = 0; u < kFilterU / 4; ++u) {
-      const int64_t col = base + (u * kBlock + tid) * 4;
-      v[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (col >= c0 && col + 4 <= c1) {
-        v[u] = *(const f32x4*)(row + col);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (col + j >= c0 && col + j < c1) v[u][j] = row[col + j];
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < kFilterU / 4; ++u) {
-      const int64_t col = base + (u * kBlock + tid) * 4;
-      unsigned pass = 0;
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        pass |= (col + j >= c0 && col + j < c1 && float_order(v[u][j]) >= tk ? 1u : 0u) << j;
-      if (__ballot(pass != 0) == 0) continue;
-      if (pass) {
-        int p = atomicAdd(&nbuf, __popc(pass));
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if ((pass >> j) & 1u) buf[p++] = make_key(v[u][j], (int)(col + j));
-      }
-    }
+    filter_round<kBlock>(row, base, c0, c1, tk, &nbuf, [&](int p, uint64_t key) { buf[p] = key; });
     __syncthreads();
     const bool full = nbuf > kFilterFlush;
     if (full) flush();
@@ -362,17 +394,19 @@ __global__ __launch_bounds__(kBlock) void row_filter_kernel(RowTopkArgs a) {
   if (nbuf > 0) flush();
 }
 
-// kCandidates: the filter's; kShortRow: the row's n <= kRowCap scores; either in 64
-// registers a thread, so that two rows share a CU (1130 rows of 1721, k = 278 63 -> 43 us);
+// kCandidates: the filter's; kShortRow: the row's n <= 8 T scores; either in 64
+// registers a thread, so that two rows of 1024 threads share a CU.  Past kNarrowRows rows
+// T is the smallest that holds the row: 2500 x 1326, k = 300 79 -> 28 us (T = 1024, 256),
+// 2500 x 2600 83 -> 40 (512); 512 rows 1.15 to 0.57 of T = 1024's time, 256 1.4 to 0.7.
 // kMidRow: its n <= 2 kRowCap scores, likewise (2386 rows of 10020, k = 2 76 -> 46 us);
-// kRow: its n <= kRowDirect scores.
-enum Source { kCandidates, kShortRow, kMidRow, kRow };
-template <Source SRC>
-__global__ __launch_bounds__(kFinal, SRC == kRow ? 1 : 8) void row_final_kernel(RowTopkArgs a) {
-  constexpr bool DIRECT = SRC != kCandidates;
-  constexpr int E = kRowCap / kFinal;
-  __shared__ uint64_t keys[kRowCap];
-  __shared__ BinScratch B;
+// kRow: its n <= kRowDirect scores; kStream: all three steps by the row's one workgroup.
+enum Source { kCandidates, kShortRow, kMidRow, kRow, kStream };
+template <Source SRC, int T = 1024>
+__global__ __launch_bounds__(T, SRC == kRow ? 1 : 8) void row_final_kernel(RowTopkArgs a) {
+  constexpr bool DIRECT = SRC != kCandidates && SRC != kStream;
+  constexpr int E = 8, kCap = T * E;
+  __shared__ uint64_t keys[kCap];
+  __shared__ BinScratch<T> B;
   __shared__ int nbuf;
   __shared__ uint64_t kth;
   const int tid = threadIdx.x;
@@ -394,13 +428,13 @@ __global__ __launch_bounds__(kFinal, SRC == kRow ? 1 : 8) void row_final_kernel(
   // keys costs several times one of the ~k that matter, so they are cut first: to
   // those that reach the k-th best of the threads' maxima (one value a thread to
   // bin), or, where that leaves too many or k is large, by bins of their own.
-  // False when neither leaves kRowCap, unless `all` fit.  (Searches over 16000 x
+  // False when neither leaves kCap, unless `all` fit.  (Searches over 16000 x
   // 768, 200 queries, k = 10, plain / one row of 3000 times the others' norm: 27 / 29 us;
   // with bins over the row's values alone 32 / 144.)
   auto finish = [&](auto each, auto key, bool all) __attribute__((always_inline)) {
     Cut cut;
     int total = kNoCut;
-    if (k <= kFinal / 2) {
+    if (k <= T / 2) {
       float mx = -__builtin_inff();
       bool any = false, nan = false;
       each([&](float v, int) {
@@ -417,72 +451,89 @@ __global__ __launch_bounds__(kFinal, SRC == kRow ? 1 : 8) void row_final_kernel(
         if (tid % kWave == 0) B.mm[0][tid / kWave] = t;
         __syncthreads();
 #pragma unroll
-        for (int i = 0; i < kFinalWaves; ++i) t = fminf(t, B.mm[0][i]);
+        for (int i = 0; i < T / kWave; ++i) t = fminf(t, B.mm[0][i]);
         each([&](float v, int e) {
           if (v >= t) {
             const int p = atomicAdd(&nbuf, 1);
-            if (p < kRowCap) keys[p] = key(e);
+            if (p < kCap) keys[p] = key(e);
           }
         });
         __syncthreads();
         total = nbuf;
-        if (total > kRowCap) {
+        if (total > kCap) {
           __syncthreads();
           if (tid == 0) nbuf = 0;
           __syncthreads();
         }
       }
     }
-    if (total > kRowCap) {
-      const int c = find_cut(B, k, 2 * kFinal, a.skip_nan, [&](auto f) {
+    if (total > kCap) {
+      const int c = find_cut(B, k, k <= T ? 2 * T : kCap, a.skip_nan, [&](auto f) {
         each([&](float v, int) { f(v); });
       }, &cut);
-      if (c > kRowCap && !all) return false;
+      if (c > kCap && !all) return false;
       each([&](float v, int e) {
-        if (c > kRowCap || cut.keeps(v)) keys[atomicAdd(&nbuf, 1)] = key(e);
+        if (c > kCap || cut.keeps(v)) keys[atomicAdd(&nbuf, 1)] = key(e);
       });
       __syncthreads();
       total = nbuf;
     }
-    sort_any(total, k, keys, [&](int i) { return keys[i]; }, put);
-    for (int i = total + tid; i < k; i += kFinal) put(i, 0ull);  // (NaNs left out)
+    sort_any<T>(total, k, keys, [&](int i) { return keys[i]; }, put);
+    for (int i = total + tid; i < k; i += T) put(i, 0ull);  // (NaNs left out)
     return true;
   };
-  const int m = DIRECT ? (int)a.n : a.count[r];
   if (tid == 0) nbuf = 0;
+  int m = (int)a.n;
+  if constexpr (SRC == kCandidates) m = a.count[r];
+  if constexpr (SRC == kStream) {
+    const uint32_t tk = sample_threshold(B, a, row);  // (its barriers: nbuf is cleared)
+    const int off = (int)((reinterpret_cast<uintptr_t>(row) >> 2) & 3);
+    if (tk != ~0u)
+      for (int64_t base = -off; base < a.n; base += T * kFilterU) {
+        filter_round<T>(row, base, 0, a.n, tk, &nbuf, [&](int p, uint64_t key) {
+          if (p < kCap) keys[p] = key;
+        });
+        if (*(volatile int*)&nbuf > kCap) break;
+      }
+    __syncthreads();
+    m = nbuf;
+    __syncthreads();
+    if (tid == 0) nbuf = 0;
+  }
   if constexpr (SRC == kMidRow || SRC == kRow) {
-    constexpr int R = (SRC == kMidRow ? 2 * kRowCap : kRowDirect) / kFinal;
+    constexpr int R = (SRC == kMidRow ? 2 * kRowCap : kRowDirect) / T;
     float v[R];
 #pragma unroll
-    for (int e = 0; e < R; ++e) v[e] = e * kFinal < m ? row[min(e * kFinal + tid, m - 1)] : 0.f;
+    for (int e = 0; e < R; ++e) v[e] = e * T < m ? row[min(e * T + tid, m - 1)] : 0.f;
     auto each = [&](auto f) __attribute__((always_inline)) {
 #pragma unroll
       for (int e = 0; e < R; ++e)
-        if (e * kFinal + tid < m) f(v[e], e);
+        if (e * T + tid < m) f(v[e], e);
     };
-    if (finish(each, [&](int e) { return make_key(v[e], e * kFinal + tid); }, false)) return;
+    if (finish(each, [&](int e) { return make_key(v[e], e * T + tid); }, false)) return;
     __syncthreads();
-  } else if (DIRECT || (m >= k && m <= kRowCap)) {
-    const uint64_t* cand = DIRECT ? nullptr : a.cand + (int64_t)r * kRowCap;
+  } else if (DIRECT || (m >= k && m <= kCap)) {
+    const uint64_t* cand = SRC == kStream ? keys : DIRECT ? nullptr : a.cand + (int64_t)r * kRowCap;
     auto get = [&](int i) -> uint64_t {
       if constexpr (!DIRECT) return cand[i];
       const float v = row[i];
       return a.skip_nan && v != v ? 0ull : make_key(v, i);
     };
-    if (m <= 256 || (m <= 2 * kFinal && 4 * k > m)) {
-      sort_any(m, k, keys, get, put);
+    if (m <= 256 || (m <= 2 * T && (4 * k > m || T == kNarrow))) {
+      sort_any<T>(m, k, keys, get, put);
       return;
     }
     uint64_t v[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-      const int i = e * kFinal + tid;
+      const int i = e * T + tid;
       v[e] = i < m ? get(i) : 0ull;
     }
+    if constexpr (SRC == kStream) __syncthreads();  // (read before finish() writes to keys)
     auto each = [&](auto f) __attribute__((always_inline)) {
 #pragma unroll
       for (int e = 0; e < E; ++e)
-        if (e * kFinal + tid < m) f(key_score(v[e]), e);
+        if (e * T + tid < m) f(key_score(v[e]), e);
     };
     finish(each, [&](int e) { return v[e]; }, true);
     return;
@@ -490,8 +541,8 @@ __global__ __launch_bounds__(kFinal, SRC == kRow ? 1 : 8) void row_final_kernel(
   // The threshold missed, or the cut (equal scores, NaNs): the row streamed, its running k best in LDS.
   if (tid == 0) kth = 0ull;
   __syncthreads();
-  constexpr int kSkip = 16 * kFinal;  // columns left out at once when none reaches the running k best
-  for (int64_t base = 0; base < a.n; base += 4 * kFinal) {
+  constexpr int kSkip = 16 * T;  // columns left out at once when none reaches the running k best
+  for (int64_t base = 0; base < a.n; base += 4 * T) {
     const uint64_t t = kth;
     auto key_at = [&](int64_t col) -> uint64_t {
       const float v = col < a.n ? row[col] : 0.f;
@@ -500,25 +551,25 @@ __global__ __launch_bounds__(kFinal, SRC == kRow ? 1 : 8) void row_final_kernel(
     if (t != 0ull && base % kSkip == 0 && base + kSkip < a.n) {  // (uniform)
       bool any = false;
 #pragma unroll
-      for (int u = 0; u < kSkip / kFinal; ++u) any |= key_at(base + u * kFinal + tid) > t;
+      for (int u = 0; u < kSkip / T; ++u) any |= key_at(base + u * T + tid) > t;
       if (!__syncthreads_or(any)) {
-        base += kSkip - 4 * kFinal;
+        base += kSkip - 4 * T;
         continue;
       }
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const uint64_t key = key_at(base + u * kFinal + tid);
+      const uint64_t key = key_at(base + u * T + tid);
       if (key > t) keys[atomicAdd(&nbuf, 1)] = key;
     }
     __syncthreads();
     const int nb = nbuf;
-    const bool last = base + 4 * kFinal >= a.n;
+    const bool last = base + 4 * T >= a.n;
     if (last) {
-      sort_any(nb, k, keys, [&](int i) { return keys[i]; }, put);
-      for (int i = nb + tid; i < k; i += kFinal) put(i, 0ull);  // (NaNs left out)
-    } else if (nb > 4 * kFinal) {
-      sort_and_put<E>(nb, k, keys, [&](int i) { return keys[i]; }, [&](int i, uint64_t key) {
+      sort_any<T>(nb, k, keys, [&](int i) { return keys[i]; }, put);
+      for (int i = nb + tid; i < k; i += T) put(i, 0ull);  // (NaNs left out)
+    } else if (nb > 4 * T) {
+      sort_and_put<T, E>(nb, k, keys, [&](int i) { return keys[i]; }, [&](int i, uint64_t key) {
         keys[i] = key;
         if (i == k - 1) kth = key;
       });
@@ -532,28 +583,36 @@ __global__ __launch_bounds__(kFinal, SRC == kRow ? 1 : 8) void row_final_kernel(
 
 hipError_t launch_row_topk(const RowTopkArgs& a, int rows, hipStream_t s) {
   if (a.k < 1 || a.k > kRowTopkMaxK || a.n < a.k || rows < 1 || a.scores == nullptr) return hipErrorInvalidValue;
-  if (a.n <= kRowDirect) {
+  const bool sampled = a.n > kRowDirect;
+  if (sampled && (a.groups < 1 || 32 * (int64_t)a.groups > a.n)) return hipErrorInvalidValue;
+  if (!sampled || a.narrow) {
     constexpr int64_t kMost = 1 << 21;  // workgroups of a launch: fewer than 2^32 threads
     for (int64_t r = 0; r < rows; r += kMost) {
       RowTopkArgs b = a;
       b.row0 = a.row0 + r;
       const dim3 grid((unsigned)(rows - r < kMost ? rows - r : kMost));
-      if (a.n <= kRowCap)
-        hipLaunchKernelGGL(row_final_kernel<kShortRow>, grid, dim3(kFinal), 0, s, b);
+      if (sampled)
+        hipLaunchKernelGGL((row_final_kernel<kStream, kNarrow>), grid, dim3(kNarrow), 0, s, b);
+      else if (a.n <= 8 * kNarrow && rows > kNarrowRows)
+        hipLaunchKernelGGL((row_final_kernel<kShortRow, kNarrow>), grid, dim3(kNarrow), 0, s, b);
+      else if (a.n <= 8 * 512 && rows > kNarrowRows)
+        hipLaunchKernelGGL((row_final_kernel<kShortRow, 512>), grid, dim3(512), 0, s, b);
+      else if (a.n <= kRowCap)
+        hipLaunchKernelGGL(row_final_kernel<kShortRow>, grid, dim3(1024), 0, s, b);
       else if (a.n <= 2 * kRowCap)
-        hipLaunchKernelGGL(row_final_kernel<kMidRow>, grid, dim3(kFinal), 0, s, b);
+        hipLaunchKernelGGL(row_final_kernel<kMidRow>, grid, dim3(1024), 0, s, b);
       else
-        hipLaunchKernelGGL(row_final_kernel<kRow>, grid, dim3(kFinal), 0, s, b);
+        hipLaunchKernelGGL(row_final_kernel<kRow>, grid, dim3(1024), 0, s, b);
       if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     }
     return hipSuccess;
   }
-  if (a.tau == nullptr || a.count == nullptr || a.cand == nullptr || a.groups < 1 || 32 * (int64_t)a.groups > a.n ||
-      a.chunks < 1 || a.len < 1 || a.len * a.chunks < a.n || (int64_t)rows * a.chunks > 0x7fffffff)
+  if (a.tau == nullptr || a.count == nullptr || a.cand == nullptr || a.chunks < 1 || a.len < 1 ||
+      a.len * a.chunks < a.n || (int64_t)rows * a.chunks > 0x7fffffff)
     return hipErrorInvalidValue;
-  hipLaunchKernelGGL(row_sample_kernel, dim3(rows), dim3(kFinal), 0, s, a);
+  hipLaunchKernelGGL(row_sample_kernel, dim3(rows), dim3(1024), 0, s, a);
   hipLaunchKernelGGL(row_filter_kernel, dim3(rows * a.chunks), dim3(kBlock), 0, s, a);
-  hipLaunchKernelGGL(row_final_kernel<kCandidates>, dim3(rows), dim3(kFinal), 0, s, a);
+  hipLaunchKernelGGL(row_final_kernel<kCandidates>, dim3(rows), dim3(1024), 0, s, a);
   return hipGetLastError();
 }
 

@@ -169,8 +169,8 @@ int cvs_fused_topk_noalloc(const void* q, const void* x, int64_t nq, int64_t n, 
  * descending then index ascending (the fused path's order).  1 <= k <= 1024,
  * k <= n.  out_v is [nq, k] fp32, out_i [nq, k] int32 (int64 with
  * CVS_FLAG_IDS_INT64; other flag bits are ignored).  Rows longer than 32768
- * are filtered by a sampled threshold first; `workspace` holds the scores that
- * reach it (size from cvs_topk_rows_plan).  With cvs_scores this is
+ * are filtered by a sampled threshold first; `workspace` holds the scores of
+ * longer rows that reach it (size from cvs_topk_rows_plan).  With cvs_scores this is
  * the exact large-k search that the reference leaves to torch (fp16 matmul +
  * torch.topk, index.py:118 / reference.py:8-15) for k > 256.
  */
@@ -178,7 +178,7 @@ int cvs_topk_rows(const float* scores, int64_t nq, int64_t n, int64_t k, int fla
                   int64_t workspace_bytes, float* out_v, void* out_i, int device, void* stream);
 
 /* Workspace bytes cvs_topk_rows needs for these sizes (0 for rows of at most
- * 32768 columns, 64 MB and a little at most); 256-byte aligned, no
+ * 32768 columns and for many rows of few more, 64 MB and a little at most); 256-byte aligned, no
  * initialisation needed. */
 int cvs_topk_rows_plan(int64_t nq, int64_t n, int64_t k, int device, int64_t* workspace_bytes);
 

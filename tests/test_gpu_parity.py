@@ -765,6 +765,40 @@ def test_topk_rows_threshold_edges(eng, nq, n, k, data):
     np.testing.assert_array_equal(v.cpu().numpy(), np.take_along_axis(s.numpy(), order, axis=1))
 
 
+@pytest.mark.parametrize("nq,n,k", [
+    (513, 255, 200), (600, 511, 511), (513, 513, 1), (600, 1326, 129), (513, 1326, 708), (513, 2047, 1024), (513, 2048, 300),
+    (513, 2049, 300), (512, 2048, 300),            # either side of the small workgroups
+    (513, 32769, 1), (520, 40000, 64), (520, 40001, 100), (520, 40002, 300), (1025, 33000, 257), (520, 33000, 1024)])
+def test_topk_rows_of_many_rows(eng, nq, n, k):
+    """Batches past the small workgroups' threshold, some rows far from the others' distribution: equal, NaN,
+    infinite or nested scores, thousands that tie at a sampled threshold, and too many that do."""
+    say(f"topk_rows nq={nq} n={n} k={k} many rows")
+    g = torch.Generator().manual_seed(n + k)
+    s = torch.randn(nq, n, generator=g)
+    s[0] = 0.25
+    s[1, 17::91] = float("nan")
+    s[2, 3::5] = float("inf")
+    s[3] = -float("inf")
+    s[4, 11] = 3e4
+    s[5, n // 2:n // 2 + 40] += 10.0 ** torch.arange(40, dtype=torch.float64).sub(4).float()
+    s[6] = (torch.arange(n) % 10 == 0).float()
+    s[7] = (torch.arange(n) % 3 == 0).float()
+    s[8] = torch.arange(n).float()
+    s[9] = -torch.arange(n).float()
+    s[10, : n // 8] += 20.0
+    v, i = eng.topk_rows(s.cuda(), k)
+    torch.cuda.synchronize()
+    for rows in (slice(0, 16), slice(nq - 4, nq)):
+        sn = np.ascontiguousarray(s[rows].numpy())
+        bits = sn.view(np.uint32).astype(np.int64)
+        key = np.where(bits & 0x80000000, 0xFFFFFFFF - bits, bits | 0x80000000)  # the order of the keys
+        order = np.lexsort((np.broadcast_to(np.arange(n), key.shape), -key), axis=1)[:, :k]
+        np.testing.assert_array_equal(i[rows].cpu().numpy(), order)
+        np.testing.assert_array_equal(v[rows].cpu().numpy(), np.take_along_axis(sn, order, axis=1))
+    np.testing.assert_array_equal(v[11:].cpu().numpy(), s[11:].topk(k).values.numpy())
+    assert torch.equal(s[11:].cuda().gather(1, i[11:].long()), v[11:])
+
+
 @pytest.mark.parametrize("nq,n,d,k,path", [
     (1, 1, 64, 1, "matrix"), (1, 5003, 384, 5, "matrix"), (16, 8192, 768, 10, "matrix"), (17, 700, 384, 256, "matrix"),
     (300, 8191, 128, 100, "matrix"), (5, 8193, 320, 3, "scan"), (1, 8192, 1600, 256, "matrix"),
