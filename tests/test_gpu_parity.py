@@ -799,6 +799,52 @@ def test_topk_rows_of_many_rows(eng, nq, n, k):
     assert torch.equal(s[11:].cuda().gather(1, i[11:].long()), v[11:])
 
 
+@pytest.mark.parametrize("nq,n,k", [(3, 400, 3), (3, 8000, 40), (3, 8000, 700), (3, 16000, 40), (3, 16000, 900), (3, 32768, 5),
+                                    (3, 32768, 600), (3, 50000, 64), (600, 1000, 90), (600, 3000, 300), (520, 40000, 30)])
+def test_topk_rows_orders_nan_by_sign(eng, nq, n, k):
+    """NaN above +inf or below -inf, as its sign bit says, fewer and more of them than k."""
+    say(f"topk_rows nan nq={nq} n={n} k={k}")
+    g = torch.Generator().manual_seed(n + k)
+    s = torch.randn(nq, n, generator=g)
+    nan = torch.tensor([0x7FC00000, -0x400000], dtype=torch.int32).view(torch.float32)
+    s[:, 7::97], s[:, 9::89] = nan[0], nan[1]
+    s[0, 3::61], s[0, 4::53] = float("inf"), -float("inf")
+    s[1, 5::7] = nan[0]
+    s[2, n // 50:] = nan[1]  # fewer than k others
+    v, i = eng.topk_rows(s.cuda(), k)
+    torch.cuda.synchronize()
+    bits = s[:16].contiguous().numpy().view(np.uint32).astype(np.int64)
+    key = np.where(bits & 0x80000000, 0xFFFFFFFF - bits, bits | 0x80000000)  # the order of the keys
+    order = np.lexsort((np.broadcast_to(np.arange(n), key.shape), -key), axis=1)[:, :k]
+    np.testing.assert_array_equal(i[:16].cpu().numpy(), order)
+    np.testing.assert_array_equal(v[:16].cpu().numpy().view(np.uint32).astype(np.int64), np.take_along_axis(bits, order, axis=1))
+
+
+def test_nan_and_equal_rows_do_not_slow_topk_rows(eng):
+    """A NaN in every row, or one row of equal scores beside others, costs no second, serial pass: 64 x 30000 with NaN
+    115 us where plain rows took 14, 600 x 200000 with a row of zeros 400 where plain ones took 161.  (Best of 20.)"""
+
+    def best(s, k):
+        t = []
+        for _ in range(20):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            eng.topk_rows(s, k)
+            e1.record()
+            torch.cuda.synchronize()
+            t.append(e0.elapsed_time(e1))
+        return min(t)
+
+    s = torch.randn(64, 30000, device="cuda", generator=torch.Generator("cuda").manual_seed(1))
+    plain = best(s, 100)
+    s[:, 5] = float("nan")
+    assert best(s, 100) < 2.5 * plain
+    s = torch.randn(600, 200000, device="cuda", generator=torch.Generator("cuda").manual_seed(2))
+    plain = best(s, 10)
+    s[0] = 0.0
+    assert best(s, 10) < 1.6 * plain
+
+
 @pytest.mark.parametrize("nq,n,d,k,path", [
     (1, 1, 64, 1, "matrix"), (1, 5003, 384, 5, "matrix"), (16, 8192, 768, 10, "matrix"), (17, 700, 384, 256, "matrix"),
     (300, 8191, 128, 100, "matrix"), (5, 8193, 320, 3, "scan"), (1, 8192, 1600, 256, "matrix"),
