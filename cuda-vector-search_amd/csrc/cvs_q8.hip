@@ -80,7 +80,8 @@ __global__ __launch_bounds__(kBlock) void q8_block_max_kernel(const uint16_t* ke
 // (the scale found here) left one workgroup per CU at d = 1024: 1140 us for
 // 300k rows.  The whole companion build (row keys, sort, blocks), against 4
 // lanes a row and rows read twice: 500k x 768 744 -> 431 us, 300k x 1024 670 ->
-// 402 us, 500k x 384 369 -> 252 us.
+// 402 us, 500k x 384 369 -> 248 us; narrow rows skip the pieces of padding (296k x
+// 128 130 -> 115).
 constexpr int kQ8Loads = 6;  // 8-element pieces per lane and round (dq is a multiple of 64 * 6)
 __global__ __launch_bounds__(512) void q8_build_kernel(Q8BuildArgs a) {
   constexpr int NW = 512 / kWave;
@@ -92,7 +93,7 @@ __global__ __launch_bounds__(512) void q8_build_kernel(Q8BuildArgs a) {
   const int64_t row = blk * 64 + (tid >> 3);
   const int part = tid & 7;
   const bool live = row < a.n;
-  const int np = live ? a.d / 64 : 0;  // this lane's pieces
+  const int np = a.d / 64;  // a lane's pieces
   const half8* src = reinterpret_cast<const half8*>(a.x + (live ? a.perm[row] : 0) * (int64_t)a.d) + part;
   const float M = a.bmeta[blk].w;
   const float s = M / 127.f;
@@ -104,20 +105,21 @@ __global__ __launch_bounds__(512) void q8_build_kernel(Q8BuildArgs a) {
   for (int i0 = 0; 64 * i0 < a.dq; i0 += kQ8Loads) {
     half8 v[kQ8Loads];
 #pragma unroll
-    for (int i = 0; i < kQ8Loads; ++i) v[i] = src[8 * max(0, min(i0 + i, np - 1))];  // (clamped: they issue together)
+    for (int i = 0; i < kQ8Loads; ++i) v[i] = i0 + i < np ? src[8 * (i0 + i)] : half8{};  // (uniform: they issue together)
 #pragma unroll
     for (int i = 0; i < kQ8Loads; ++i) {
-      if (i0 + i >= np) v[i] = half8{};
       unsigned lo = 0, hi = 0;
+      if (i0 + i < np) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float xv = (float)v[i][j];
-        const signed char c = q8_quant(xv, inv);
-        const float f = fmaf(-s, (float)c, xv);
-        ff = fmaf(f, f, ff);
-        xx = fmaf(xv, xv, xx);
-        if (j < 4) lo |= (unsigned)(unsigned char)c << (8 * j);
-        else hi |= (unsigned)(unsigned char)c << (8 * (j - 4));
+        for (int j = 0; j < 8; ++j) {
+          const float xv = live ? (float)v[i][j] : 0.f;
+          const signed char c = q8_quant(xv, inv);
+          const float f = fmaf(-s, (float)c, xv);
+          ff = fmaf(f, f, ff);
+          xx = fmaf(xv, xv, xx);
+          if (j < 4) lo |= (unsigned)(unsigned char)c << (8 * j);
+          else hi |= (unsigned)(unsigned char)c << (8 * (j - 4));
+        }
       }
       *reinterpret_cast<int2*>(dst + 64 * (i0 + i)) = int2{(int)lo, (int)hi};  // (zero past d)
     }
@@ -148,7 +150,9 @@ __global__ __launch_bounds__(512) void q8_build_kernel(Q8BuildArgs a) {
     }
     a.bmeta[blk] = meta;
     // the corpus-wide maximum: non-negative floats order like their bits (a NaN norm is left out)
-    if (meta.z >= 0.f) atomicMax(reinterpret_cast<int*>(a.xmax), __float_as_int(meta.z));
+    // (A look first: thousands of atomics on one word queue up.  A stale value is only a smaller one.)
+    if (meta.z > *reinterpret_cast<volatile float*>(a.xmax))
+      atomicMax(reinterpret_cast<int*>(a.xmax), __float_as_int(meta.z));
   }
 }
 
